@@ -1074,8 +1074,8 @@ __global__ __launch_bounds__(kPackBlock) void obsListKernel(Dev d, float* out, i
         });
 }
 
-// Everything an env step does after its ticks, for kStepSims simulations per
-// workgroup: rewards and dones, the transition state and the transition
+// Everything an env step does after its ticks, for `sims` simulations per
+// workgroup (at most kStepSims; stepSims): rewards and dones, the transition state and the transition
 // observations of finished simulations, their resets, the match state, the
 // observations and the state, with the reference's data dependences (the
 // transition rows read the state before the resets, the others after).  A
@@ -1085,8 +1085,14 @@ __global__ __launch_bounds__(kPackBlock) void obsListKernel(Dev d, float* out, i
 // finished ones are known to each wave without a barrier; the transition
 // observations of the first finished ones are built in the same round as
 // the transition state, in the LDS left over by the state rows.
+//
+// Up to the headline's size the kernel is a chain of load-build-store rounds
+// in each workgroup, so few large workgroups leave the GPU empty: the host
+// spreads a small run over more of them.  At 65,536 1v1 simulations it writes
+// its outputs at the rate of a plain copy (156 MB in 32 us).
 constexpr int kStepSims = 64;
 static_assert(kStepSims == 64, "one simulation per lane of each wave");
+constexpr int kStepMinRows = 32;   // observation rows a packing workgroup keeps at least
 
 struct StepIO {
     float *rewards, *tstate, *tobs, *obs, *state;
@@ -1104,12 +1110,12 @@ HDI size_t stepLdsBytes(int obsDim, int stateDim)
     return a > b ? a : b;
 }
 
-__global__ __launch_bounds__(kPackBlock) void stepEnvKernel(Dev d, StepIO io)
+__global__ __launch_bounds__(kPackBlock) void stepEnvKernel(Dev d, StepIO io, int sims)
 {
     extern __shared__ float packLds[];
     __shared__ int listedRow[64];   // tobs row of each transition observation built in round 1
     const int t = threadIdx.x, lane = t & 63, q = t >> 6, nC = d.nCars;
-    const int s0 = blockIdx.x * kStepSims, s1 = min(s0 + kStepSims, d.nSim);
+    const int s0 = blockIdx.x * sims, s1 = min(s0 + sims, d.nSim);
     const int s = s0 + lane;
     // the match words and the first action words are loaded first and used
     // after the transition state's loads have been issued
@@ -1651,11 +1657,12 @@ struct carl_env {
     hipEvent_t fork = nullptr, join[kMaxTickStreams - 1] = {};
     int windowSims = kDefaultWindowSims;  // simulations per block of the tick-window kernel (0: phase kernels)
     // Until the caller sets windowSims, a run too small to fill the device's
-    // resident window workgroups uses smaller ones (down to kAutoWindowMin
-    // simulations): the kernel's time is one workgroup's latency chain, so
-    // spreading the simulations over more compute units shortens it.
+    // resident window workgroups uses smaller ones (effectiveWindowSims): the
+    // kernel's time is one workgroup's latency chain, so spreading the
+    // simulations over more compute units shortens it.
     bool windowAuto = true;
     int windowResident = 0;   // window workgroups the device holds at once
+    int stepResident = 0;     // packing workgroups the device holds at once
     int timing = 0;                      // CARL_TIME_* flags
     // timing: a start and an end event per timed launch not yet folded
     // (a pool of at most kTimedPool pairs) and the launch's kernel id;
@@ -2026,6 +2033,20 @@ int resetPadRows(carl_env* e, Selection sel)
     return CARL_OK;
 }
 
+// Simulations per packing workgroup: kStepSims, halved while the workgroups
+// still fit the device together and each keeps kStepMinRows observation rows
+// (fewer leave most of its lanes without a row to build).  Packing of 4v4 at
+// 4,099 simulations 114 -> 32 us (4 per workgroup), 3v3 at 16,384 69 -> 41 us
+// (16), 2v2 at 10,007 42 -> 23 us (16), 1v1 at 8,192 and 1,000 17.5 -> 13.7
+// and 11.7 us (16); with 8 or 4 there 15.2 and 12.9 us, and twice the
+// workgroups the device holds 25 us.
+int stepSims(const carl_env* e)
+{
+    int sims = kStepSims;
+    while (sims / 2 * e->nCars >= kStepMinRows && e->grid(e->nSim, sims / 2) <= e->stepResident) sims /= 2;
+    return sims;
+}
+
 int checkEnv(carl_env* e)
 {
     if (!e) return fail(CARL_ERR_VALUE, "null environment handle");
@@ -2095,6 +2116,10 @@ int carl_env_create(int nSim, int nBlue, int nOrange, int seed, int frameskip, i
                    &perCu, windowKernelFor(e->nCars, false), kWindowBlock, 0) != hipSuccess)
             return bail(fail(CARL_ERR_RUNTIME, "window kernel occupancy query failed"));
         e->windowResident = perCu * cus;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCu, stepEnvKernel, kPackBlock,
+                                                         stepLdsBytes(e->obsDim, e->stateDim)) != hipSuccess)
+            return bail(fail(CARL_ERR_RUNTIME, "packing kernel occupancy query failed"));
+        e->stepResident = perCu * cus;
     }
     const size_t nT = (size_t)e->nTotal, nS = (size_t)nSim;
     int rc = CARL_OK;
@@ -2183,8 +2208,9 @@ int carl_env_step(carl_env* e, int kind, const void* actions)
     io.frameskip = e->frameskip; io.tickCount = e->tickCount; io.nOrange = e->nOrange;
     io.rule = e->rule();
     const size_t lds = stepLdsBytes(e->obsDim, e->stateDim);
-    CARL_TRY(launchTick(e, true, CARL_KERNEL_STEP_ENV, stepEnvKernel, dim3(e->grid(e->nSim, kStepSims)),
-                        dim3(kPackBlock), (uint32_t)lds, e->stream, e->dev(), io));
+    const int sims = stepSims(e);
+    CARL_TRY(launchTick(e, true, CARL_KERNEL_STEP_ENV, stepEnvKernel, dim3(e->grid(e->nSim, sims)),
+                        dim3(kPackBlock), (uint32_t)lds, e->stream, e->dev(), io, sims));
     HIP_TRY(hipGetLastError());
     return CARL_OK;
 }
