@@ -443,7 +443,6 @@ __global__ __launch_bounds__(kTickBlock) void finishKernel(Dev d, int simsPerBlo
 constexpr int kWindowBlock = CARL_WINDOW_BLOCK;
 constexpr int kWindowWaves = kWindowBlock / 64;
 constexpr int kDefaultWindowSims = CARL_WINDOW_SIMS;
-constexpr int kAutoWindowMin = 8;   // smallest automatic window workgroup (simulations)
 // rounds of candidate-index loads the window kernel's contact search keeps in
 // flight beyond the round of screening-data loads
 #ifndef CARL_WINDOW_CONTACT_LEAD
@@ -469,9 +468,9 @@ union WaveLds {
     uint32_t hand[kWsPlanes * 64];   // the contact phase's results, read by the car-arena phase
     BallLds ball;
 };
-// Car car0 + 64 w + l is contact owner l of wave w and car-arena thread
-// 64 w + l: a block holds at most kWindowBlock cars, one contact group per
-// wave, so each car's handoff stays in the lane that produced it.
+// Lane l of wave w is contact owner and car-arena thread of the same car: a
+// block holds at most kWindowBlock cars, one contact group per wave, so each
+// car's handoff stays in the lane that produced it.
 static_assert(kWindowContactOwners == 64, "the LDS handoff pairs contact owners with car-arena threads");
 struct WindowLds {
     WaveLds wave[kWindowWaves];
@@ -645,6 +644,13 @@ DI void tickWindowBody(Dev d0, uint32_t* __restrict__ ws, int screen, int kind, 
     const int sim0 = range.begin + blockIdx.x * simsPerBlock;
     const int simEnd = min(sim0 + simsPerBlock, range.end);
     const int car0 = sim0 * d.nCars, carEnd = simEnd * d.nCars;
+    // Undealt: the block's cars split evenly between the waves, whole pairs
+    // of cars to each (a 1v1 simulation's two cars sit in lanes 2i, 2i + 1).
+    // A block that is not full (a small run) would otherwise leave all of its
+    // cars to the first wave: window launch of 2v2 at 10,007 simulations 662
+    // -> 616 us, 4v4 at 4,099 806 -> 735 us, 1v0 at 30,011 308 -> 282 us.
+    const int waveCars = (carEnd - car0 + 2 * kWindowWaves - 1) / (2 * kWindowWaves) * 2;
+    const int waveCar0 = car0 + wave * waveCars, waveCarEnd = min(waveCar0 + waveCars, carEnd);
     unsigned long long acc[kWindowStages] = {}, first = 0, last = 0;
     auto mark = [&](int stage) {
         if constexpr (Profile) {
@@ -673,9 +679,9 @@ DI void tickWindowBody(Dev d0, uint32_t* __restrict__ ws, int screen, int kind, 
                 }
             }
         } else {
-            for (int g = car0 + wave * kWindowContactOwners; g < carEnd; g += kWindowWaves * kWindowContactOwners)
+            for (int g = waveCar0; g < waveCarEnd; g += kWindowContactOwners)
                 contactGroup<kWindowContactLead, kWindowContactOwners>(d, LdsHandoff{ L.wave[wave].hand }, screen,
-                                                                         g + lane, g + lane < carEnd,
+                                                                         g + lane, g + lane < waveCarEnd,
                                                                          L.wave[wave].contact, lane);
         }
         __syncthreads();
@@ -683,7 +689,7 @@ DI void tickWindowBody(Dev d0, uint32_t* __restrict__ ws, int screen, int kind, 
         if constexpr (Balanced) {
             carArenaCar(d, LdsHandoff{ L.wave[wave].hand }, kind, actions, tick, slotCar(t), lane);
         } else {
-            for (int c = car0 + t; c < carEnd; c += kWindowBlock)
+            for (int c = waveCar0 + lane; c < waveCarEnd; c += 64)
                 carArenaCar(d, LdsHandoff{ L.wave[wave].hand }, kind, actions, tick, c, lane);
         }
         __syncthreads();
@@ -707,7 +713,7 @@ DI void tickWindowBody(Dev d0, uint32_t* __restrict__ ws, int screen, int kind, 
             finishCar(d, slotCar(t));
             if (t < kBlockSims) finishBall(d, slotSim(t));
         } else {
-            for (int c = car0 + t; c < carEnd; c += kWindowBlock) finishCar(d, c);
+            for (int c = waveCar0 + lane; c < waveCarEnd; c += 64) finishCar(d, c);
             for (int s = sim0 + t; s < simEnd; s += kWindowBlock) finishBall(d, s);
         }
         __syncthreads();
@@ -1806,9 +1812,21 @@ int launchTick(carl_env* e, bool timed, int kernel, void (*k)(P...), dim3 grid, 
 // otherwise four phase kernels per tick.  Timing events bracket partition
 // 0's launches.
 // Simulations per window workgroup for the next launch: the set size capped
-// at a workgroup's cars; until the caller sets it, halved (down to
-// kAutoWindowMin) while every partition's workgroups together still fit the
-// device's resident window workgroups.
+// at a workgroup's cars; until the caller sets it, the fewest with which
+// every partition's workgroups together still fit the device's resident
+// window workgroups.  A launch lasts as long as its slowest workgroup's chain
+// of phases, and that chain grows with the cars per wave (the candidate lists
+// its wave walks, the branches its lanes take between them).  Window launch
+// of 1v1 at 1,000 simulations 405 -> 325 us (1 per workgroup, was 8), 50,001
+// 706 -> 673 us (49, was 64), 2v2 at 10,007 616 -> 596 us (10, was 16), 3v3
+// clustered at 16,384 876 -> 817 us (16, was 21).
+constexpr int kDealMinTicks = 4;   // balancedLaunch
+bool dealable(const carl_env* e)
+{
+    const int bs = dealBlockSims(e->nCars);
+    return e->balance && bs > 0 && !e->native() && e->dealList && std::min(e->tickStreams, e->nSim) == 1
+           && e->nSim % bs == 0;
+}
 int effectiveWindowSims(const carl_env* e)
 {
     if (e->windowSims <= 0) return 0;
@@ -1823,7 +1841,12 @@ int effectiveWindowSims(const carl_env* e)
         }
         return total;
     };
-    while (wsb / 2 >= kAutoWindowMin && blocks(wsb / 2) <= e->windowResident) wsb /= 2;
+    // full workgroups that the deal evens out are kept while half as many
+    // simulations each would not fit
+    if (dealable(e) && wsb == dealBlockSims(e->nCars) && e->frameskip >= kDealMinTicks
+        && blocks(wsb / 2) > e->windowResident)
+        return wsb;
+    while (wsb > 1 && blocks(wsb - 1) <= e->windowResident) wsb--;
     return wsb;
 }
 
@@ -1833,12 +1856,9 @@ int effectiveWindowSims(const carl_env* e)
 // launch of fewer ticks has less tail to even out than the scattered units
 // cost it: 2v2 stepped one tick at a time at 131,072 simulations ran 370 ->
 // 377 us per launch dealt.)
-constexpr int kDealMinTicks = 4;
 bool balancedLaunch(const carl_env* e, int ticks)
 {
-    const int bs = dealBlockSims(e->nCars);
-    return e->balance && bs > 0 && !e->native() && e->dealList && std::min(e->tickStreams, e->nSim) == 1
-           && effectiveWindowSims(e) == bs && e->nSim % bs == 0 && ticks >= kDealMinTicks;
+    return dealable(e) && effectiveWindowSims(e) == dealBlockSims(e->nCars) && ticks >= kDealMinTicks;
 }
 
 int launchTicks(carl_env* e, int kind, const void* actions, int n)
