@@ -44,6 +44,109 @@ struct KeyHash {
     }
 };
 
+// ---- candidate lists: for every cell of a cubic grid over the broadphase
+// box, the triangles that come within `reach` of the cell, ascending.
+
+struct D3 {
+    double x, y, z;
+};
+D3 operator-(D3 a, D3 b) { return { a.x - b.x, a.y - b.y, a.z - b.z }; }
+D3 along(D3 a, D3 d, double t) { return { a.x + d.x * t, a.y + d.y * t, a.z + d.z * t }; }
+double dot3(D3 a, D3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
+D3 cross3(D3 a, D3 b) { return { a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x }; }
+double clampD(double v, double lo, double hi) { return v < lo ? lo : (v > hi ? hi : v); }
+
+// closest point of the triangle to p: its plane's foot when that lies inside,
+// else the nearest point of the nearest edge
+D3 nearestOnTriangle(D3 p, const D3 (&v)[3], D3 n)
+{
+    const D3 foot = along(p, n, -dot3(p - v[0], n));
+    bool inside = true;
+    D3 best{};
+    double bestSq = 1e300;
+    for (int e = 0; e < 3; e++) {
+        const D3 a = v[e], edge = v[(e + 1) % 3] - a;
+        if (dot3(cross3(edge, foot - a), n) >= 0.0) continue;
+        inside = false;
+        const D3 q = along(a, edge, clampD(dot3(p - a, edge) / dot3(edge, edge), 0.0, 1.0));
+        const double sq = dot3(p - q, p - q);
+        if (sq < bestSq) { bestSq = sq; best = q; }
+    }
+    return inside ? foot : best;
+}
+
+// Whether the triangle provably stays farther than `reach` from the cube of
+// half side h around c: some direction separates the two by more.  Tried are
+// the direction between the triangle's box and the cube, the triangle's
+// normal, and the directions that alternating projections between the cube
+// and the triangle give (they converge to the closest pair).  A pair that no
+// tried direction separates counts as near.
+bool fartherThan(double reach, const D3 (&v)[3], D3 n, D3 lo, D3 hi, D3 c, double h)
+{
+    const D3 gap{ std::max(0.0, std::max(lo.x - c.x, c.x - hi.x) - h), std::max(0.0, std::max(lo.y - c.y, c.y - hi.y) - h),
+                  std::max(0.0, std::max(lo.z - c.z, c.z - hi.z) - h) };
+    if (dot3(gap, gap) > reach * reach) return true;
+    if (std::fabs(dot3(c - v[0], n)) - h * (std::fabs(n.x) + std::fabs(n.y) + std::fabs(n.z)) > reach) return true;
+    D3 q = c;
+    for (int i = 0; i < 4; i++) {
+        const D3 t = nearestOnTriangle(q, v, n);
+        q = D3{ clampD(t.x, c.x - h, c.x + h), clampD(t.y, c.y - h, c.y + h), clampD(t.z, c.z - h, c.z + h) };
+        const D3 d = t - q;
+        const double len = std::sqrt(dot3(d, d));
+        if (len <= reach) return false;   // two points within reach
+        const double tri = std::min(dot3(v[0], d), std::min(dot3(v[1], d), dot3(v[2], d)));
+        const double cube = dot3(c, d) + h * (std::fabs(d.x) + std::fabs(d.y) + std::fabs(d.z));
+        if (tri - cube > reach * len) return true;
+    }
+    return false;
+}
+
+// The lists of a grid of nx x ny x nz cells: triangle t is listed in every
+// cell it is not provably farther than `reach` from.
+void buildLists(const HostArena& arena, const std::vector<V3>& lo, const std::vector<V3>& hi, double cell, int nx, int ny,
+                int nz, double reach, std::vector<int>& start, std::vector<int>& list)
+{
+    const int nTris = (int)lo.size(), n[3] = { nx, ny, nz };
+    const double o[3] = { kArenaMin.x, kArenaMin.y, kArenaMin.z };
+    // the listed cells of every triangle, then the lists by counting
+    std::vector<int> cells;
+    std::vector<size_t> end(nTris);
+    start.assign((size_t)nx * ny * nz + 1, 0);
+    for (int t = 0; t < nTris; t++) {
+        D3 v[3];
+        for (int k = 0; k < 3; k++) {
+            const float* p = &arena.verts[3 * (size_t)arena.tris[3 * (size_t)t + k]];
+            v[k] = D3{ p[0], p[1], p[2] };
+        }
+        D3 nrm = cross3(v[1] - v[0], v[2] - v[0]);
+        const double nl = std::sqrt(dot3(nrm, nrm));
+        nrm = D3{ nrm.x / nl, nrm.y / nl, nrm.z / nl };
+        const D3 l{ lo[t].x, lo[t].y, lo[t].z }, h{ hi[t].x, hi[t].y, hi[t].z };
+        const double lv[3] = { l.x, l.y, l.z }, hv[3] = { h.x, h.y, h.z };
+        int a[3], b[3];
+        for (int k = 0; k < 3; k++) {
+            a[k] = std::max(0, (int)std::floor((lv[k] - reach - o[k]) / cell));
+            b[k] = std::min(n[k] - 1, (int)std::floor((hv[k] + reach - o[k]) / cell));
+        }
+        for (int z = a[2]; z <= b[2]; z++)
+            for (int y = a[1]; y <= b[1]; y++)
+                for (int x = a[0]; x <= b[0]; x++) {
+                    const D3 c{ o[0] + (x + 0.5) * cell, o[1] + (y + 0.5) * cell, o[2] + (z + 0.5) * cell };
+                    if (fartherThan(reach, v, nrm, l, h, c, 0.5 * cell)) continue;
+                    const int flat = x + nx * (y + ny * z);
+                    cells.push_back(flat);
+                    start[flat + 1]++;
+                }
+        end[t] = cells.size();
+    }
+    for (size_t c = 0; c + 1 < start.size(); c++) start[c + 1] += start[c];
+    list.assign(cells.size(), 0);
+    std::vector<int> at(start.begin(), start.end() - 1);
+    size_t i = 0;
+    for (int t = 0; t < nTris; t++)
+        for (; i < end[t]; i++) list[(size_t)at[cells[i]]++] = t;
+}
+
 }  // namespace
 
 std::string findArenaObj(const std::string& libraryDir)
@@ -267,92 +370,34 @@ std::string buildArena(const std::string& objPath, HostArena& out)
                               (float)s1, (float)s2, (float)s3, (float)epsEdge };
         std::memcpy(&screen[16 * (size_t)t], f, sizeof f);
     }
-    // ball candidate grid, also the cars' contact-search lists.  A ball only
-    // tests triangles registered in the broadphase cells its box overlaps, a
-    // car those of its own broadphase cell; each reference carries the
-    // triangle's edge angles and its registration range (x0 x1 y0 y1 6 bits
-    // each, z0 z1 4 bits) so that either can apply its rule itself, and the
-    // triangle's contact-search screening data.
+    // per triangle: edge angles and packed registration range (x0 x1 y0 y1 6
+    // bits each, z0 z1 4 bits), from which the searches apply the broadphase
+    // rule themselves (a ball only tests triangles registered in the cells its
+    // box overlaps, a car those of its own cell)
+    out.triAux.assign(4 * (size_t)nTris, 0.f);
+    for (int t = 0; t < nTris; t++) {
+        const auto& r = range[t];
+        const uint32_t reg = (uint32_t)r[0] | (uint32_t)r[3] << 6 | (uint32_t)r[1] << 12 | (uint32_t)r[4] << 18 |
+                             (uint32_t)r[2] << 24 | (uint32_t)r[5] << 28;
+        std::memcpy(&out.triAux[4 * (size_t)t], &out.angles[3 * (size_t)t], 3 * sizeof(float));
+        std::memcpy(&out.triAux[4 * (size_t)t + 3], &reg, sizeof reg);
+    }
+    // ball candidate grid: each reference as its record and its aux words
     {
-        const double reach = (double)kBallRadius + (double)kBallArenaBreak + 1.0;
-        auto fineRange = [&](int t, int (&a)[3], int (&b)[3]) {
-            const double l[3] = { lo[t].x, lo[t].y, lo[t].z }, h[3] = { hi[t].x, hi[t].y, hi[t].z };
-            const double o[3] = { kArenaMin.x, kArenaMin.y, kArenaMin.z };
-            const int n[3] = { kFineX, kFineY, kFineZ };
-            for (int k = 0; k < 3; k++) {
-                a[k] = std::max(0, (int)std::floor((l[k] - reach - o[k]) / kFineCell));
-                b[k] = std::min(n[k] - 1, (int)std::floor((h[k] + reach - o[k]) / kFineCell));
-            }
-        };
-        std::vector<int> fcount(kFineCells + 1, 0);
-        for (int t = 0; t < nTris; t++) {
-            int a[3], b[3];
-            fineRange(t, a, b);
-            for (int z = a[2]; z <= b[2]; z++)
-                for (int y = a[1]; y <= b[1]; y++)
-                    for (int x = a[0]; x <= b[0]; x++) fcount[x + kFineX * (y + kFineY * z)]++;
-        }
-        out.fineStart.assign(kFineCells + 1, 0);
-        for (int c = 0; c < kFineCells; c++) out.fineStart[c + 1] = out.fineStart[c] + fcount[c];
-        const size_t nFine = (size_t)out.fineStart[kFineCells];
-        out.fineRecords.assign(16 * nFine, 0.f);
-        out.fineAux.assign(4 * nFine, 0.f);
-        out.triAux.assign(4 * (size_t)nTris, 0.f);
-        std::fill(fcount.begin(), fcount.end(), 0);
-        for (int t = 0; t < nTris; t++) {
-            int a[3], b[3];
-            fineRange(t, a, b);
-            const auto& r = range[t];
-            const uint32_t reg = (uint32_t)r[0] | (uint32_t)r[3] << 6 | (uint32_t)r[1] << 12 | (uint32_t)r[4] << 18 |
-                                 (uint32_t)r[2] << 24 | (uint32_t)r[5] << 28;
-            std::memcpy(&out.triAux[4 * (size_t)t], &out.angles[3 * (size_t)t], 3 * sizeof(float));
-            std::memcpy(&out.triAux[4 * (size_t)t + 3], &reg, sizeof reg);
-            for (int z = a[2]; z <= b[2]; z++)
-                for (int y = a[1]; y <= b[1]; y++)
-                    for (int x = a[0]; x <= b[0]; x++) {
-                        const int c = x + kFineX * (y + kFineY * z);
-                        const size_t f = (size_t)out.fineStart[c] + fcount[c]++;
-                        std::memcpy(&out.fineRecords[16 * f], &out.triRecords[16 * (size_t)t], 16 * sizeof(float));
-                        std::memcpy(&out.fineAux[4 * f], &out.triAux[4 * (size_t)t], 4 * sizeof(float));
-                    }
+        std::vector<int> list;
+        buildLists(out, lo, hi, kFineCell, kFineX, kFineY, kFineZ, (double)kBallRadius + (double)kBallArenaBreak + 1.0,
+                   out.fineStart, list);
+        out.fineRecords.resize(16 * list.size());
+        out.fineAux.resize(4 * list.size());
+        for (size_t f = 0; f < list.size(); f++) {
+            const size_t t = (size_t)list[f];
+            std::memcpy(&out.fineRecords[16 * f], &out.triRecords[16 * t], 16 * sizeof(float));
+            std::memcpy(&out.fineAux[4 * f], &out.triAux[4 * t], 4 * sizeof(float));
         }
     }
     // car candidate grid: the same rule with the car's reach, triangle
-    // indices only, ascending within a cell
-    {
-        const double reach = (double)kCarGridReach;
-        auto carRange = [&](int t, int (&a)[3], int (&b)[3]) {
-            const double l[3] = { lo[t].x, lo[t].y, lo[t].z }, h[3] = { hi[t].x, hi[t].y, hi[t].z };
-            const double o[3] = { kArenaMin.x, kArenaMin.y, kArenaMin.z };
-            const int n[3] = { kCarX, kCarY, kCarZ };
-            for (int k = 0; k < 3; k++) {
-                a[k] = std::max(0, (int)std::floor((l[k] - reach - o[k]) / kCarCell));
-                b[k] = std::min(n[k] - 1, (int)std::floor((h[k] + reach - o[k]) / kCarCell));
-            }
-        };
-        std::vector<int> ccount(kCarCells + 1, 0);
-        for (int t = 0; t < nTris; t++) {
-            int a[3], b[3];
-            carRange(t, a, b);
-            for (int z = a[2]; z <= b[2]; z++)
-                for (int y = a[1]; y <= b[1]; y++)
-                    for (int x = a[0]; x <= b[0]; x++) ccount[x + kCarX * (y + kCarY * z)]++;
-        }
-        out.carStart.assign(kCarCells + 1, 0);
-        for (int c = 0; c < kCarCells; c++) out.carStart[c + 1] = out.carStart[c] + ccount[c];
-        out.carTris.assign((size_t)out.carStart[kCarCells], 0);
-        std::fill(ccount.begin(), ccount.end(), 0);
-        for (int t = 0; t < nTris; t++) {
-            int a[3], b[3];
-            carRange(t, a, b);
-            for (int z = a[2]; z <= b[2]; z++)
-                for (int y = a[1]; y <= b[1]; y++)
-                    for (int x = a[0]; x <= b[0]; x++) {
-                        const int c = x + kCarX * (y + kCarY * z);
-                        out.carTris[(size_t)out.carStart[c] + ccount[c]++] = t;
-                    }
-        }
-    }
+    // indices only
+    buildLists(out, lo, hi, kCarCell, kCarX, kCarY, kCarZ, (double)kCarGridReach, out.carStart, out.carTris);
     for (int r = 0; r < nRefs; r++)
         std::memcpy(&out.records[16 * (size_t)r], &out.triRecords[16 * (size_t)out.cellTris[r]], 16 * sizeof(float));
     return "";

@@ -27,10 +27,9 @@ constexpr float kCellY = (kArenaMax.y - kArenaMin.y) / 48.f;
 constexpr float kCellZ = (kArenaMax.z - kArenaMin.z) / 10.f;
 constexpr float kBoundaryEdge = 2.f * kPi;
 // ball candidate grid: cubic cells over the broadphase box; a cell lists every
-// triangle whose box comes within ball reach (+1 uu) of the cell.  64 uu cells
-// list about half the triangles of 128 uu ones near the curved walls (1.46 M
-// references, 210 MB, against 0.26 M); the cars' contact search, which walks
-// the same lists, runs 3.5% faster per step once cars have spread to the walls.
+// triangle that comes within ball reach (+1 uu) of the cell (0.96 M
+// references, 77 MB).  The distance is the triangle's own: its box comes as
+// near to half as many cells again (1.46 M references).
 constexpr float kFineCell = 64.f;
 constexpr int kFineX = 129, kFineY = 188, kFineZ = 33;   // ceil(extent / kFineCell)
 constexpr int kFineCells = kFineX * kFineY * kFineZ;
@@ -39,9 +38,9 @@ static_assert(kFineX * kFineCell >= kArenaMax.x - kArenaMin.x && kFineY * kFineC
               "ball grid must cover the broadphase box");
 // car candidate grid: the same lists for the cars' contact search, in 32 uu
 // cells and with the car's own reach (every car test stays within 76.6 uu of
-// the car's centre, engine.hip), so a car near a curved wall walks about 30%
-// fewer candidates than in the ball's lists.  Each list is triangle indices
-// only (6.67 M references, 27 MB).
+// the car's centre, engine.hip).  Each list is triangle indices only (4.0 M
+// references, 16 MB; 6.7 M by the triangles' boxes).  Cars of a 1v1 rollout
+// list 3.1 triangles each on average, by the boxes 5.2.
 constexpr float kCarCell = 32.f;
 constexpr float kCarGridReach = 78.f;
 constexpr int kCarX = 257, kCarY = 375, kCarZ = 66;   // ceil(extent / kCarCell)

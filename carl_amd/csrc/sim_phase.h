@@ -597,7 +597,7 @@ DI int gatherBallContacts(const Dev& d, V3 center, BallContact* cs)
 }
 
 // ---- cooperative gather over the ball candidate grid.  A ball's candidates
-// are the list of the grid cell holding its centre: every triangle whose box
+// are the list of the grid cell holding its centre: every triangle that
 // comes within reach + 1 uu of that cell, each once, in ascending triangle
 // order.  The reference tests the triangles registered in the broadphase cells
 // its box overlaps, merged in ascending index order, so an item counts only
