@@ -43,7 +43,7 @@ DI Q4 integrateRotation(Q4 rot, V3 ang)
         axis = ang * (s / speed);
     }
     const Q4 delta{ axis.x, axis.y, axis.z, c };
-    const Q4 basis = quatFromColumns(rotate(rot, kX), rotate(rot, kY), rotate(rot, kZ));
+    const Q4 basis = quatFromColumns(rotateX(rot), rotateY(rot), rotateZ(rot));
     return qnormalize(qmul(delta, basis));
 }
 
@@ -56,7 +56,7 @@ DI void integratePose(V3& pos, V3& cen, Q4& rot, V3 vel, V3 ang)
 
 DI V3 boxAabbMin(V3 cen, Q4 rot)
 {
-    const V3 rx = rotate(rot, kX), ry = rotate(rot, kY), rz = rotate(rot, kZ);
+    const V3 rx = rotateX(rot), ry = rotateY(rot), rz = rotateZ(rot);
     const V3 half = (vabs(rx) * kHalf.x + vabs(ry) * kHalf.y) + vabs(rz) * kHalf.z;
     return cen - half;
 }
@@ -132,12 +132,19 @@ DI bool rayBox(V3 start, V3 dir, V3 center, Q4 rot, float maxDist, float& dist, 
     return true;
 }
 
-// Every wheel ray ends within kWheelReach of the car's box centre: the
-// anchors lie at most 56.1 uu from it, and a ray is at most the longer of the
-// two ray lengths; 4 uu spare cover the rounding of the rays' arithmetic.  A
-// body whose centre is farther than kWheelReach plus its bounding radius
-// meets no wheel ray, so its rays are not cast (each would miss).
-constexpr float kWheelReach = 56.1f + (kFrontRay > kBackRay ? kFrontRay : kBackRay) + 4.f;
+// The four wheel rays lie within kWheelReach of the point kRayMid along them
+// from the car's box centre (the anchors sit in the centre's plane, at most
+// 56.1 uu from it, and the rays run half of kBackRay to either side of the
+// point); 4 uu spare cover the rounding of the rays' arithmetic.  A body
+// whose centre is farther from that point than kWheelReach plus its bounding
+// radius meets no wheel ray, so its rays are not cast (each would miss).  A
+// wave casts them as soon as one of its cars does: with the reach taken from
+// the box centre (105.7 uu) twice as many did.
+constexpr float kRayMid = 0.5f * kBackRay;
+constexpr float kWheelReach = 61.5f + 4.f;           // hypot(56.1, 24.8) rounded up, and the spare
+static_assert(kBackRay >= kFrontRay && kBackX * kBackX + kBackY * kBackY + kRayMid * kRayMid < 61.5f * 61.5f &&
+                  kFrontX * kFrontX + kFrontY * kFrontY + kRayMid * kRayMid < 61.5f * 61.5f,
+              "the wheel rays' bounding sphere");
 constexpr float kCarRayReach = kWheelReach + 80.f;   // + |kHalf| (76.6) rounded up
 constexpr float kBallRayReach = kWheelReach + kBallRadius;
 
@@ -176,6 +183,7 @@ DI void raycastBodies(const Dev& d, int car, int sim, V3 cen, const V3* start, V
 {
     const int base = sim * d.nCars;
     const V3 ball = d.sv(CARL_SIM_BALL_POS, sim);
+    const V3 mid = cen + dir * kRayMid;
     for (int o = 0; o < d.nCars; o++) {
         const int oc = base + o;
         // the other car's words are loaded together, before its demolished
@@ -183,10 +191,10 @@ DI void raycastBodies(const Dev& d, int car, int sim, V3 cen, const V3* start, V
         const int demoed = d.ci(CARL_CAR_DEMOED, oc);
         const V3 ocen = d.cv(CARL_CAR_CEN, oc);
         const Q4 orot = d.cq(CARL_CAR_ROT, oc);
-        if (oc == car || demoed || lensq(ocen - cen) > kCarRayReach * kCarRayReach) continue;
+        if (oc == car || demoed || lensq(ocen - mid) > kCarRayReach * kCarRayReach) continue;
         raycastCar(start, dir, ocen, orot, w);
     }
-    if (!(lensq(ball - cen) > kBallRayReach * kBallRayReach)) raycastBall(start, dir, ball, w);
+    if (!(lensq(ball - mid) > kBallRayReach * kBallRayReach)) raycastBall(start, dir, ball, w);
 }
 
 DI void storeWheelOutputs(const Dev& d, int car, const Wheels& w)
@@ -331,15 +339,18 @@ DI void storeRegs(const Dev& d, int c, const CarRegs& r)
     d.setv(CARL_CAR_MANIFOLD_NORMAL, c, r.manNormal);
 }
 
+// The curves choose a lane's segment first and divide once: a branch per
+// segment would run every segment's division for a wave of mixed speeds.
+// (x - 0 is x, so the first segment's rounding is unchanged.)
 DI float steerCurve(float x)
 {
-    if (x <= 0.f) return 0.53356f;
-    if (x <= 500.f) return 0.53356f + (0.31930f - 0.53356f) * (x / 500.f);
-    if (x <= 1000.f) return 0.31930f + (0.18203f - 0.31930f) * ((x - 500.f) / 500.f);
-    if (x <= 1500.f) return 0.18203f + (0.10570f - 0.18203f) * ((x - 1000.f) / 500.f);
-    if (x <= 1750.f) return 0.10570f + (0.08507f - 0.10570f) * ((x - 1500.f) / 250.f);
-    if (x <= 3000.f) return 0.08507f + (0.03454f - 0.08507f) * ((x - 1750.f) / 1250.f);
-    return 0.03454f;
+    float x0 = 0.f, width = 500.f, y0 = 0.53356f, dy = 0.31930f - 0.53356f;
+    if (x > 500.f) { x0 = 500.f; y0 = 0.31930f; dy = 0.18203f - 0.31930f; }
+    if (x > 1000.f) { x0 = 1000.f; y0 = 0.18203f; dy = 0.10570f - 0.18203f; }
+    if (x > 1500.f) { x0 = 1500.f; width = 250.f; y0 = 0.10570f; dy = 0.08507f - 0.10570f; }
+    if (x > 1750.f) { x0 = 1750.f; width = 1250.f; y0 = 0.08507f; dy = 0.03454f - 0.08507f; }
+    const float y = y0 + dy * ((x - x0) / width);
+    return x <= 0.f ? 0.53356f : (x <= 3000.f ? y : 0.03454f);
 }
 
 DI float slideSteerCurve(float x)
@@ -351,10 +362,10 @@ DI float slideSteerCurve(float x)
 
 DI float driveTorqueCurve(float x)
 {
-    if (x <= 0.f) return 1.f;
-    if (x >= 1410.f) return 0.f;
-    if (x <= 1400.f) return 1.f - (x / 1400.f) * 0.9f;
-    return 0.1f * (1.f - (x - 1400.f) / 10.f);
+    const bool low = x <= 1400.f;
+    const float t = (low ? x : x - 1400.f) / (low ? 1400.f : 10.f);
+    const float y = low ? 1.f - t * 0.9f : 0.1f * (1.f - t);
+    return x <= 0.f ? 1.f : (x >= 1410.f ? 0.f : y);
 }
 
 struct Frame {
@@ -397,8 +408,8 @@ DI void applyControls(CarRegs& r, const Controls& c, const Wheels& w)
 {
     Frame f;
     f.rot = r.rot;
-    f.fwd = rotate(r.rot, kX);
-    f.up = rotate(r.rot, kZ);
+    f.fwd = rotateX(r.rot);
+    f.up = rotateZ(r.rot);
     f.fwdSpeed = dot(r.vel, f.fwd);
     f.absFwdSpeed = fabsf(f.fwdSpeed);
     int n = 0;
@@ -492,7 +503,7 @@ DI void applyControls(CarRegs& r, const Controls& c, const Wheels& w)
             const bool hasInput = lensq(input) > 0.f;
 #pragma unroll
             for (int i = 0; i < 3; i++) {
-                const V3 dir = i == 0 ? -rotate(f.rot, kY) : (i == 1 ? f.up : -f.fwd);
+                const V3 dir = i == 0 ? -rotateY(f.rot) : (i == 1 ? f.up : -f.fwd);
                 const float control = comp(input, i) * comp(ctlScale, i);
                 const float proj = dot(dir, r.ang);
                 const float damp = proj * comp(kAirDamping, i) * (1.f - fabsf(comp(dampIn, i)));
@@ -527,7 +538,7 @@ DI void applyControls(CarRegs& r, const Controls& c, const Wheels& w)
     // auto-flip against an upward facing contact of the previous tick (Drive.cuh:134-178)
     {
         if (f.jumpPressed && r.manCount != 0 && r.manNormal.z > kAutoflipNormZ) {
-            const V3 right = rotate(f.rot, kY);
+            const V3 right = rotateY(f.rot);
             const float roll = -atan2_(right.z, f.up.z);
             const float absRoll = fabsf(roll);
             if (absRoll > kAutoflipRoll) {
@@ -1095,9 +1106,14 @@ DI void waveSync()
 
 DI unsigned long long lanesBelow(int lane) { return lane ? (~0ull >> (64 - lane)) : 0ull; }
 
+// The screen's arithmetic is bounds, not results: fused multiply-adds and the
+// hardware's min and max serve it (fewer roundings than its margins allow for,
+// and about two thirds of the operations).
+DI float fdot(V3 a, V3 b) { return __builtin_fmaf(a.z, b.z, __builtin_fmaf(a.y, b.y, a.x * b.x)); }
+
 DI bool boxAxisMiss(V3 axis, V3 w, V3 half, float face)
 {
-    return fabsf(dot(axis, w)) - dot(vabs(axis), half) > face + kSatMargin;
+    return fabsf(fdot(axis, w)) - fdot(vabs(axis), half) > face + kSatMargin;
 }
 
 // screen stage: queue the item unless the heavy stage provably rejects it
@@ -1114,18 +1130,19 @@ DI void contactScreen(ContactLdsT<Owners>& L, const RefBox& b, int o, int lane)
     const V3 n{ b.lo.w, b.hi.w, b.pl.x };
     // the car box against the triangle's plane, within the normal axis bound
     const float dist = l1norm(w) + l1norm(half);
-    const float dev = kRotErr2 * dist + b.sat.w;
-    const float dn = (dev * b.sat.x + dev * dev * b.sat.y) + b.sat.z;
-    const float boxR = dot(vabs(V3{ dot(n, ax), dot(n, ay), dot(n, az) }), kHalf);
-    const float planeGap = fabsf(b.pl.y - dot(n, V3{ s0.x, s0.y, s0.z })) - boxR;
-    const float planeTol = (dn * (dist + kHalfLen) + kRotErr * dist) + kPlaneSlack;
+    const float dev = __builtin_fmaf(kRotErr2, dist, b.sat.w);
+    const float dn = __builtin_fmaf(dev, __builtin_fmaf(dev, b.sat.y, b.sat.x), b.sat.z);
+    const float nz = fdot(n, az);
+    const float boxR = fdot(vabs(V3{ fdot(n, ax), fdot(n, ay), nz }), kHalf);
+    const float planeGap = fabsf(b.pl.y - fdot(n, V3{ s0.x, s0.y, s0.z })) - boxR;
+    const float planeTol = __builtin_fmaf(dn, dist + kHalfLen, __builtin_fmaf(kRotErr, dist, kPlaneSlack));
     const bool satMiss = s4.w == 0.f || boxAxisMiss(ax, w, half, kHalf.x) || boxAxisMiss(ay, w, half, kHalf.y) ||
                          boxAxisMiss(az, w, half, kHalf.z) || (dn <= 0.5f && planeGap > planeTol);
-    const float gap = fmax_(fmax_(fmax_(tlo.x - rhi.x, rlo.x - thi.x), fmax_(tlo.y - rhi.y, rlo.y - thi.y)),
-                            fmax_(tlo.z - rhi.z, rlo.z - thi.z));
-    const float cosDir = fabsf(dot(n, az)) - 1e-6f;
-    const float sc = dot(n, (rlo + rhi) * 0.5f) - b.pl.y;
-    const float sh = dot(vabs(n), (rhi - rlo) * 0.5f);
+    const float gap = fmaxf(fmaxf(fmaxf(tlo.x - rhi.x, rlo.x - thi.x), fmaxf(tlo.y - rhi.y, rlo.y - thi.y)),
+                            fmaxf(tlo.z - rhi.z, rlo.z - thi.z));
+    const float cosDir = fabsf(nz) - 1e-6f;
+    const float sc = fdot(n, (rlo + rhi) * 0.5f) - b.pl.y;
+    const float sh = fdot(vabs(n), (rhi - rlo) * 0.5f);
     const bool rayMiss = (gap > kGapSlack && cosDir * (gap - kGapSlack) > b.pl.z) || sc - sh > b.pl.w ||
                          sc + sh < -b.pl.w;
     const bool keep = b.live && (s4.z == 0.f || !(satMiss && rayMiss));
@@ -1275,13 +1292,13 @@ DI void contactPrepare(ContactLdsT<Owners>& L, int lane, bool sat, V3 cen, Q4 ro
 {
     if (lane == 0) L.candN = 0;
     if (lane >= Owners) return;
-    const V3 dir = -rotate(rot, kZ);
+    const V3 dir = -rotateZ(rot);
     L.first[lane] = first;
     L.fine[lane] = fine;
     L.bcell[lane] = bcell;
     L.satOn[lane] = sat;
     L.rot[0][lane] = rot.x; L.rot[1][lane] = rot.y; L.rot[2][lane] = rot.z; L.rot[3][lane] = rot.w;
-    const V3 ax = rotate(rot, kX), ay = rotate(rot, kY), az = rotate(rot, kZ);
+    const V3 ax = rotateX(rot), ay = rotateY(rot), az = rotateZ(rot);
     V3 lo{ kFltMax, kFltMax, kFltMax }, hi{ -kFltMax, -kFltMax, -kFltMax };
 #pragma unroll
     for (int k = 0; k < kWheels; k++) {
@@ -1317,7 +1334,7 @@ DI void contactPrepare(ContactLdsT<Owners>& L, int lane, bool sat, V3 cen, Q4 ro
 template <int Owners, class Bodies>
 DI int contactFinishWith(const ContactLdsT<Owners>& L, int lane, V3 cen, Q4 rot, Wheels& w, Bodies bodies)
 {
-    const V3 up = rotate(rot, kZ);
+    const V3 up = rotateZ(rot);
     const V3 dir = -up;
     V3 start[kWheels];
 #pragma unroll
@@ -1411,10 +1428,10 @@ DI float nonStickyFriction(float z)
 DI void applySuspension(Body& b, CarRegs& r, const Wheels& w, int tick)
 {
     const float brakeTorque = r.brakePrev * (kCarMass * (14.25f + 1.f / 3.f));
-    const V3 up = rotate(b.rot, kZ);
+    const V3 up = rotateZ(b.rot);
     const V3 cenOffset = b.cen - b.pos;
-    const V3 fwd = rotate(b.rot, kX);
-    const V3 right = rotate(b.rot, kY);
+    const V3 fwd = rotateX(b.rot);
+    const V3 right = rotateY(b.rot);
     const V3 vel0 = b.vel, ang0 = b.ang;
     const V3 angCrossUp = cross(b.ang, up);
     const float pushDt = tick <= 1 ? kPushbackDtFirst : kDt;

@@ -142,6 +142,33 @@ HDI V3 rotate(Q4 q, V3 v)
     return (v + t * q.w) + cross(u, t);
 }
 HDI V3 unrotate(Q4 q, V3 v) { return rotate(qconj(q), v); }
+// rotate(q, kX), rotate(q, kY), rotate(q, kZ) without the products with the
+// axis's zeros: 14 operations instead of 27, the same bits.  A dropped term is
+// +-0 and only ever added to a sum that starts from the axis's +0 or 1 and is
+// therefore never -0, so it changes no bit; `zero` is +0, and NaN for a q
+// that is not finite or too short for 2 / |q|^2, as rotate's result is there.
+HDI float finiteZero(Q4 q)
+{
+    return __builtin_fmaf(q.x, 0.f, __builtin_fmaf(q.y, 0.f, __builtin_fmaf(q.z, 0.f, __builtin_fmaf(q.w, 0.f, 0.f))));
+}
+HDI V3 rotateX(Q4 q)
+{
+    const float k = 2.f / qdot(q, q), zero = finiteZero(q) * k;
+    const float ty = q.z * k, tz = -q.y * k;
+    return V3{ (zero + 1.f) + (q.y * tz - q.z * ty), (zero + ty * q.w) - q.x * tz, (zero + tz * q.w) + q.x * ty };
+}
+HDI V3 rotateY(Q4 q)
+{
+    const float k = 2.f / qdot(q, q), zero = finiteZero(q) * k;
+    const float tx = -q.z * k, tz = q.x * k;
+    return V3{ (zero + tx * q.w) + q.y * tz, (zero + 1.f) + (q.z * tx - q.x * tz), (zero + tz * q.w) - q.y * tx };
+}
+HDI V3 rotateZ(Q4 q)
+{
+    const float k = 2.f / qdot(q, q), zero = finiteZero(q) * k;
+    const float tx = q.y * k, ty = -q.x * k;
+    return V3{ (zero + tx * q.w) - q.z * ty, (zero + ty * q.w) + q.z * tx, (zero + 1.f) + (q.x * ty - q.y * tx) };
+}
 HDI Q4 yawQuat(float a)
 {
     float s, c;

@@ -220,9 +220,10 @@ DI WalkCost contactGroup(const Dev& d, const Handoff& out, int screen, int car, 
     if (ok) {
         if (d.nCars == 2)
             best = contactFinishWith(L, lane, cen, rot, w, [&](const V3* start, V3 dir, Wheels& ww) {
-                if (!odemoed && !(lensq(ocen - cen) > kCarRayReach * kCarRayReach))
+                const V3 mid = cen + dir * kRayMid;
+                if (!odemoed && !(lensq(ocen - mid) > kCarRayReach * kCarRayReach))
                     raycastCar(start, dir, ocen, orot, ww);
-                if (!(lensq(ball - cen) > kBallRayReach * kBallRayReach)) raycastBall(start, dir, ball, ww);
+                if (!(lensq(ball - mid) > kBallRayReach * kBallRayReach)) raycastBall(start, dir, ball, ww);
             });
         else
             best = contactFinish(d, L, lane, car, car / d.nCars, cen, rot, w);
@@ -266,9 +267,13 @@ __global__ __launch_bounds__(kContactBlock) void contactKernel(Dev d, uint32_t* 
 
 // A2: controls, car-arena contacts, suspension and the contact solve.
 // two waves per SIMD keep all of its waves resident at 65536 1v1 simulations
+// The stored controls are the same at every tick of a launch and nothing else
+// writes them, and of the stored wheel results only the last tick's are read
+// (by the outputs), so a launch of several ticks stores the controls at its
+// first and the wheels at its last.
 template <class Handoff>
 DI void carArenaCar(const Dev& d, const Handoff& in, int kind, const void* __restrict__ actions, int tick, int car,
-                    int lane)
+                    int lane, bool first, bool last)
 {
     Wheels w;
 #pragma unroll
@@ -290,15 +295,17 @@ DI void carArenaCar(const Dev& d, const Handoff& in, int kind, const void* __res
     const bool demoed = d.ci(CARL_CAR_DEMOED, car) != 0;
     CarRegs r;
     loadRegs(d, car, r);
-    storeWheelOutputs(d, car, w);
-    d.setf(CARL_CAR_CTRL_THROTTLE, car, ctl.throttle);
-    d.setf(CARL_CAR_CTRL_STEER, car, ctl.steer);
-    d.setf(CARL_CAR_CTRL_YAW, car, ctl.yaw);
-    d.setf(CARL_CAR_CTRL_PITCH, car, ctl.pitch);
-    d.setf(CARL_CAR_CTRL_ROLL, car, ctl.roll);
-    d.seti(CARL_CAR_CTRL_JUMP, car, ctl.jump);
-    d.seti(CARL_CAR_CTRL_BOOST, car, ctl.boost);
-    d.seti(CARL_CAR_CTRL_SLIDE, car, ctl.slide);
+    if (last) storeWheelOutputs(d, car, w);
+    if (first) {
+        d.setf(CARL_CAR_CTRL_THROTTLE, car, ctl.throttle);
+        d.setf(CARL_CAR_CTRL_STEER, car, ctl.steer);
+        d.setf(CARL_CAR_CTRL_YAW, car, ctl.yaw);
+        d.setf(CARL_CAR_CTRL_PITCH, car, ctl.pitch);
+        d.setf(CARL_CAR_CTRL_ROLL, car, ctl.roll);
+        d.seti(CARL_CAR_CTRL_JUMP, car, ctl.jump);
+        d.seti(CARL_CAR_CTRL_BOOST, car, ctl.boost);
+        d.seti(CARL_CAR_CTRL_SLIDE, car, ctl.slide);
+    }
     if (demoed) return;
     applyControls(r, ctl, w);
     solveCarArena(r, w, best >= 0, bestPt, tick);
@@ -311,7 +318,8 @@ __global__ __launch_bounds__(kTickBlock, 2) void carArenaKernel(Dev d, const uin
 {
     const int car = range.begin * d.nCars + blockIdx.x * kTickBlock + threadIdx.x;
     if (car < range.end * d.nCars)
-        carArenaCar(d, WsHandoff{ const_cast<uint32_t*>(ws), d.nTotal }, kind, actions, tick, car, (int)threadIdx.x & 63);
+        carArenaCar(d, WsHandoff{ const_cast<uint32_t*>(ws), d.nTotal }, kind, actions, tick, car,
+                    (int)threadIdx.x & 63, true, true);
 }
 
 // Episode clock and the car-car pairs of one simulation, (b, a) with b the
@@ -370,6 +378,7 @@ DI void ballGroup(const Dev& d, int tick, int sim, bool ok, BallLds& L, int lane
     int count = 0;
     bool hit = false;
     int roundBase = 0;
+    const int before = waveInclusiveScan(items) - items;   // this ball's first item
     waveItemsPipelined(
         items, L.excl, [&](int o, int q, bool valid) { return ballGatherFetch(d, L, o, q, valid); },
         [&](const BallItem& item, int o, int, int) { hit = ballGatherItem(L, item, o, lane); },
@@ -380,7 +389,7 @@ DI void ballGroup(const Dev& d, int tick, int sim, bool ok, BallLds& L, int lane
             const unsigned long long hits = __ballot(hit);
             hit = false;
             if (items > 0) {
-                const int a = L.excl[lane] - roundBase, b = L.excl[lane] + items - roundBase;
+                const int a = before - roundBase, b = before + items - roundBase;
                 if (b > 0 && a < 64) foldStashedContacts(L, hits, a > 0 ? a : 0, b < 64 ? b : 64, cs, count);
             }
             roundBase += 64;
@@ -687,10 +696,12 @@ DI void tickWindowBody(Dev d0, uint32_t* __restrict__ ws, int screen, int kind, 
         __syncthreads();
         mark(kStageContact);
         if constexpr (Balanced) {
-            carArenaCar(d, LdsHandoff{ L.wave[wave].hand }, kind, actions, tick, slotCar(t), lane);
+            carArenaCar(d, LdsHandoff{ L.wave[wave].hand }, kind, actions, tick, slotCar(t), lane, k == 0,
+                        k == ticks - 1);
         } else {
             for (int c = waveCar0 + lane; c < waveCarEnd; c += 64)
-                carArenaCar(d, LdsHandoff{ L.wave[wave].hand }, kind, actions, tick, c, lane);
+                carArenaCar(d, LdsHandoff{ L.wave[wave].hand }, kind, actions, tick, c, lane, k == 0,
+                            k == ticks - 1);
         }
         __syncthreads();
         mark(kStageCarArena);

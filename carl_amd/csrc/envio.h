@@ -30,8 +30,8 @@ DI void packCar(const Dev& d, int c, bool inv, float* o, int& k)
     put3(o, k, mirrorXY(d.cv(CARL_CAR_POS, c), inv));
     put3(o, k, mirrorXY(d.cv(CARL_CAR_VEL, c), inv));
     put3(o, k, mirrorXY(d.cv(CARL_CAR_ANG, c), inv));
-    put3(o, k, mirrorXY(rotate(rot, kX), inv));
-    put3(o, k, mirrorXY(rotate(rot, kZ), inv));
+    put3(o, k, mirrorXY(rotateX(rot), inv));
+    put3(o, k, mirrorXY(rotateZ(rot), inv));
     o[k++] = d.cf(CARL_CAR_BOOST, c);
     o[k++] = (float)d.ci(CARL_CAR_ON_GROUND, c);
     o[k++] = (float)(d.ci(CARL_CAR_DEMOED, c) != 0);

@@ -423,7 +423,7 @@ DI void carCarPair(const Dev& d, int ia, int ib, int tick)
         const bool grounded = aB ? gndB : gndA;
         const float fwdScale = grounded ? bumpCurve(closing, 5.f / 6.f, 1100.f, 1530.f)
                                         : bumpCurve(closing, 5.f / 6.f, 1390.f, 1945.f);
-        const V3 up = grounded ? rotate(aB ? bB.rot : bA.rot, kZ) : kZ;
+        const V3 up = grounded ? rotateZ(aB ? bB.rot : bA.rot) : kZ;
         const V3 imp = velDir * fwdScale + up * bumpCurve(closing, 2.f / 6.f, 278.f, 417.f);
         d.setv(CARL_CAR_IMP, victim, (aB ? impB : impA) + imp);
         d.seti(CARL_CAR_CONTACT_IDX, bumper, victim);
@@ -1219,7 +1219,7 @@ DI bool ballCarPair(const Dev& d, int sim, int c, V3 preBallVel, int tick, V3& b
         const float hl = lensq(hd);
         if (hl > 1e-12f) {
             hd = hd * rsqrt_(hl);
-            const V3 fwd = rotate(rot, kX);
+            const V3 fwd = rotateX(rot);
             hd = hd - fwd * (dot(hd, fwd) * (1.f - kExtraFwdScale));
             const float al = lensq(hd);
             if (al > 1e-12f) hd = hd * rsqrt_(al);

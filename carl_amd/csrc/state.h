@@ -75,17 +75,23 @@ DI Tri unpackTri(const float4* rec)
 DI Tri loadTri(const ArenaView& a, int ref) { return unpackTri(a.rec + 4 * (size_t)ref); }
 DI Tri loadTriIdx(const ArenaView& a, int idx) { return unpackTri(a.tri + 4 * (size_t)idx); }
 
+// max(x, 0) / c as the correctly rounded quotient, by a reciprocal and one
+// residual step (4 operations where the division's own scaling takes 10; the
+// three cell sizes checked against / for every float in [0, 1e5]).  Beyond
+// 1e5 the caller's clamp to the grid decides, and there x is held at 1e5.
+HDI float overCell(float x, float c)
+{
+    const float r = 1.f / c;   // folded: c is a constant
+    x = fmin_(fmax_(x, 0.f), 1e5f);
+    const float q = x * r;
+    return __builtin_fmaf(__builtin_fmaf(-q, c, x), r, q);
+}
+
 HDI void cellOf(V3 p, int& cx, int& cy, int& cz)
 {
-    float x = (p.x - kArenaMin.x) / kCellX;
-    float y = (p.y - kArenaMin.y) / kCellY;
-    float z = (p.z - kArenaMin.z) / kCellZ;
-    x = fmin_(fmax_(x, 0.f), 48.f - 1.f);
-    y = fmin_(fmax_(y, 0.f), 48.f - 1.f);
-    z = fmin_(fmax_(z, 0.f), 10.f - 1.f);
-    cx = (int)x;
-    cy = (int)y;
-    cz = (int)z;
+    cx = (int)fmin_(overCell(p.x - kArenaMin.x, kCellX), 48.f - 1.f);
+    cy = (int)fmin_(overCell(p.y - kArenaMin.y, kCellY), 48.f - 1.f);
+    cz = (int)fmin_(overCell(p.z - kArenaMin.z, kCellZ), 10.f - 1.f);
 }
 HDI int flatCell(int cx, int cy, int cz) { return cx + cy * kGridX + cz * kGridX * kGridY; }
 
