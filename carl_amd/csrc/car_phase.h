@@ -184,15 +184,27 @@ DI void raycastBodies(const Dev& d, int car, int sim, V3 cen, const V3* start, V
     const int base = sim * d.nCars;
     const V3 ball = d.sv(CARL_SIM_BALL_POS, sim);
     const V3 mid = cen + dir * kRayMid;
-    for (int o = 0; o < d.nCars; o++) {
-        const int oc = base + o;
-        // the other car's words are loaded together, before its demolished
-        // flag is tested (one round trip instead of two)
-        const int demoed = d.ci(CARL_CAR_DEMOED, oc);
-        const V3 ocen = d.cv(CARL_CAR_CEN, oc);
-        const Q4 orot = d.cq(CARL_CAR_ROT, oc);
-        if (oc == car || demoed || lensq(ocen - mid) > kCarRayReach * kCarRayReach) continue;
-        raycastCar(start, dir, ocen, orot, w);
+    // every car's centre and flag are loaded before the first is tested (one
+    // round trip instead of one per car)
+    V3 ocen[kMaxCars];
+    bool out[kMaxCars];
+#pragma unroll
+    for (int o = 0; o < kMaxCars; o++) {
+        out[o] = true;
+        ocen[o] = kZero;
+        if (o < d.nCars) {
+            out[o] = d.ci(CARL_CAR_DEMOED, base + o) != 0;
+            ocen[o] = d.cv(CARL_CAR_CEN, base + o);
+        }
+    }
+    unsigned near = 0;
+#pragma unroll
+    for (int o = 0; o < kMaxCars; o++)
+        if (!out[o] && base + o != car && !(lensq(ocen[o] - mid) > kCarRayReach * kCarRayReach)) near |= 1u << o;
+    while (near) {
+        const int o = __builtin_ctz(near);
+        near &= near - 1;
+        raycastCar(start, dir, d.cv(CARL_CAR_CEN, base + o), d.cq(CARL_CAR_ROT, base + o), w);
     }
     if (!(lensq(ball - mid) > kBallRayReach * kBallRayReach)) raycastBall(start, dir, ball, w);
 }

@@ -215,8 +215,10 @@ HDI float respawnX(int i) { return i == 0 ? 2688.f : (i == 1 ? 2304.f : (i == 2 
 constexpr float kRespawnY = -4608.f;
 constexpr float kRespawnYaw = kPi2 * 1;
 
+constexpr int kMaxCars = 8;   // per simulation
+
 // boost pad positions (x, y, z) - big pads first
-static __device__ __constant__ const float kPadPos[kPads][3] = {
+static __device__ __constant__ constexpr float kPadPos[kPads][3] = {
     { -3584.f, 0.f, 73.f }, { 3584.f, 0.f, 73.f }, { -3072.f, 4096.f, 73.f }, { 3072.f, 4096.f, 73.f },
     { -3072.f, -4096.f, 73.f }, { 3072.f, -4096.f, 73.f },
     { 0.f, -4240.f, 70.f }, { -1792.f, -4184.f, 70.f }, { 1792.f, -4184.f, 70.f }, { -940.f, -3308.f, 70.f },

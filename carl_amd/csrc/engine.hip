@@ -323,13 +323,65 @@ __global__ __launch_bounds__(kTickBlock, 2) void carArenaKernel(Dev d, const uin
 }
 
 // Episode clock and the car-car pairs of one simulation, (b, a) with b the
-// later car (Kernels.cu:42-55, CarCar/Solve.cuh:63-151).
-DI void carCarSim(const Dev& d, int sim, int tick)
+// later car (Kernels.cu:42-55, CarCar/Solve.cuh:63-151).  Returns, for more
+// than two cars, how many pairs came within twice the pair test's distance
+// bound (what they may cost soon).
+//
+// With more than two cars the pairs' distance tests run first, on centres and
+// flags loaded in one batch; then the pairs that passed are taken in order.
+// A solved pair moves its cars, so the pairs after it that share one are taken
+// too: the pair's own test decides on the poses of the moment, as in the plain
+// double loop (whose loads, a round trip per pair, are 28 in 4v4).
+DI int carCarSim(const Dev& d, int sim, int tick)
 {
     d.sseti(CARL_SIM_EPISODE_TICKS, sim, d.si(CARL_SIM_EPISODE_TICKS, sim) + 1);
-    const int base = sim * d.nCars;
-    for (int a = 0; a < d.nCars - 1; a++)
-        for (int b = a + 1; b < d.nCars; b++) carCarPair(d, base + b, base + a, tick);
+    const int n = d.nCars, base = sim * n;
+    if (n == 2) {
+        carCarPair(d, base + 1, base, tick);
+        return 0;
+    }
+    V3 cen[kMaxCars];
+    bool demoed[kMaxCars];
+#pragma unroll
+    for (int k = 0; k < kMaxCars; k++) {
+        demoed[k] = true;
+        cen[k] = kZero;
+        if (k < n) {
+            demoed[k] = d.ci(CARL_CAR_DEMOED, base + k) != 0;
+            cen[k] = d.cv(CARL_CAR_CEN, base + k);
+        }
+    }
+    const float maxDist = 2.f * len(kHalf);
+    unsigned due[kMaxCars];   // per first car a: its later cars b still to be taken
+    int close = 0;
+#pragma unroll
+    for (int a = 0; a < kMaxCars; a++) {
+        due[a] = 0;
+#pragma unroll
+        for (int b = a + 1; b < kMaxCars; b++) {
+            if (b >= n || demoed[a] || demoed[b]) continue;
+            const float sq = lensq(cen[a] - cen[b]);
+            if (!(sq > maxDist * maxDist)) due[a] |= 1u << b;
+            close += sq < 4.f * (maxDist * maxDist) ? 1 : 0;
+        }
+    }
+    unsigned any = 0;
+#pragma unroll
+    for (int a = 0; a < kMaxCars; a++) any |= due[a];
+    if (any == 0) return close;
+    unsigned moved = 0;   // cars that a solve has moved or demolished
+    for (int a = 0; a < n - 1; a++) {
+        unsigned mine = 0;
+#pragma unroll
+        for (int k = 0; k < kMaxCars; k++)
+            if (k == a) mine = due[k];
+        for (int b = a + 1; b < n; b++) {
+            const unsigned both = 1u << a | 1u << b;
+            if (((mine >> b) & 1u) == 0 && (moved & both) == 0) continue;
+            if (carCarPair(d, base + b, base + a, tick)) moved |= both;
+        }
+    }
+    return close;
 }
 
 // B: per simulation the episode clock and the car-car pairs, then ball-arena
@@ -342,22 +394,22 @@ DI void carCarSim(const Dev& d, int sim, int tick)
 constexpr int kBallBlock = 64;
 constexpr int kBallOwners = 32;
 
-// One simulation per lane of the first kBallOwners (sim, where ok) by one
-// wave; L is that wave's own LDS.  Every lane of the wave calls it; it
-// synchronises the wave only.  With Native (arena metadata) each owner lane
-// gathers and solves its ball against the native meshes alone.
+// One simulation per lane (sim, where ok) by one wave; L is that wave's own
+// LDS.  Every lane of the wave calls it; it synchronises the wave only.  With
+// Native (arena metadata) each owner lane gathers and solves its ball against
+// the native meshes alone.  Returns carCarSim's count of close pairs.
 template <bool Native>
-DI void ballGroup(const Dev& d, int tick, int sim, bool ok, BallLds& L, int lane)
+DI int ballGroup(const Dev& d, int tick, int sim, bool ok, BallLds& L, int lane)
 {
-    ok = ok && lane < kBallOwners;
+    int pairs = 0;
     if constexpr (Native) {
         if (ok) {
             carCarSim(d, sim, tick);
             nativeBallTick(d, sim, tick);
         }
-        return;
+        return 0;
     }
-    if (ok) carCarSim(d, sim, tick);
+    if (ok) pairs = carCarSim(d, sim, tick);
     const bool awake = ok && !ballSleeping(d, sim);
     const V3 center = ok ? d.sv(CARL_SIM_BALL_POS, sim) : kZero;
     int items = 0, first = 0, cell = 0;
@@ -397,16 +449,17 @@ DI void ballGroup(const Dev& d, int tick, int sim, bool ok, BallLds& L, int lane
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         });
-    if (!ok) return;
+    if (!ok) return 0;
     if (sequential) count = gatherBallContacts(d, center, cs);
     ballTick(d, sim, tick, cs, count);
+    return pairs;
 }
 
 __global__ __launch_bounds__(kBallBlock) void ballKernel(Dev d, int tick, SimRange range)
 {
     __shared__ BallLds L;
     const int sim = range.begin + blockIdx.x * kBallOwners + (int)threadIdx.x;
-    ballGroup<false>(d, tick, sim, sim < range.end, L, threadIdx.x);
+    ballGroup<false>(d, tick, sim, threadIdx.x < kBallOwners && sim < range.end, L, threadIdx.x);
 }
 
 // the same with the native arena meshes
@@ -414,7 +467,7 @@ __global__ __launch_bounds__(kBallBlock) void ballNativeKernel(Dev d, int tick, 
 {
     __shared__ BallLds L;
     const int sim = range.begin + blockIdx.x * kBallOwners + (int)threadIdx.x;
-    ballGroup<true>(d, tick, sim, sim < range.end, L, threadIdx.x);
+    ballGroup<true>(d, tick, sim, threadIdx.x < kBallOwners && sim < range.end, L, threadIdx.x);
 }
 
 // C + D: integration and impulse caches of every car and ball, then the
@@ -504,52 +557,43 @@ enum ProfWord {
     kProfWords
 };
 
-// Balanced 1v1 and 2v2 launches deal the simulations to the workgroups in
-// units of kUnitCars cars (dealUnitSims consecutive simulations): slot s
-// of workgroup b (wave 2 b + s / kWaveUnits) holds one unit, its cars in
-// kUnitCars consecutive lanes and its balls in as many lanes as it has
-// simulations.  Simulations share nothing, so the deal changes no result; it
-// is made so that the workgroups finish together.  A unit's cars fill whole
-// 128-byte lines of every car field (1v1 units of 8 simulations left half
-// lines to workgroups on other XCDs, whose L2s then fetched the same lines:
-// the launch read 2.5 times the bytes).
+// A window launch's simulations go to its waves in units of unitSims
+// consecutive simulations (WindowMap): wave w holds the simulations of at most
+// `rounds` units, their cars in consecutive lanes (at most 64) and their balls
+// likewise.  Simulations share nothing and every phase of a simulation runs in
+// its own wave, so the waves wait for nobody: each runs its ticks from end to
+// end with no workgroup barrier.
 //
-// The deal needs no pass of its own.  At its last tick every launch files
-// each unit under the class of its cost (dealClass) in an output list: one
-// atomic per unit on a count, then the unit at that position of the list.
-// Each class has kDealSubs lists, unit u going to list u % kDealSubs, so
-// that units of equal cost (the kickoffs, early on) do not all wait on one
-// count.  The next launch reads the lists back in rank order, costliest
-// class first (any order within a class), and deals them to the
-// waves in rounds: round 0 gives the costliest units, one to each wave in
-// order; every later round gives its units in reverse order, so that the
-// waves holding the costliest units get the cheapest of each round (the
-// costs have a long tail: a car whose box meets the arena every tick, a pair
-// that may collide).  Two units of pairs that may collide thus fall to the
-// two waves of one workgroup, whose pair solves run side by side.  Three
-// list sets rotate: launch L reads set L % 3, files into set (L + 1) % 3
-// (cleared by launch L - 1) and clears the counts of set (L + 2) % 3, which
-// no launch touches again before L + 1.
-constexpr int kUnitCars = 32;                            // one 128-byte line of each car field
-constexpr int kUnitSlots = 4;                            // units per balanced workgroup
-constexpr int kWaveUnits = kUnitSlots / 2;               // units per wave
-// simulations per unit and per balanced workgroup, by cars per simulation
-// (0: no balanced launch)
-HDI constexpr int dealUnitSims(int cars) { return cars == 2 || cars == 4 ? kUnitCars / cars : 0; }
-HDI constexpr int dealBlockSims(int cars) { return kUnitSlots * dealUnitSims(cars); }
+// A dealt launch gives out the units so that the waves finish together.  At
+// its last tick every launch files each unit under the class of its cost
+// (dealClass) in an output list: one atomic per unit on a count, then the
+// unit at that position of the list.  Each class has kDealSubs lists, unit u
+// going to list u % kDealSubs, so that units of equal cost (the kickoffs,
+// early on) do not all wait on one count.  The next launch reads the lists
+// back in rank order, costliest class first (any order within a class), and
+// deals them to the waves in rounds: round 0 gives the costliest units, one to
+// each wave in order; every later round gives its units in reverse order, so
+// that the waves holding the costliest units get the cheapest of each round,
+// or none where the units do not go round (the costs have a long tail: a car
+// whose box meets the arena every tick, a pair that may collide).  Three list
+// sets rotate: launch L reads set L % 3, files into set (L + 1) % 3 (cleared
+// by launch L - 1) and clears the counts of set (L + 2) % 3, which no launch
+// touches again before L + 1.
+constexpr int kUnitCars = 32;        // cars of a unit of a large run: one 128-byte line of each car field
+constexpr int kMaxWaveUnits = 16;    // units a wave may hold
 constexpr int kDealClasses = 32;
 constexpr int kDealSubs = 4;
 constexpr int kDealLists = kDealClasses * kDealSubs;
-constexpr int kListsPerThread = kDealLists / 128;   // of a balanced workgroup's threads, in the deal's scan
+constexpr int kListsPerLane = kDealLists / 64;   // of a wave's lanes, in the deal's scan
 constexpr int kDealSets = 3;
 // A unit's cost is its contact work in the launch's last tick, in candidate
 // items (each about 0.04 us of its wave's time).  A car whose box met the
 // arena costs its wave about 6 us of contact generation (160 items),
 // counted at half, kSatCost, since it persists less from one launch to the
 // next than a candidate count does; a pair that may collide (cars within
-// twice their box diagonal) costs about 25 us per tick of its serial solve,
-// kPairCost items.  (The cost summed over the launch's ticks ranked the
-// units no better.)
+// twice the pair test's distance bound) costs about 25 us per tick of its
+// serial solve, kPairCost items.  (The cost summed over the launch's ticks
+// ranked the units no better.)
 constexpr int kSatCost = 80;
 constexpr int kPairCost = 720;
 
@@ -560,305 +604,343 @@ DI int dealClass(int cost)
     return min(kDealClasses - 1, 1 + (int)(4.f * __log2f((float)cost * (1.f / 8.f))));
 }
 
-// list k = kDealSubs c + j of a set holds up to nUnits / kDealSubs units
-// from outList + k nUnits / kDealSubs, its count at outCount[k]
+// Workgroups are handed to the 8 XCDs in turn, each with an L2 of its own, so
+// consecutive shares would put the cars of one cache line on several XCDs.
+// The units are therefore parted into contiguous groups, one per XCD, group g
+// for the workgroups b with b % groups == g, and each group is dealt among its
+// own waves.  (Were the workgroups handed out otherwise, only the locality
+// would be lost.)  Launches of more workgroups than are resident run as one
+// group, in order through memory.
+constexpr int kXcds = 8;
+HDI int groupBlocksBefore(int blocks, int groups, int g)
+{
+    return g * (blocks / groups) + (g < blocks % groups ? g : blocks % groups);
+}
+HDI int groupFirstUnit(int nUnits, int blocks, int groups, int g)
+{
+    return (int)((long long)nUnits * groupBlocksBefore(blocks, groups, g) / blocks);
+}
+
+// list k = kDealSubs c + j of group g in a set holds up to listLen units from
+// outList + (g kDealLists + k) listLen, its count at outCount[g kDealLists + k]
 struct WindowMap {
-    const int* inCount;   // the deal's counts and lists (null: slot s of workgroup b holds unit 4 b + s)
+    const int* inCount;   // the deal's counts and lists (null: a group's units go to its waves in order)
     const int* inList;
-    int* outCount;        // this launch's filing
+    int* outCount;        // this launch's filing (null: none)
     int* outList;
     int* clearCount;      // the counts the next launch files into
-    int nUnits;
+    int unitSims, nUnits, rounds, listLen, groups;
 };
 
-// The window kernel's body.  With Profile, thread 0 of each workgroup reads
-// the wall clock (the constant-rate counter) at the start and after every
-// phase barrier; a phase's time runs from the barrier before it to its own,
-// barrier wait included.  At the end each workgroup adds its phase times to
-// the kProfStages sums, and the launch's last workgroup to finish adds its
-// own phase times, its start delay and the launch's span.  Without Profile
-// the code is the plain kernel.
-template <bool Profile, bool Native, int Cars, bool Balanced>
-DI void tickWindowBody(Dev d0, uint32_t* __restrict__ ws, int screen, int kind, const void* __restrict__ actions,
-                       int tick0, int ticks, int simsPerBlock, SimRange range, WindowMap map,
-                       unsigned long long* __restrict__ prof)
+// What a wave of the window kernel keeps in LDS about its share.
+struct WaveShare {
+    int car[64];                  // the car of each lane (-1: none)
+    int sim[64];                  // the simulation whose ball each lane takes (-1: none)
+    int unit[kMaxWaveUnits];      // -1: none
+    int cost[kMaxWaveUnits];
+    unsigned long long stage[kWindowStages], first, last;   // stage profile
+};
+
+// The window kernel's body, for one wave.  With prof, lane 0 reads the wall
+// clock (the constant-rate counter) at the start and after every phase.  At
+// the end each wave adds its phase times to the kProfStages sums, and the
+// launch's last wave to finish adds its own phase times, its start delay and
+// the launch's span.
+template <int Cars>
+DI void tickWindowBody(const Dev& d0, int screen, int kind, const void* __restrict__ actions, int tick0, int ticks,
+                       SimRange range, const WindowMap& map, unsigned long long* __restrict__ prof, WaveLds& L,
+                       WaveShare& m, int wave, int lane)
 {
-    static_assert(!Balanced || dealUnitSims(Cars) > 0, "balanced launches are 1v1 or 2v2");
-    constexpr int kUnitSims = Balanced ? dealUnitSims(Cars) : 1, kBlockSims = kUnitSlots * kUnitSims;
-    static_assert(kWindowBlock == 2 * 64 && kWaveUnits * kUnitCars == 64 && kWaveUnits * kUnitSims <= kBallOwners,
-                  "a balanced wave holds kWaveUnits units: 64 cars, at most kBallOwners balls");
     // a fixed car count (Cars > 0) lets every per-simulation loop fold
     Dev d = d0;
     if constexpr (Cars > 0) d.nCars = Cars;
-    __shared__ WindowLds L;
-    __shared__ int unit[Balanced ? kUnitSlots : 1];
-    const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
-    // balanced: the car of thread (or contact owner) i, the simulation of
-    // workgroup position j (ball owners, finish and pads)
-    auto slotCar = [&](int i) { return unit[i / kUnitCars] * kUnitCars + i % kUnitCars; };
-    auto slotSim = [&](int j) { return unit[j / kUnitSims] * kUnitSims + j % kUnitSims; };
-    if constexpr (Balanced) {
-        if (map.inCount) {
-            // the lists' first ranks, costliest class first, in the LDS the
-            // contact phase takes over afterwards; each thread scans
-            // kListsPerThread of them: lists k in rank order hold class
-            // kDealClasses - 1 - k / kDealSubs
-            static_assert(kListsPerThread * kWindowBlock == kDealLists && kDealLists * sizeof(int) <= sizeof(WaveLds),
-                          "the deal's scan: whole lists per thread, in one wave's LDS");
-            int* first = reinterpret_cast<int*>(&L.wave[0]);
-            __shared__ int waveSum[kWindowWaves];
-            int n[kListsPerThread], sum = 0;
+    // this wave among its group's waves, and the group's units
+    const int blocks = (int)gridDim.x, groups = map.groups, group = (int)blockIdx.x % groups;
+    const int wv = (int)blockIdx.x / groups * kWindowWaves + wave;
+    const int waves = (groupBlocksBefore(blocks, groups, group + 1) - groupBlocksBefore(blocks, groups, group)) * kWindowWaves;
+    const int unit0 = groupFirstUnit(map.nUnits, blocks, groups, group);
+    const int nUnits = groupFirstUnit(map.nUnits, blocks, groups, group + 1) - unit0;
+    if (lane < kMaxWaveUnits) {
+        m.unit[lane] = -1;
+        m.cost[lane] = 0;
+    }
+    waveSync();
+    if (map.inCount) {
+        // the lists' first ranks, costliest class first, in the LDS the
+        // contact phase takes over afterwards; each lane scans kListsPerLane
+        // of them: list k in rank order holds class kDealClasses - 1 - k / kDealSubs
+        static_assert(kListsPerLane * 64 == kDealLists && kDealLists * sizeof(int) <= sizeof(WaveLds),
+                      "the deal's scan: whole lists per lane, in one wave's LDS");
+        int* first = reinterpret_cast<int*>(&L);
+        int n[kListsPerLane], sum = 0;
 #pragma unroll
-            for (int i = 0; i < kListsPerThread; i++) {
-                const int k = kListsPerThread * t + i;
-                n[i] = map.inCount[(kDealClasses - 1 - k / kDealSubs) * kDealSubs + k % kDealSubs];
-                sum += n[i];
-            }
-            int incl = sum;
-            for (int o = 1; o < 64; o <<= 1) {
-                const int y = __shfl_up(incl, o);
-                if (lane >= o) incl += y;
-            }
-            if (lane == 63) waveSum[wave] = incl;
-            __syncthreads();
-            int r = incl - sum;
-            for (int v = 0; v < wave; v++) r += waveSum[v];
+        for (int i = 0; i < kListsPerLane; i++) {
+            const int k = kListsPerLane * lane + i;
+            n[i] = map.inCount[group * kDealLists + (kDealClasses - 1 - k / kDealSubs) * kDealSubs + k % kDealSubs];
+            sum += n[i];
+        }
+        int r = waveInclusiveScan(sum) - sum;
 #pragma unroll
-            for (int i = 0; i < kListsPerThread; i++) {
-                first[kListsPerThread * t + i] = r;
-                r += n[i];
-            }
-            __syncthreads();
-            if (t < kUnitSlots) {
-                const int waves = map.nUnits / kWaveUnits, wv = 2 * blockIdx.x + t / kWaveUnits, r = t % kWaveUnits;
-                const int rank = r == 0 ? wv : r * waves + (waves - 1 - wv);
+        for (int i = 0; i < kListsPerLane; i++) {
+            first[kListsPerLane * lane + i] = r;
+            r += n[i];
+        }
+        waveSync();
+        if (lane < map.rounds) {
+            const int rank = lane == 0 ? wv : lane * waves + (waves - 1 - wv);
+            if (rank < nUnits) {
                 // the last list whose first rank is at most rank
                 int lo = 0;
                 for (int step = kDealLists / 2; step > 0; step >>= 1)
                     if (lo + step < kDealLists && first[lo + step] <= rank) lo += step;
-                const int per = map.nUnits / kDealSubs;
                 const int k = (kDealClasses - 1 - lo / kDealSubs) * kDealSubs + lo % kDealSubs;
-                unit[t] = map.inList[(size_t)k * per + min(rank - first[lo], per - 1)];
+                m.unit[lane] = map.inList[(size_t)(group * kDealLists + k) * map.listLen + min(rank - first[lo], map.listLen - 1)];
             }
-            __syncthreads();   // the scan's LDS is the contact phase's
-        } else if (t < kUnitSlots) {
-            unit[t] = blockIdx.x * kUnitSlots + t;
         }
-        if (blockIdx.x == 0) {
-#pragma unroll
-            for (int i = 0; i < kListsPerThread; i++) map.clearCount[kListsPerThread * t + i] = 0;
-        }
-        __syncthreads();
+    } else if (lane < map.rounds) {
+        const int u = wv * map.rounds + lane;
+        m.unit[lane] = u < nUnits ? unit0 + u : -1;
     }
-    const int sim0 = range.begin + blockIdx.x * simsPerBlock;
-    const int simEnd = min(sim0 + simsPerBlock, range.end);
-    const int car0 = sim0 * d.nCars, carEnd = simEnd * d.nCars;
-    // Undealt: the block's cars split evenly between the waves, whole pairs
-    // of cars to each (a 1v1 simulation's two cars sit in lanes 2i, 2i + 1).
-    // A block that is not full (a small run) would otherwise leave all of its
-    // cars to the first wave: window launch of 2v2 at 10,007 simulations 662
-    // -> 616 us, 4v4 at 4,099 806 -> 735 us, 1v0 at 30,011 308 -> 282 us.
-    const int waveCars = (carEnd - car0 + 2 * kWindowWaves - 1) / (2 * kWindowWaves) * 2;
-    const int waveCar0 = car0 + wave * waveCars, waveCarEnd = min(waveCar0 + waveCars, carEnd);
-    unsigned long long acc[kWindowStages] = {}, first = 0, last = 0;
+    if (map.clearCount && wv == 0) {
+#pragma unroll
+        for (int i = 0; i < kListsPerLane; i++) map.clearCount[group * kDealLists + kListsPerLane * lane + i] = 0;
+    }
+    waveSync();
+    // each lane's car, and the simulation whose ball it takes
+    {
+        const int unitCars = map.unitSims * d.nCars, slot = lane / unitCars, at = lane - slot * unitCars;
+        int car = -1, sim = -1;
+        if (slot < map.rounds && m.unit[slot] >= 0) {
+            const int s = range.begin + m.unit[slot] * map.unitSims + at / d.nCars;
+            if (s < range.end) car = s * d.nCars + at % d.nCars;
+        }
+        const int bslot = lane / map.unitSims;
+        if (bslot < map.rounds && m.unit[bslot] >= 0) {
+            const int s = range.begin + m.unit[bslot] * map.unitSims + (lane - bslot * map.unitSims);
+            if (s < range.end) sim = s;
+        }
+        m.car[lane] = car;
+        m.sim[lane] = sim;
+    }
+    if (prof && lane == 0) {
+        for (int st = 0; st < kWindowStages; st++) m.stage[st] = 0;
+        m.first = m.last = wall_clock64();
+    }
+    waveSync();
     auto mark = [&](int stage) {
-        if constexpr (Profile) {
-            if (t == 0) {
-                const unsigned long long now = wall_clock64();
-                acc[stage] += now - last;
-                last = now;
-            }
+        if (prof && lane == 0) {
+            const unsigned long long now = wall_clock64();
+            m.stage[stage] += now - m.last;
+            m.last = now;
         }
     };
-    if constexpr (Profile) {
-        if (t == 0) first = last = wall_clock64();
-    }
+    int padTick = 0;   // ticks since the cooldowns were last counted down
     for (int k = 0; k < ticks; k++) {
         const int tick = tick0 + k;
-        if constexpr (Balanced) {
+        const bool file = k == ticks - 1 && map.outCount != nullptr;
+        {
+            const int car = m.car[lane];
             const WalkCost c = contactGroup<kWindowContactLead, kWindowContactOwners>(
-                d, LdsHandoff{ L.wave[wave].hand }, screen, slotCar(t), true, L.wave[wave].contact, lane);
-            if (k == ticks - 1) {
-                // the unit's cost for the next deal (a pair counted at its first car)
-                int w = c.items + (c.sat ? kSatCost : 0) + (c.near && (lane & 1) == 0 ? kPairCost : 0);
-                for (int o = kUnitCars / 2; o > 0; o >>= 1) w += __shfl_xor(w, o);
-                if (lane % kUnitCars == 0) {
-                    const int u = unit[t / kUnitCars], l = dealClass(w) * kDealSubs + u % kDealSubs;
-                    map.outList[(size_t)l * (map.nUnits / kDealSubs) + atomicAdd(&map.outCount[l], 1)] = u;
-                }
+                d, LdsHandoff{ L.hand }, screen, max(car, 0), car >= 0, L.contact, lane);
+            if (file && car >= 0) {
+                // the unit's cost for the next deal (in 1v1 a close pair counted at its first car)
+                const int w = c.items + (c.sat ? kSatCost : 0) + (c.near && (lane & 1) == 0 ? kPairCost : 0);
+                atomicAdd(&m.cost[lane / (map.unitSims * d.nCars)], w);
             }
-        } else {
-            for (int g = waveCar0; g < waveCarEnd; g += kWindowContactOwners)
-                contactGroup<kWindowContactLead, kWindowContactOwners>(d, LdsHandoff{ L.wave[wave].hand }, screen,
-                                                                         g + lane, g + lane < waveCarEnd,
-                                                                         L.wave[wave].contact, lane);
         }
-        __syncthreads();
+        waveSync();
         mark(kStageContact);
-        if constexpr (Balanced) {
-            carArenaCar(d, LdsHandoff{ L.wave[wave].hand }, kind, actions, tick, slotCar(t), lane, k == 0,
-                        k == ticks - 1);
-        } else {
-            for (int c = waveCar0 + lane; c < waveCarEnd; c += 64)
-                carArenaCar(d, LdsHandoff{ L.wave[wave].hand }, kind, actions, tick, c, lane, k == 0,
-                            k == ticks - 1);
+        {
+            const int car = m.car[lane];
+            if (car >= 0)
+                carArenaCar(d, LdsHandoff{ L.hand }, kind, actions, tick, car, lane, k == 0, k == ticks - 1);
         }
-        __syncthreads();
+        waveSync();
         mark(kStageCarArena);
-        if constexpr (Balanced) {
-            constexpr int kWaveSims = kWaveUnits * kUnitSims;
-            ballGroup<Native>(d, tick, slotSim(kWaveSims * wave + lane % kWaveSims), lane < kWaveSims,
-                              L.wave[wave].ball, lane);
-        } else {
-            // the block's simulations split evenly between the waves (a
-            // block of 21 3v3 or 32 2v2 simulations would otherwise leave
-            // the second wave idle): at most kBallOwners per wave and group
-            const int per = (simEnd - sim0 + kWindowWaves - 1) / kWindowWaves;
-            const int wEnd = min(sim0 + (wave + 1) * per, simEnd);
-            for (int g = sim0 + wave * per; g < wEnd; g += kBallOwners)
-                ballGroup<Native>(d, tick, g + lane, g + lane < wEnd, L.wave[wave].ball, lane);
+        {
+            const int sim = m.sim[lane];
+            const int pairs = ballGroup<false>(d, tick, max(sim, 0), sim >= 0, L.ball, lane);
+            if (file && pairs > 0) atomicAdd(&m.cost[lane / map.unitSims], pairs * kPairCost);
         }
-        __syncthreads();
+        waveSync();
         mark(kStageBall);
-        if constexpr (Balanced) {
-            finishCar(d, slotCar(t));
-            if (t < kBlockSims) finishBall(d, slotSim(t));
-        } else {
-            for (int c = waveCar0 + lane; c < waveCarEnd; c += 64) finishCar(d, c);
-            for (int s = sim0 + t; s < simEnd; s += kWindowBlock) finishBall(d, s);
+        const int car = m.car[lane];
+        FinishedCar f{ kZero, false };
+        {
+            const int sim = m.sim[lane];
+            if (car >= 0) f = finishCar(d, car);
+            if (sim >= 0) finishBall(d, sim);
         }
-        __syncthreads();
+        waveSync();
         mark(kStageFinish);
-        if constexpr (Balanced) {
-            int tp = t;
-            asm volatile("" : "+v"(tp));
-            constexpr int kParts = kWindowBlock / kBlockSims;   // pad ranges per simulation
-            const int q = tp / kBlockSims, j = tp - q * kBlockSims;
-            if constexpr (kParts == kWindowWaves && Cars > 0) {
-                // one pad range per wave (1v1), fixed at compile time: each
-                // wave loads only its own pads' cooldowns (1,000-step bench:
-                // pad phase 5.0 -> 4.4 us per tick)
-                static_assert(kPads % 2 == 0, "two equal pad ranges");
-                if (__builtin_amdgcn_readfirstlane(wave) == 0)
-                    boostPadsRangeT<Cars, 0, kPads / 2>(d, slotSim(j), 0, kPads / 2);
-                else
-                    boostPadsRangeT<Cars, kPads / 2, kPads>(d, slotSim(j), kPads / 2, kPads);
-            } else {
-                boostPadsSpan(d, slotSim(j), kPads * q / kParts, kPads * (q + 1) / kParts, kParts);
-            }
-        } else {
-            // boost pads: the workgroup's threads split into kWindowBlock /
-            // simsPerBlock parts, each taking a contiguous range of every
-            // simulation's pads (in 1v1 two parts, one wave each).  The
-            // split is derived here from a copy of the thread index that the
-            // optimiser cannot hoist, so it holds no registers through the
-            // other phases.
-            int tp = t;
-            asm volatile("" : "+v"(tp));
-            const int parts = kWindowBlock / simsPerBlock, q = tp / simsPerBlock, j = tp - q * simsPerBlock;
-            if (parts == kWindowWaves) {
-                // one range per wave (at most two cars per simulation): fixed
-                // at compile time, as in dealt 1v1 launches
-                if (j < simEnd - sim0) {
-                    if (__builtin_amdgcn_readfirstlane(wave) == 0)
-                        boostPadsRangeT<2, 0, kPads / 2>(d, sim0 + j, 0, kPads / 2);
-                    else
-                        boostPadsRangeT<2, kPads / 2, kPads>(d, sim0 + j, kPads / 2, kPads);
-                }
-            } else if (q < parts && j < simEnd - sim0) {
-                boostPadsSpan(d, sim0 + j, kPads * q / parts, kPads * (q + 1) / parts, parts);
-            }
+        padPickups(d, max(car, 0), f, padTick);
+        if (++padTick == kPadTicks || k == ticks - 1) {
+            // the pads' cooldowns, by the lanes left over per simulation,
+            // each a range of its pads; the ranges are derived from a copy of
+            // the lane that the optimiser cannot hoist out of the tick loop,
+            // where they would hold registers (43 of them, spilled)
+            waveSync();
+            int l = lane;
+            asm volatile("" : "+v"(l));
+            const int n = map.rounds * map.unitSims, parts = 64 / n, q = l / n;
+            const int sim = q < parts ? m.sim[l - q * n] : -1;
+            padCooldowns(d, max(sim, 0), kPads * q / parts, sim >= 0 ? kPads * (q + 1) / parts : 0, parts, padTick);
+            padTick = 0;
         }
-        __syncthreads();
+        waveSync();
         mark(kStagePads);
     }
-    if constexpr (Profile) {
-        if (t == 0) {
-            for (int st = 0; st < kWindowStages; st++) atomicAdd(&prof[kProfStages + st], acc[st]);
-            atomicMin(&prof[kProfFirst], first);
-            atomicMax(&prof[kProfEnd], last);
+    if (map.outCount && lane < map.rounds && m.unit[lane] >= 0) {
+        const int u = m.unit[lane], l = group * kDealLists + dealClass(m.cost[lane]) * kDealSubs + u % kDealSubs;
+        map.outList[(size_t)l * map.listLen + atomicAdd(&map.outCount[l], 1)] = u;
+    }
+    if (prof && lane == 0) {
+        for (int st = 0; st < kWindowStages; st++) atomicAdd(&prof[kProfStages + st], m.stage[st]);
+        atomicMin(&prof[kProfFirst], m.first);
+        atomicMax(&prof[kProfEnd], m.last);
+        __threadfence();
+        if (atomicAdd(&prof[kProfDone], 1ull) == (unsigned long long)blocks * kWindowWaves - 1) {
+            // every other wave has published its start and end
             __threadfence();
-            if (atomicAdd(&prof[kProfDone], 1ull) == gridDim.x - 1) {
-                // every other workgroup has published its start and end
-                __threadfence();
-                const unsigned long long first0 = atomicMin(&prof[kProfFirst], ~0ull);
-                const unsigned long long end1 = atomicMax(&prof[kProfEnd], 0ull);
-                for (int st = 0; st < kWindowStages; st++) atomicAdd(&prof[kProfLast + st], acc[st]);
-                atomicAdd(&prof[kProfLastDelay], first - first0);
-                atomicAdd(&prof[kProfSpan], end1 - first0);
-                atomicExch(&prof[kProfFirst], ~0ull);
-                atomicExch(&prof[kProfEnd], 0ull);
-                atomicExch(&prof[kProfDone], 0ull);
-            }
+            const unsigned long long first0 = atomicMin(&prof[kProfFirst], ~0ull);
+            const unsigned long long end1 = atomicMax(&prof[kProfEnd], 0ull);
+            for (int st = 0; st < kWindowStages; st++) atomicAdd(&prof[kProfLast + st], m.stage[st]);
+            atomicAdd(&prof[kProfLastDelay], m.first - first0);
+            atomicAdd(&prof[kProfSpan], end1 - first0);
+            atomicExch(&prof[kProfFirst], ~0ull);
+            atomicExch(&prof[kProfEnd], 0ull);
+            atomicExch(&prof[kProfDone], 0ull);
         }
     }
 }
 
 // two waves per SIMD (the second bound is waves per execution unit): 256
-// VGPRs.  Cars > 0: instantiated for that many cars per simulation (1v1, the
-// common case, measured 6% faster than the same kernel with the count
-// read at run time; 2v2 and 3v3 5% and 3%); 0: any count.  Balanced: the
-// 1v1 instance that takes its simulations from the deal (WindowMap).
-template <int Cars, bool Balanced>
-__global__ __launch_bounds__(kWindowBlock, 2) void tickWindowKernel(Dev d, uint32_t* __restrict__ ws, int screen,
-                                                                 int kind, const void* __restrict__ actions,
-                                                                 int tick0, int ticks, int simsPerBlock,
-                                                                 SimRange range, WindowMap map)
+// VGPRs.  Cars > 0: instantiated for that many cars per simulation; 0: any count.
+template <int Cars>
+__global__ __launch_bounds__(kWindowBlock, 2) void tickWindowKernel(Dev d, int screen, int kind,
+                                                                 const void* __restrict__ actions, int tick0,
+                                                                 int ticks, SimRange range, WindowMap map,
+                                                                 unsigned long long* __restrict__ prof)
 {
-    tickWindowBody<false, false, Cars, Balanced>(d, ws, screen, kind, actions, tick0, ticks, simsPerBlock, range,
-                                                 map, nullptr);
+    __shared__ WindowLds L;
+    __shared__ WaveShare share[kWindowWaves];
+    static_assert(4 * (sizeof(WindowLds) + sizeof(share)) <= 160 * 1024, "four window workgroups per CU");
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+    tickWindowBody<Cars>(d, screen, kind, actions, tick0, ticks, range, map, prof, L.wave[wave], share[wave], wave,
+                         lane);
 }
 
-using WindowKernel = void (*)(Dev, uint32_t*, int, int, const void*, int, int, int, SimRange, WindowMap);
+using WindowKernel = void (*)(Dev, int, int, const void*, int, int, SimRange, WindowMap, unsigned long long*);
 
-// the instance for a car count: 1v1, 2v2 and 3v3 have their own
-WindowKernel windowKernelFor(int nCars, bool balanced)
+// the instance for a car count: one for each team size against itself and for a single car
+WindowKernel windowKernelFor(int nCars)
 {
     switch (nCars) {
-    case 2: return balanced ? tickWindowKernel<2, true> : tickWindowKernel<2, false>;
-    case 4: return balanced ? tickWindowKernel<4, true> : tickWindowKernel<4, false>;
-    case 6: return tickWindowKernel<6, false>;
-    default: return tickWindowKernel<0, false>;
+    case 1: return tickWindowKernel<1>;
+    case 2: return tickWindowKernel<2>;
+    case 4: return tickWindowKernel<4>;
+    case 6: return tickWindowKernel<6>;
+    case 8: return tickWindowKernel<8>;
+    default: return tickWindowKernel<0>;
     }
 }
 
-// the same with the native arena meshes
-__global__ __launch_bounds__(kWindowBlock, 2) void tickWindowNativeKernel(Dev d, uint32_t* __restrict__ ws,
-                                                                       int screen, int kind,
-                                                                       const void* __restrict__ actions, int tick0,
-                                                                       int ticks, int simsPerBlock, SimRange range,
-                                                                       WindowMap map)
+// The same ticks with every phase shared by the workgroup's two waves and a
+// barrier after each, for what the waves cannot hold apart: the native arena
+// meshes, and set workgroup sizes whose half is not whole simulations of 64
+// cars (21 3v3 simulations).  A block owns simulations
+// [begin + blockIdx.x * simsPerBlock, +simsPerBlock), its cars split evenly
+// between the waves, whole pairs of cars to each (a 1v1 simulation's two cars
+// sit in lanes 2i, 2i + 1).  With prof, thread 0 of each workgroup reads the
+// wall clock at every barrier.
+template <bool Native>
+__global__ __launch_bounds__(kWindowBlock, 2) void tickWindowBlockKernel(Dev d, int screen, int kind,
+                                                                      const void* __restrict__ actions, int tick0,
+                                                                      int ticks, int simsPerBlock, SimRange range,
+                                                                      unsigned long long* __restrict__ prof)
 {
-    tickWindowBody<false, true, 0, false>(d, ws, screen, kind, actions, tick0, ticks, simsPerBlock, range, map,
-                                          nullptr);
-}
-
-// the same kernel with the stage profile
-template <int Cars, bool Balanced>
-__global__ __launch_bounds__(kWindowBlock, 2) void tickWindowProfileKernel(Dev d, uint32_t* __restrict__ ws,
-                                                                        int screen, int kind,
-                                                                        const void* __restrict__ actions, int tick0,
-                                                                        int ticks, int simsPerBlock, SimRange range,
-                                                                        WindowMap map,
-                                                                        unsigned long long* __restrict__ prof)
-{
-    tickWindowBody<true, false, Cars, Balanced>(d, ws, screen, kind, actions, tick0, ticks, simsPerBlock, range,
-                                                map, prof);
-}
-
-using ProfileKernel = void (*)(Dev, uint32_t*, int, int, const void*, int, int, int, SimRange, WindowMap,
-                               unsigned long long*);
-
-// the profiled twin of windowKernelFor's instance for a car count
-ProfileKernel profileKernelFor(int nCars, bool balanced)
-{
-    switch (nCars) {
-    case 2: return balanced ? tickWindowProfileKernel<2, true> : tickWindowProfileKernel<2, false>;
-    case 4: return balanced ? tickWindowProfileKernel<4, true> : tickWindowProfileKernel<4, false>;
-    case 6: return tickWindowProfileKernel<6, false>;
-    default: return tickWindowProfileKernel<0, false>;
+    __shared__ WindowLds L;
+    __shared__ unsigned long long stage[kWindowStages], first, last;
+    const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
+    const int sim0 = range.begin + blockIdx.x * simsPerBlock;
+    const int simEnd = min(sim0 + simsPerBlock, range.end);
+    const int car0 = sim0 * d.nCars, carEnd = simEnd * d.nCars;
+    const int waveCars = (carEnd - car0 + 2 * kWindowWaves - 1) / (2 * kWindowWaves) * 2;
+    const int waveCar0 = car0 + wave * waveCars, waveCarEnd = min(waveCar0 + waveCars, carEnd);
+    auto mark = [&](int st) {
+        if (prof && t == 0) {
+            const unsigned long long now = wall_clock64();
+            stage[st] += now - last;
+            last = now;
+        }
+    };
+    if (prof && t == 0) {
+        for (int st = 0; st < kWindowStages; st++) stage[st] = 0;
+        first = last = wall_clock64();
+    }
+    for (int k = 0; k < ticks; k++) {
+        const int tick = tick0 + k;
+        const int car = waveCar0 + lane;
+        contactGroup<kWindowContactLead, kWindowContactOwners>(d, LdsHandoff{ L.wave[wave].hand }, screen, car,
+                                                               car < waveCarEnd, L.wave[wave].contact, lane);
+        __syncthreads();
+        mark(kStageContact);
+        if (car < waveCarEnd)
+            carArenaCar(d, LdsHandoff{ L.wave[wave].hand }, kind, actions, tick, car, lane, k == 0, k == ticks - 1);
+        __syncthreads();
+        mark(kStageCarArena);
+        // the block's simulations split evenly between the waves: at most
+        // kBallOwners per wave and group
+        const int per = (simEnd - sim0 + kWindowWaves - 1) / kWindowWaves;
+        const int wEnd = min(sim0 + (wave + 1) * per, simEnd);
+        for (int g = sim0 + wave * per; g < wEnd; g += kBallOwners)
+            ballGroup<Native>(d, tick, g + lane, lane < kBallOwners && g + lane < wEnd, L.wave[wave].ball, lane);
+        __syncthreads();
+        mark(kStageBall);
+        if (car < waveCarEnd) finishCar(d, car);
+        if (sim0 + t < simEnd) finishBall(d, sim0 + t);
+        __syncthreads();
+        mark(kStageFinish);
+        // a simulation's cars in one wave: the pickups compare them lane by lane
+        const int waveSims = 64 / d.nCars;
+        for (int g = sim0 + wave * waveSims; g < simEnd; g += kWindowWaves * waveSims) {
+            const int c = g * d.nCars + lane;
+            FinishedCar f{ kZero, false };
+            if (lane < waveSims * d.nCars && c < carEnd)
+                f = FinishedCar{ d.cv(CARL_CAR_POS, c), d.ci(CARL_CAR_DEMOED, c) == 0 };
+            padPickups(d, c, f, 0);
+        }
+        __syncthreads();
+        int u = t;
+        asm volatile("" : "+v"(u));   // as in tickWindowBody
+        const int parts = kWindowBlock / simsPerBlock, q = u / simsPerBlock, j = u - q * simsPerBlock;
+        if (q < parts && j < simEnd - sim0)
+            padCooldowns(d, sim0 + j, kPads * q / parts, kPads * (q + 1) / parts, parts, 1);
+        __syncthreads();
+        mark(kStagePads);
+    }
+    if (prof && t == 0) {
+        for (int st = 0; st < kWindowStages; st++) atomicAdd(&prof[kProfStages + st], stage[st]);
+        atomicMin(&prof[kProfFirst], first);
+        atomicMax(&prof[kProfEnd], last);
+        __threadfence();
+        if (atomicAdd(&prof[kProfDone], 1ull) == gridDim.x - 1) {
+            // every other workgroup has published its start and end
+            __threadfence();
+            const unsigned long long first0 = atomicMin(&prof[kProfFirst], ~0ull);
+            const unsigned long long end1 = atomicMax(&prof[kProfEnd], 0ull);
+            for (int st = 0; st < kWindowStages; st++) atomicAdd(&prof[kProfLast + st], stage[st]);
+            atomicAdd(&prof[kProfLastDelay], first - first0);
+            atomicAdd(&prof[kProfSpan], end1 - first0);
+            atomicExch(&prof[kProfFirst], ~0ull);
+            atomicExch(&prof[kProfEnd], 0ull);
+            atomicExch(&prof[kProfDone], 0ull);
+        }
     }
 }
+
+// The counts of every deal set and group (one workgroup each).
+__global__ void clearDealKernel(int* counts) { counts[blockIdx.x * blockDim.x + threadIdx.x] = 0; }
 
 __global__ void resetKernel(Dev d, int nOrange)
 {
@@ -1661,12 +1743,15 @@ struct carl_env {
     float* cactions = nullptr;
     uint32_t* ws = nullptr;  // per-tick car workspace (kWsPlanes planes)
     int* rowList = nullptr;  // a masked reset's selected rows (n_sim), then their count
-    // 1v1: the deal of balanced window launches, kDealSets sets of class
-    // counts and lists, and the balanced launches so far
+    // the deal of window launches, kDealSets sets of class counts and lists
+    // (dealRoom words each), the dealt launches so far and the units and
+    // groups they dealt in (a launch that deals in others starts over)
     int* dealCount = nullptr;
     int* dealList = nullptr;
+    size_t dealRoom = 0;      // words of one set of lists
+    int dealUnitSims = 0, dealGroups = 0;
     long long dealLaunches = 0;
-    int balance = 1;                     // deal 1v1 window launches by cost
+    int balance = 1;                     // deal window launches by cost
     float* ballScratch = nullptr;    // with it: kNativeMaxContacts slots of kNativeSlotWords per simulation
     int tickStreams = 1;                 // partitions of the tick, one stream each
     int contactScreen = 1;               // screen (car, triangle) pairs in the contact search
@@ -1696,8 +1781,7 @@ struct carl_env {
     double stageKernelMs[CARL_TICK_KERNELS] = {};
     int stageTicks = 0;
     int stagePath = 0;  // 1: window kernel, 2: phase kernels
-    int profResident = 0;  // window workgroups the device holds at once
-    int profSlots = 0;     // of those, the ones a profiled launch fills
+    int profSlots = 0;     // waves (or workgroups) a profiled launch keeps resident together
     bool profMixed = false;  // profiled launches of different shapes
     double clockMHz = 0.0;  // the wall clock read by wall_clock64
 
@@ -1816,62 +1900,92 @@ int launchTick(carl_env* e, bool timed, int kernel, void (*k)(P...), dim3 grid, 
         if (rc_ != CARL_OK) return rc_;   \
     } while (0)
 
+// How a window launch over n simulations spreads them over its waves.
+struct WindowShape {
+    bool block = false;    // the workgroup-wide kernel (simsPerBlock simulations each)
+    bool dealt = false;
+    int blocks = 0, simsPerBlock = 0;          // simsPerBlock: at most, of a workgroup's two waves
+    int unitSims = 0, nUnits = 0, rounds = 0, listLen = 0, groups = 1;  // WindowMap
+};
+
+// The deal's unit for waves of up to waveSims simulations: in a large run one
+// 128-byte line of each car field where whole simulations fill it (1v1 units
+// of half a line left the other half to a wave on another XCD, whose L2
+// fetched the line again: 2.0 against 1.1 GB of HBM reads per launch), else a
+// quarter of a wave's share, which leaves the deal something to choose from.
+int dealUnitFor(int waveSims, int nCars)
+{
+    if (kUnitCars % nCars == 0 && waveSims * nCars > kUnitCars) return kUnitCars / nCars;
+    int u = std::max(1, waveSims / 4);
+    while (u > 1 && (waveSims + u - 1) / u * u * nCars > 64) u--;
+    return u;
+}
+
+// Launches of fewer ticks have less tail to even out than the scattered units
+// cost them (2v2 stepped one tick at a time at 131,072 simulations ran 370 ->
+// 377 us per launch dealt).
+constexpr int kDealMinTicks = 4;
+
+// The launch of `ticks` ticks over n of the environment's simulations (one of
+// `parts` partitions).  Until the caller sets windowSims, each wave takes the
+// fewest simulations with which the partitions' workgroups together still fit
+// the device: a launch lasts as long as its slowest wave's chain of phases,
+// and that chain grows with the cars per wave (the candidate lists it walks,
+// the branches its lanes take between them).  A set windowSims gives each of
+// a workgroup's waves half of it.
+//
+// Dealt are launches whose waves are all resident at once, where the slowest
+// one sets the end; with more workgroups than that, and with a set
+// windowSims, 1v1 and 2v2 launches of whole workgroups of 128 cars.
+WindowShape windowShape(const carl_env* e, int n, int parts, int ticks)
+{
+    WindowShape w;
+    const int nC = e->nCars, most = 64 / nC;   // whole simulations of a wave
+    const int line = kUnitCars % nC == 0 && nC > 1 ? kUnitCars / nC : 0;
+    const int resident = std::max(1, e->windowResident / parts) * kWindowWaves;
+    int waveSims;
+    bool dealable = e->balance && !e->native() && parts == 1 && ticks >= kDealMinTicks && e->dealList;
+    if (e->windowAuto && !e->native()) {
+        waveSims = std::min(most, std::max(1, e->grid(n, resident)));
+        if (waveSims * (long long)resident < n) dealable = dealable && (nC == 2 || nC == 4) && n % (4 * line) == 0;
+    } else {
+        w.simsPerBlock = std::min(e->windowSims, kWindowBlock / nC);
+        waveSims = e->grid(w.simsPerBlock, kWindowWaves);
+        dealable = dealable && (nC == 2 || nC == 4) && w.simsPerBlock == 4 * line && n % (4 * line) == 0;
+        if (e->native() || waveSims > most) {
+            w.block = true;
+            w.blocks = e->grid(n, w.simsPerBlock);
+            return w;
+        }
+    }
+    w.simsPerBlock = kWindowWaves * waveSims;
+    w.blocks = e->grid(n, w.simsPerBlock);
+    w.groups = kWindowWaves * w.blocks <= resident && w.blocks >= kXcds ? kXcds : 1;
+    auto take = [&](int unitSims) {
+        w.unitSims = unitSims;
+        w.nUnits = e->grid(n, unitSims);
+        w.rounds = w.listLen = 0;
+        for (int g = 0; g < w.groups; g++) {
+            const int waves = (groupBlocksBefore(w.blocks, w.groups, g + 1) - groupBlocksBefore(w.blocks, w.groups, g)) * kWindowWaves;
+            const int units = groupFirstUnit(w.nUnits, w.blocks, w.groups, g + 1) - groupFirstUnit(w.nUnits, w.blocks, w.groups, g);
+            w.rounds = std::max(w.rounds, e->grid(units, waves));
+            w.listLen = std::max(w.listLen, e->grid(units, kDealSubs));
+        }
+        return w.rounds <= kMaxWaveUnits && w.rounds * unitSims <= most;
+    };
+    w.dealt = dealable && take(dealUnitFor(waveSims, nC)) && (size_t)w.groups * kDealLists * w.listLen <= e->dealRoom;
+    // one unit to a wave when not dealt: the groups part the waves' shares
+    // evenly, so that takes no wave beyond its share
+    if (!w.dealt) take(waveSims);
+    return w;
+}
+
 // Ticks run as e->tickStreams partitions of the simulations, partition 0 on
 // the environment stream and the others on auxiliary streams forked from and
 // joined back into it; the partitions share no data within a tick.  With
 // windowSims > 0 each partition runs all n ticks in one tick-window launch,
 // otherwise four phase kernels per tick.  Timing events bracket partition
 // 0's launches.
-// Simulations per window workgroup for the next launch: the set size capped
-// at a workgroup's cars; until the caller sets it, the fewest with which
-// every partition's workgroups together still fit the device's resident
-// window workgroups.  A launch lasts as long as its slowest workgroup's chain
-// of phases, and that chain grows with the cars per wave (the candidate lists
-// its wave walks, the branches its lanes take between them).  Window launch
-// of 1v1 at 1,000 simulations 405 -> 325 us (1 per workgroup, was 8), 50,001
-// 706 -> 673 us (49, was 64), 2v2 at 10,007 616 -> 596 us (10, was 16), 3v3
-// clustered at 16,384 876 -> 817 us (16, was 21).
-constexpr int kDealMinTicks = 4;   // balancedLaunch
-bool dealable(const carl_env* e)
-{
-    const int bs = dealBlockSims(e->nCars);
-    return e->balance && bs > 0 && !e->native() && e->dealList && std::min(e->tickStreams, e->nSim) == 1
-           && e->nSim % bs == 0;
-}
-int effectiveWindowSims(const carl_env* e)
-{
-    if (e->windowSims <= 0) return 0;
-    int wsb = std::min(e->windowSims, kWindowBlock / e->nCars);
-    if (!e->windowAuto) return wsb;
-    const int parts = std::min(e->tickStreams, e->nSim);
-    auto blocks = [&](int sims) {
-        int total = 0;
-        for (int p = 0; p < parts; p++) {
-            const int begin = (int)((int64_t)e->nSim * p / parts), end = (int)((int64_t)e->nSim * (p + 1) / parts);
-            total += e->grid(end - begin, sims);
-        }
-        return total;
-    };
-    // full workgroups that the deal evens out are kept while half as many
-    // simulations each would not fit
-    if (dealable(e) && wsb == dealBlockSims(e->nCars) && e->frameskip >= kDealMinTicks
-        && blocks(wsb / 2) > e->windowResident)
-        return wsb;
-    while (wsb > 1 && blocks(wsb - 1) <= e->windowResident) wsb--;
-    return wsb;
-}
-
-// Whether a window launch of `ticks` ticks deals its simulations by cost:
-// 1v1 or 2v2 on the mesh arena, one partition, workgroups of dealBlockSims
-// simulations, all of them full, and at least kDealMinTicks ticks.  (A
-// launch of fewer ticks has less tail to even out than the scattered units
-// cost it: 2v2 stepped one tick at a time at 131,072 simulations ran 370 ->
-// 377 us per launch dealt.)
-bool balancedLaunch(const carl_env* e, int ticks)
-{
-    return dealable(e) && effectiveWindowSims(e) == dealBlockSims(e->nCars) && ticks >= kDealMinTicks;
-}
-
 int launchTicks(carl_env* e, int kind, const void* actions, int n)
 {
     if (n <= 0) return CARL_OK;
@@ -1889,41 +2003,53 @@ int launchTicks(carl_env* e, int kind, const void* actions, int n)
         for (int p = 1; p < parts; p++) HIP_TRY(hipStreamWaitEvent(stream[p], e->fork, 0));
     }
     if (e->windowSims > 0) {
-        const int wsb = effectiveWindowSims(e);
-        const bool balanced = balancedLaunch(e, n);
-        WindowMap map{};
-        if (balanced) {
-            // the first balanced launch deals the identity
-            const int nU = e->nSim / dealUnitSims(e->nCars);
-            const long long l = e->dealLaunches++;
-            auto set = [&](long long k, int* base, size_t per) { return base + (size_t)(k % kDealSets) * per; };
-            map.inCount = l > 0 ? set(l, e->dealCount, kDealLists) : nullptr;
-            map.inList = l > 0 ? set(l, e->dealList, (size_t)kDealClasses * nU) : nullptr;
-            map.outCount = set(l + 1, e->dealCount, kDealLists);
-            map.outList = set(l + 1, e->dealList, (size_t)kDealClasses * nU);
-            map.clearCount = set(l + 2, e->dealCount, kDealLists);
-            map.nUnits = nU;
-        }
         for (int p = 0; p < parts; p++) {
             const SimRange r = range[p];
             const bool timed = p == 0;
-            const int blocks = e->grid(r.end - r.begin, wsb);
+            const WindowShape w = windowShape(e, r.end - r.begin, parts, n);
+            unsigned long long* prof = nullptr;
             if (timed && (e->timing & CARL_TIME_STAGES)) {
-                // the clock sums are divided by one resident-workgroup count
-                const int slots = std::min(blocks, e->profResident);
+                // the clock sums, of waves or (block kernel) workgroups, are
+                // divided by one resident count
+                prof = e->prof;
+                const int slots = std::min(w.blocks, e->windowResident) * (w.block ? 1 : kWindowWaves);
                 if (e->profSlots != 0 && e->profSlots != slots) e->profMixed = true;
                 e->profSlots = slots;
-                CARL_MARK(launchTick(e, timed, CARL_KERNEL_WINDOW, profileKernelFor(e->nCars, balanced),
-                                     dim3(blocks),
-                                     dim3(kWindowBlock), 0, stream[p], d, e->ws, e->contactScreen, kind, actions,
-                                     e->tickCount + 1, n, wsb, r, map, e->prof));
-            } else {
-                CARL_MARK(launchTick(e, timed, CARL_KERNEL_WINDOW,
-                                     e->native() ? tickWindowNativeKernel : windowKernelFor(e->nCars, balanced),
-                                     dim3(blocks),
-                                     dim3(kWindowBlock), 0, stream[p], d, e->ws, e->contactScreen, kind, actions,
-                                     e->tickCount + 1, n, wsb, r, map));
             }
+            if (w.block) {
+                CARL_MARK(launchTick(e, timed, CARL_KERNEL_WINDOW,
+                                     e->native() ? tickWindowBlockKernel<true> : tickWindowBlockKernel<false>,
+                                     dim3(w.blocks), dim3(kWindowBlock), 0, stream[p], d, e->contactScreen, kind, actions,
+                                     e->tickCount + 1, n, w.simsPerBlock, r, prof));
+                continue;
+            }
+            WindowMap map{};
+            map.unitSims = w.unitSims;
+            map.nUnits = w.nUnits;
+            map.rounds = w.rounds;
+            map.listLen = w.listLen;
+            map.groups = w.groups;
+            if (w.dealt) {
+                if (e->dealUnitSims != w.unitSims || e->dealGroups != w.groups) {
+                    // lists of other units (or none): the first launch of
+                    // these deals the identity and files into cleared counts
+                    clearDealKernel<<<kDealSets * kXcds, kDealLists, 0, stream[p]>>>(e->dealCount);
+                    e->dealUnitSims = w.unitSims;
+                    e->dealGroups = w.groups;
+                    e->dealLaunches = 0;
+                }
+                const long long l = e->dealLaunches++;
+                const size_t per = (size_t)map.groups * kDealLists * map.listLen;
+                auto set = [&](long long k, int* base, size_t len) { return base + (size_t)(k % kDealSets) * len; };
+                map.inCount = l > 0 ? set(l, e->dealCount, kXcds * kDealLists) : nullptr;
+                map.inList = l > 0 ? set(l, e->dealList, per) : nullptr;
+                map.outCount = set(l + 1, e->dealCount, kXcds * kDealLists);
+                map.outList = set(l + 1, e->dealList, per);
+                map.clearCount = set(l + 2, e->dealCount, kXcds * kDealLists);
+            }
+            CARL_MARK(launchTick(e, timed, CARL_KERNEL_WINDOW, windowKernelFor(e->nCars), dim3(w.blocks),
+                                 dim3(kWindowBlock), 0, stream[p], d, e->contactScreen, kind, actions, e->tickCount + 1, n,
+                                 r, map, prof));
         }
     }
     for (int k = 0; e->windowSims == 0 && k < n; k++) {
@@ -1957,6 +2083,13 @@ int launchTicks(carl_env* e, int kind, const void* actions, int n)
     }
     e->tickCount += n;
     return CARL_OK;
+}
+
+// the first partition's next step launch
+WindowShape launchShape(const carl_env* e)
+{
+    const int parts = std::min(e->tickStreams, e->nSim);
+    return windowShape(e, e->nSim / parts, parts, e->frameskip);
 }
 
 int packObs(carl_env* e, float* out, const bool* mask)
@@ -2144,7 +2277,7 @@ int carl_env_create(int nSim, int nBlue, int nOrange, int seed, int frameskip, i
         if (hipGetDevice(&device) != hipSuccess
             || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess
             || hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                   &perCu, windowKernelFor(e->nCars, false), kWindowBlock, 0) != hipSuccess)
+                   &perCu, windowKernelFor(e->nCars), kWindowBlock, 0) != hipSuccess)
             return bail(fail(CARL_ERR_RUNTIME, "window kernel occupancy query failed"));
         e->windowResident = perCu * cus;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCu, stepEnvKernel, kPackBlock,
@@ -2172,9 +2305,24 @@ int carl_env_create(int nSim, int nBlue, int nOrange, int seed, int frameskip, i
     rc = rc ? rc : devAlloc(&e->cactions, nT * 7);
     rc = rc ? rc : devAlloc(&e->ws, (size_t)kWsPlanes * tiledItems(e->nTotal));
     rc = rc ? rc : devAlloc(&e->rowList, nS + 1);
-    if (dealBlockSims(e->nCars) > 0 && nS % dealBlockSims(e->nCars) == 0) {
-        rc = rc ? rc : devAlloc(&e->dealCount, (size_t)kDealSets * kDealLists);
-        rc = rc ? rc : devAlloc(&e->dealList, (size_t)kDealSets * kDealClasses * (nS / dealUnitSims(e->nCars)));
+    if (!e->native()) {
+        // the lists of the launches this environment may deal (windowShape):
+        // with every wave resident, and of whole lines of cars in full 1v1 and
+        // 2v2 workgroups
+        const int nC = e->nCars, most = 64 / nC, line = nC == 2 || nC == 4 ? kUnitCars / nC : 0;
+        const long long waves = (long long)std::max(1, e->windowResident) * kWindowWaves;
+        int units = 0;
+        if (nSim <= most * waves)
+            units = e->grid(nSim, dealUnitFor(std::max(1, (int)((nSim + waves - 1) / waves)), nC));
+        if (line && nSim % (4 * line) == 0) units = std::max(units, nSim / line);
+        if (units > 0) {
+            // a group holds an eighth of the units, and up to a workgroup's
+            // share more where the workgroups do not divide by 8
+            const int group = e->grid(units, kXcds) + kWindowWaves * kMaxWaveUnits;
+            e->dealRoom = (size_t)kXcds * kDealLists * e->grid(group, kDealSubs);
+            rc = rc ? rc : devAlloc(&e->dealCount, (size_t)kDealSets * kXcds * kDealLists);
+            rc = rc ? rc : devAlloc(&e->dealList, kDealSets * e->dealRoom);
+        }
     }
     if (e->native()) rc = rc ? rc : devAlloc(&e->ballScratch, (size_t)kNativeMaxContacts * kNativeSlotWords * nS);
     if (rc) return bail(rc);
@@ -2423,10 +2571,12 @@ int carl_env_get_param(carl_env* e, int p, int* v)
     case CARL_PARAM_TICK_STREAMS: *v = e->tickStreams; break;
     case CARL_PARAM_CONTACT_SCREEN: *v = e->contactScreen; break;
     case CARL_PARAM_TICK_WINDOW: *v = e->windowSims; break;
-    case CARL_PARAM_TICK_WINDOW_LAUNCH: *v = effectiveWindowSims(e); break;
+    case CARL_PARAM_TICK_WINDOW_LAUNCH:
+        *v = e->windowSims > 0 ? launchShape(e).simsPerBlock : 0;
+        break;
     case CARL_PARAM_NATIVE_ARENA: *v = e->native(); break;
     case CARL_PARAM_TICK_BALANCE: *v = e->balance; break;
-    case CARL_PARAM_TICK_BALANCED_LAUNCH: *v = balancedLaunch(e, e->frameskip); break;
+    case CARL_PARAM_TICK_BALANCED_LAUNCH: *v = e->windowSims > 0 && launchShape(e).dealt; break;
     default: return fail(CARL_ERR_VALUE, "unknown parameter");
     }
     return CARL_OK;
@@ -2449,14 +2599,10 @@ int carl_env_enable_timing(carl_env* e, int enable)
     if (e->timing & CARL_TIME_STAGES) {
         if (!e->prof) CARL_TRY(devAlloc(&e->prof, kProfWords));
         CARL_TRY(clearProfile(e));
-        int device = 0, cus = 0, perCu = 0, khz = 0;
+        int device = 0, khz = 0;
         HIP_TRY(hipGetDevice(&device));
-        HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
         HIP_TRY(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device));
-        HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCu, profileKernelFor(e->nCars, false), kWindowBlock,
-                                                             0));
-        if (khz <= 0 || perCu <= 0) return fail(CARL_ERR_RUNTIME, "no wall-clock rate or window occupancy");
-        e->profResident = perCu * cus;
+        if (khz <= 0) return fail(CARL_ERR_RUNTIME, "no wall-clock rate");
         e->clockMHz = khz / 1000.0;
     }
     return CARL_OK;
@@ -2503,7 +2649,7 @@ int carl_env_stage_timing(carl_env* e, double* stageUs, double* lastUs, double* 
     if (n == 0) return CARL_OK;
     if (path == 1) {
         const double us = 1.0 / (e->clockMHz * n);  // clock ticks -> us per tick
-        // workgroup time of each phase over the workgroups resident at once
+        // the waves' (or workgroups') time in each phase over those resident at once
         for (int s = 0; s < CARL_STAGES; s++) {
             stageUs[s] = clocks[kProfStages + s] * us / slots;
             lastUs[s] = clocks[kProfLast + s] * us;

@@ -331,19 +331,20 @@ DI void storeBody(const Dev& d, int c, const Body& b)
     d.setq(CARL_CAR_ROT, c, b.rot);
 }
 
-// one car pair; ia is body A (later car), ib body B (CarCar/Solve.cuh:63-151)
-DI void carCarPair(const Dev& d, int ia, int ib, int tick)
+// one car pair; ia is body A (later car), ib body B (CarCar/Solve.cuh:63-151).
+// True when the pair was in contact (its cars' poses have been rewritten).
+DI bool carCarPair(const Dev& d, int ia, int ib, int tick)
 {
-    if (d.ci(CARL_CAR_DEMOED, ia) || d.ci(CARL_CAR_DEMOED, ib)) return;
+    if (d.ci(CARL_CAR_DEMOED, ia) || d.ci(CARL_CAR_DEMOED, ib)) return false;
     const Box A{ d.cv(CARL_CAR_CEN, ia), d.cq(CARL_CAR_ROT, ia) };
     const Box B{ d.cv(CARL_CAR_CEN, ib), d.cq(CARL_CAR_ROT, ib) };
     const float maxDist = 2.f * len(kHalf);
-    if (lensq(B.cen - A.cen) > maxDist * maxDist) return;
+    if (lensq(B.cen - A.cen) > maxDist * maxDist) return false;
     const Sat s = boxBoxSat(A, B);
-    if (!s.overlap) return;
+    if (!s.overlap) return false;
     PairContact cts[kMaxManifold];
     const int count = boxBoxContacts(s, A, B, cts);
-    if (count == 0) return;
+    if (count == 0) return false;
 
     // demolition check on the pre-solve state
     int demoBumper = -1, demoVictim = -1;
@@ -404,7 +405,7 @@ DI void carCarPair(const Dev& d, int ia, int ib, int tick)
         const uint32_t seed = (uint32_t)d.seed ^ (uint32_t)demoVictim * 0x9e3779b9u ^ (uint32_t)tick;
         d.seti(CARL_CAR_RESPAWN_IDX, demoVictim, pickIndex(seed, 4));
         d.seti(CARL_CAR_LAST_RESPAWN_DIR, demoVictim, 0);
-        return;
+        return true;
     }
 
     for (int side = 0; side < 2; side++) {
@@ -429,6 +430,7 @@ DI void carCarPair(const Dev& d, int ia, int ib, int tick)
         d.seti(CARL_CAR_CONTACT_IDX, bumper, victim);
         d.setf(CARL_CAR_CONTACT_COOLDOWN, bumper, kBumpCooldown);
     }
+    return true;
 }
 
 // ------------------------------------------------------------- ball vs arena
@@ -1360,8 +1362,14 @@ DI void respawnCar(const Dev& d, int c)
     resetInternal(d, c);
 }
 
+// What the boost pads need of a car once it has moved.
+struct FinishedCar {
+    V3 pos;
+    bool alive;   // not demolished
+};
+
 // integrate, then apply the impulse cache / demo timer (Solve.cuh:316-327, FinishTick.cuh:100-141)
-DI void finishCar(const Dev& d, int c)
+DI FinishedCar finishCar(const Dev& d, int c)
 {
     V3 pos = d.cv(CARL_CAR_POS, c), cen;
     Q4 rot = d.cq(CARL_CAR_ROT, c);
@@ -1383,8 +1391,9 @@ DI void finishCar(const Dev& d, int c)
         }
         timer = fmax_(timer - kDt, 0.f);
         d.setf(CARL_CAR_DEMO_TIMER, c, timer);
-        if (timer <= 0.f) respawnCar(d, c);
-        return;
+        if (timer > 0.f) return FinishedCar{ pos, false };
+        respawnCar(d, c);
+        return FinishedCar{ d.cv(CARL_CAR_POS, c), true };
     }
     integratePose(pos, cen, rot, vel, ang);
     clampCarVelocity(vel, ang);
@@ -1400,6 +1409,7 @@ DI void finishCar(const Dev& d, int c)
     d.setv(CARL_CAR_VEL, c, vel);
     d.setv(CARL_CAR_ANG, c, ang);
     if (cd > 0.f) d.setf(CARL_CAR_CONTACT_COOLDOWN, c, fmax_(cd - kDt, 0.f));
+    return FinishedCar{ pos, true };
 }
 
 DI void finishBall(const Dev& d, int s)
@@ -1421,18 +1431,13 @@ DI void finishBall(const Dev& d, int s)
 // boosts are written back once.  The pass is instantiated for two, four and
 // eight cars, so that 1v1 runs a quarter of the 8-car code (measured 3% per
 // step on the 1v1 window kernel).
-constexpr int kMaxCars = 8;
 
-// Boost pads [p0, p1) of simulation s: cooldowns, pickups and the boost
+// Boost pads of simulation s in one thread: cooldowns, pickups and the boost
 // they give.  No car position lies in two pads' cylinders (the closest pair
 // of cylinders is 773 uu apart), so a car takes boost from at most one pad per
-// tick: disjoint pad ranges of one simulation can run in different threads,
-// in any order, with the same result.  A thread reads every car's boost but
-// uses it only for a car inside one of its own pads, the only case in which
-// it writes that boost.  [P0, P1) bounds the range at compile time (a
-// caller whose range is fixed loads only those pads' cooldowns).
-template <int MaxCars, int P0 = 0, int P1 = kPads>
-DI void boostPadsRangeT(const Dev& d, int s, int p0, int p1)
+// tick.
+template <int MaxCars>
+DI void boostPadsT(const Dev& d, int s)
 {
     const int base = s * d.nCars;
     V3 cp[MaxCars];
@@ -1449,16 +1454,13 @@ DI void boostPadsRangeT(const Dev& d, int s, int p0, int p1)
             boost[k] = d.cf(CARL_CAR_BOOST, base + k);
         }
     }
-    // all cooldowns are read before any is written back, each load
-    // unconditional (one batch in flight; a load under a per-pad range test
-    // would wait for its own round trip), those outside the range unused
+    // all cooldowns are read before any is written back
     float cool[kPads];
 #pragma unroll
-    for (int p = P0; p < P1; p++) cool[p] = d.sf(CARL_SIM_PAD_COOLDOWN + p, s);
+    for (int p = 0; p < kPads; p++) cool[p] = d.sf(CARL_SIM_PAD_COOLDOWN + p, s);
     int changed = 0;
 #pragma unroll
-    for (int p = P0; p < P1; p++) {
-        if (p < p0 || p >= p1) continue;
+    for (int p = 0; p < kPads; p++) {
         const float prev = cool[p];
         float cd = prev;
         if (cd > 0.f) cd = fmax_(cd - kDt, 0.f);
@@ -1491,95 +1493,143 @@ DI void boostPadsRangeT(const Dev& d, int s, int p0, int p1)
         if (changed & (1 << k)) d.setf(CARL_CAR_BOOST, base + k, boost[k]);
 }
 
-// The same for a range of at most Span pads whose bounds vary from lane to
-// lane (the workgroup's pad parts do not line up with its waves): the pads
-// are visited as positions p0 + i, i < Span, so every lane runs the same
-// iterations, with the pads' positions read from the table by index; only
-// the range's cooldowns are loaded (all before the first is used).
-template <int MaxCars, int Span>
-DI void boostPadsSpanT(const Dev& d, int s, int p0, int p1)
+// The window kernel's pads, in two parts that together do the same: the
+// pickups at every tick, and the cooldowns once for up to kPadTicks ticks (a
+// pad taken in between cannot run out before), so that the 34 words of a
+// simulation are read and written once per launch instead of at every tick.
+// Until the cooldowns are counted down their words hold the values of the
+// first of those ticks; a pad taken at the tick after t of them holds a mark
+// with t, a NaN, which like any cooldown left is not <= 0.
+constexpr int kPadTicks = 64;
+constexpr uint32_t kPadTaken = 0x7fd00000u;   // | big pad << 8 | t
+static_assert(kPadTicks <= 256 && kPadTicks < 120 * 4, "no pad recovers within kPadTicks ticks of 1/120 s");
+
+// a cooldown n ticks on
+DI float countDown(float cool, int n)
 {
-    const int base = s * d.nCars;
-    V3 cp[MaxCars];
-    bool alive[MaxCars];
-    float boost[MaxCars];
+    for (int i = 0; i < n; i++)
+        if (cool > 0.f) cool = fmax_(cool - kDt, 0.f);
+    return cool;
+}
+
+// The cooldowns of pads [p0, p1) of simulation s, at most Span of them, n
+// ticks on: every lane visits positions p0 + i, i < Span, all loads issued
+// before the first use (each unconditional: under a range test it would wait
+// for its own round trip).
+template <int Span>
+DI void padCooldownsT(const Dev& d, int s, int p0, int p1, int n)
+{
+    uint32_t word[Span];
 #pragma unroll
-    for (int k = 0; k < MaxCars; k++) {
-        alive[k] = false;
-        cp[k] = kZero;
-        boost[k] = 0.f;
-        if (k < d.nCars) {
-            alive[k] = !d.ci(CARL_CAR_DEMOED, base + k);
-            cp[k] = d.cv(CARL_CAR_POS, base + k);
-            boost[k] = d.cf(CARL_CAR_BOOST, base + k);
-        }
-    }
-    float cool[Span];
-#pragma unroll
-    for (int i = 0; i < Span; i++) cool[i] = d.sf(CARL_SIM_PAD_COOLDOWN + min(p0 + i, kPads - 1), s);
-    int changed = 0;
+    for (int i = 0; i < Span; i++) word[i] = d.swLane(CARL_SIM_PAD_COOLDOWN + min(p0 + i, kPads - 1), s);
 #pragma unroll
     for (int i = 0; i < Span; i++) {
-        const int p = p0 + i;
-        if (p >= p1) break;
-        const float prev = cool[i];
-        float cd = prev;
-        if (cd > 0.f) cd = fmax_(cd - kDt, 0.f);
-        if (cd <= 0.f) {
-            const bool big = p < 6;
-            const float radius = big ? kBigPadRadius : kSmallPadRadius;
-            const float px = kPadPos[p][0], py = kPadPos[p][1], pz = kPadPos[p][2];
-            int locked = -1;
-            float have = 0.f;
-#pragma unroll
-            for (int k = 0; k < MaxCars; k++) {
-                if (k >= d.nCars || !alive[k]) continue;
-                const float dx = cp[k].x - px, dy = cp[k].y - py;
-                if (dx * dx + dy * dy < radius * radius && fabsf(cp[k].z - pz) < kPadHeight) {
-                    locked = k;
-                    have = boost[k];
-                }
-            }
-            if (locked >= 0 && have < kBoostMax) {
-                const float next = fmin_(have + (big ? kBigPadAmount : kSmallPadAmount), kBoostMax);
-                setAt(boost, locked, next);
-                changed |= 1 << locked;
-                cd = big ? kBigPadCooldown : kSmallPadCooldown;
-            }
-        }
-        if (__float_as_uint(cd) != __float_as_uint(prev)) d.ssetf(CARL_SIM_PAD_COOLDOWN + p, s, cd);
+        const uint32_t w = word[i];
+        const bool taken = (w & 0xfffffe00u) == kPadTaken;
+        if (p0 + i >= p1 || !(taken || __uint_as_float(w) > 0.f)) continue;
+        const float from = taken ? ((w & 0x100u) ? kBigPadCooldown : kSmallPadCooldown) : __uint_as_float(w);
+        d.swPutLane(CARL_SIM_PAD_COOLDOWN + p0 + i, s,
+                    __float_as_uint(countDown(from, taken ? n - 1 - (int)(w & 0xffu) : n)));
     }
-#pragma unroll
-    for (int k = 0; k < MaxCars; k++)
-        if (changed & (1 << k)) d.setf(CARL_CAR_BOOST, base + k, boost[k]);
 }
 
-// pads [p0, p1) of simulation s, the range at most ceil(kPads / parts) long
-DI void boostPadsSpan(const Dev& d, int s, int p0, int p1, int parts)
+// the range at most ceil(kPads / parts) long
+DI void padCooldowns(const Dev& d, int s, int p0, int p1, int parts, int n)
 {
     const int span = (kPads + parts - 1) / parts;
-    if (d.nCars <= 2) {
-        if (span <= 3) boostPadsSpanT<2, 3>(d, s, p0, p1);
-        else if (span <= 9) boostPadsSpanT<2, 9>(d, s, p0, p1);
-        else if (span <= kPads / 2) boostPadsSpanT<2, kPads / 2>(d, s, p0, p1);
-        else boostPadsSpanT<2, kPads>(d, s, p0, p1);
-    } else if (d.nCars <= 4) {
-        if (span <= 3) boostPadsSpanT<4, 3>(d, s, p0, p1);
-        else if (span <= 9) boostPadsSpanT<4, 9>(d, s, p0, p1);
-        else boostPadsSpanT<4, kPads>(d, s, p0, p1);
-    } else {
-        if (span <= 6) boostPadsSpanT<kMaxCars, 6>(d, s, p0, p1);
-        else boostPadsSpanT<kMaxCars, kPads>(d, s, p0, p1);
-    }
+    if (span <= 5) padCooldownsT<5>(d, s, p0, p1, n);
+    else if (span <= 9) padCooldownsT<9>(d, s, p0, p1, n);
+    else if (span <= kPads / 2) padCooldownsT<kPads / 2>(d, s, p0, p1, n);
+    else padCooldownsT<kPads>(d, s, p0, p1, n);
 }
 
-DI void boostPadsRange(const Dev& d, int s, int p0, int p1)
+// Pickups, one car per lane (car, with what its finish left in registers; a
+// simulation's cars in adjacent lanes of the wave), at the tick after t of
+// those since the cooldowns were counted down.  The pads lie
+// symmetric to both axes, so the car is tested in the first quadrant, against
+// 11 places with their coordinates as immediates, and no table is read: the
+// circle test of |x| and |y| is bit for bit that of x and y against the pad's
+// own signs.  The circles are disjoint, so at most one place passes.  Only a
+// wave with a car on a pad goes on.  The last overlapping car of a simulation
+// takes the pad, if it has room for boost.
+struct PadPlace {
+    float x, y;       // of the pads (+-x, +-y)
+    int first;        // the pad at (-x, -y)
+    int xStep, ySum;  // the pad at (x, -y) is first + xStep; at (sx x, y) it is ySum minus that at (-sx x, -y)
+};
+constexpr PadPlace kPadPlaces[11] = {
+    { 3584.f, 0.f, 0, 1, 1 },       { 3072.f, 4096.f, 4, 1, 7 },    { 0.f, 4240.f, 6, 0, 39 },
+    { 1792.f, 4184.f, 7, 1, 39 },   { 940.f, 3308.f, 9, 1, 39 },    { 0.f, 2816.f, 11, 0, 39 },
+    { 3584.f, 2484.f, 12, 1, 39 },  { 1788.f, 2300.f, 14, 1, 39 },  { 2048.f, 1036.f, 16, 2, 39 },
+    { 0.f, 1024.f, 17, 0, 39 },     { 1024.f, 0.f, 19, 1, 39 },
+};
+HDI constexpr bool padPlaceBig(int i) { return i < 2; }
+// the pad of place i on the side of the signs (negative x, negative y)
+HDI constexpr int padAtPlace(int first, int xStep, int ySum, bool nx, bool ny)
 {
-    if (d.nCars <= 2) boostPadsRangeT<2>(d, s, p0, p1);
-    else if (d.nCars <= 4) boostPadsRangeT<4>(d, s, p0, p1);
-    else boostPadsRangeT<kMaxCars>(d, s, p0, p1);
+    return ny ? first + (nx ? 0 : xStep) : ySum - (first + (nx ? xStep : 0));
+}
+constexpr bool padPlacesMatch()
+{
+    int seen = 0;
+    for (int i = 0; i < 11; i++) {
+        const PadPlace q = kPadPlaces[i];
+        for (int k = 0; k < 4; k++) {
+            const bool nx = (k & 1) != 0, ny = (k & 2) != 0;
+            if ((q.x == 0.f && nx) || (q.y == 0.f && ny)) continue;
+            const int p = padAtPlace(q.first, q.xStep, q.ySum, nx, ny);
+            if (p < 0 || p >= kPads || (p < 6) != padPlaceBig(i)) return false;
+            if (kPadPos[p][0] != (nx ? -q.x : q.x) || kPadPos[p][1] != (ny ? -q.y : q.y)) return false;
+            if (kPadPos[p][2] != (padPlaceBig(i) ? 73.f : 70.f)) return false;
+            seen++;
+        }
+    }
+    return seen == kPads;
+}
+static_assert(padPlacesMatch(), "the places are the pads");
+
+DI void padPickups(const Dev& d, int car, const FinishedCar& f, int t)
+{
+    const float ax = fabsf(f.pos.x), ay = fabsf(f.pos.y);
+    int place = -1;
+#pragma unroll
+    for (int i = 0; i < 11; i++) {
+        const float radius = padPlaceBig(i) ? kBigPadRadius : kSmallPadRadius;
+        const float dx = ax - kPadPlaces[i].x, dy = ay - kPadPlaces[i].y;
+        if (dx * dx + dy * dy < radius * radius) place = i;
+    }
+    const bool big = place >= 0 && place < 2;
+    const bool over = f.alive && place >= 0 && fabsf(f.pos.z - (big ? 73.f : 70.f)) < kPadHeight;
+    if (__ballot(over) == 0) return;
+    int first = 0, xStep = 0, ySum = 0;
+#pragma unroll
+    for (int i = 0; i < 11; i++)
+        if (place == i) {
+            first = kPadPlaces[i].first;
+            xStep = kPadPlaces[i].xStep;
+            ySum = kPadPlaces[i].ySum;
+        }
+    const int pad = padAtPlace(first, xStep, ySum, f.pos.x < 0.f, f.pos.y < 0.f);
+    // a later car of the simulation on the same pad takes precedence
+    const int local = car % d.nCars, sim = car / d.nCars, mine = over ? pad : -1;
+    bool last = over;
+    for (int k = 1; k < d.nCars; k++) {
+        const int other = __shfl_down(mine, k);
+        if (local + k < d.nCars && other == mine) last = false;
+    }
+    if (!last) return;
+    const float have = d.cf(CARL_CAR_BOOST, car);
+    const float cool = __uint_as_float(d.swLane(CARL_SIM_PAD_COOLDOWN + pad, sim));
+    if (!(have < kBoostMax) || !(countDown(cool, t + 1) <= 0.f)) return;
+    d.setf(CARL_CAR_BOOST, car, fmin_(have + (big ? kBigPadAmount : kSmallPadAmount), kBoostMax));
+    d.swPutLane(CARL_SIM_PAD_COOLDOWN + pad, sim, kPadTaken | (big ? 0x100u : 0u) | (uint32_t)t);
 }
 
-DI void boostPads(const Dev& d, int s) { boostPadsRange(d, s, 0, kPads); }
+DI void boostPads(const Dev& d, int s)
+{
+    if (d.nCars <= 2) boostPadsT<2>(d, s);
+    else if (d.nCars <= 4) boostPadsT<4>(d, s);
+    else boostPadsT<kMaxCars>(d, s);
+}
 
 }  // namespace carl

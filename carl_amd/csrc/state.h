@@ -138,6 +138,11 @@ struct Dev {
         return __builtin_amdgcn_raw_buffer_load_b32(simRsrc(), itemOff(s, CARL_SIM_FIELDS) + f * 256, 0, 0);
     }
 
+    DI void swPutLane(int f, int s, uint32_t v) const
+    {
+        __builtin_amdgcn_raw_buffer_store_b32(v, simRsrc(), itemOff(s, CARL_SIM_FIELDS) + f * 256, 0, 0);
+    }
+
     DI float sf(int f, int s) const { return __uint_as_float(sw(f, s)); }
     DI int si(int f, int s) const { return (int)sw(f, s); }
     DI V3 sv(int f, int s) const { return V3{ sf(f, s), sf(f + 1, s), sf(f + 2, s) }; }

@@ -123,9 +123,9 @@ enum {
                                       provably reject before running them; 0: it runs them on every pair.
                                       Results are identical; no reference counterpart (default 1) */
     CARL_PARAM_TICK_WINDOW = 13,   /* > 0: all ticks of a step in one launch per partition, this many
-                                      simulations per workgroup (at most 128 cars; default 64, until it is
-                                      set fewer for runs too small to fill the GPU); 0: four
-                                      phase kernels per tick.  Results are identical; no reference
+                                      simulations per workgroup of two waves (at most 128 cars; until it
+                                      is set, the fewest with which the workgroups still fit the
+                                      GPU together); 0: four phase kernels per tick.  Results are identical; no reference
                                       counterpart */
     CARL_PARAM_NATIVE_ARENA = 14,  /* read-only: 1 when the environment was created with native mesh
                                       metadata (the reference's ArenaMesh::hasNativeMetadata) */
@@ -133,18 +133,18 @@ enum {
                                           uses (CARL_PARAM_TICK_WINDOW capped at 128 cars, after the
                                           automatic sizing of small runs; 0: phase kernels); no
                                           reference counterpart */
-    CARL_PARAM_TICK_BALANCE = 16,  /* 1: 1v1 and 2v2 window launches of 64- and 32-simulation
-                                      workgroups deal the simulations to the workgroups in units of
-                                      32 cars (16 or 8 simulations), ordered by the contact work
-                                      each unit did in the balanced launch before, so that the
-                                      workgroups finish together; 0: workgroup b takes simulations
-                                      [S b, S b + S).  Results are identical; no reference
-                                      counterpart (default 1) */
+    CARL_PARAM_TICK_BALANCE = 16,  /* 1: window launches deal the simulations to the waves in units
+                                      of consecutive simulations, ordered by the contact work each
+                                      unit did in the dealt launch before, so that the waves finish
+                                      together; 0: every wave takes consecutive simulations.
+                                      Results are identical; no reference counterpart (default 1) */
     CARL_PARAM_TICK_BALANCED_LAUNCH = 17 /* read-only: 1 when the next step's window launch is
-                                            dealt (1v1 or 2v2, one partition, workgroups of 64 or
-                                            32 simulations, n_sim a multiple of that, mesh arena,
-                                            frameskip at least 4, CARL_PARAM_TICK_BALANCE on); no
-                                            reference counterpart */
+                                            dealt: one partition, mesh arena, frameskip at least 4,
+                                            CARL_PARAM_TICK_BALANCE on, and the launch's waves all
+                                            resident at once, or (larger runs, and with
+                                            CARL_PARAM_TICK_WINDOW set to it) full 1v1 or 2v2
+                                            workgroups of 64 or 32 simulations; no reference
+                                            counterpart */
 };
 
 /* ---- persistent state layout (export / import) ------------------------
@@ -402,22 +402,23 @@ enum {
     CARL_STAGES = 5
 };
 
-/* With CARL_TIME_STAGES enabled, the tick window launches of partition 0 run
- * a twin of the window kernel in which each workgroup reads the device's
- * constant-rate wall clock at its start and at every phase barrier (the plain
- * kernel is left as it is: it is the one measured otherwise).
+/* With CARL_TIME_STAGES enabled, each wave of the tick window launches of
+ * partition 0 reads the device's constant-rate wall clock at its start and
+ * after every phase.  (A launch whose waves share phases - with native mesh
+ * metadata excluded, only a set CARL_PARAM_TICK_WINDOW whose half is not whole
+ * simulations of at most 64 cars - counts its workgroups instead.)
  * carl_env_stage_timing synchronises and returns, for the ticks since the
  * profile was enabled or last read, in us per tick:
  *   stage_us[CARL_STAGES]  each stage's share of the device: the stage's time
- *       summed over all workgroups / the workgroups resident at once
- *       (min(grid, occupancy x CUs)).  Workgroups that finish early leave
+ *       summed over all waves / the waves resident at once (those of
+ *       min(grid, occupancy x CUs) workgroups).  Waves that finish early leave
  *       their slots idle until the launch ends, so these sum to less than
  *       the launch time by the launch's imbalance.
- *   last_us[CARL_STAGES + 1]  the critical path: the stages of the workgroup
- *       that finished each launch last, then its start after the launch's
- *       first workgroup start; they sum to span_us.
- *   span_us    the launch's first workgroup start to its last workgroup end
- *       (wall clock).
+ *   last_us[CARL_STAGES + 1]  the critical path: the stages of the wave that
+ *       finished each launch last, then its start after the launch's first
+ *       wave start; they sum to span_us.
+ *   span_us    the launch's first wave start to its last wave end (wall
+ *       clock).
  *   launch_us  the launch itself (HIP events).
  *   ticks      ticks covered;
  * then clears them.  With the phase kernels each stage is one kernel's
