@@ -697,8 +697,21 @@ DI void polyPut(Poly& p, V3 x)
     p.n++;
 }
 
-DI Poly clipPolygon(const Poly& in, V3 normal, float dist)
+// outside(v): the distance of v beyond the plane.  Each vertex's is taken once
+// (it serves as the end of one edge and the start of the next), and a polygon
+// with no vertex outside is returned as it is, which is what the general pass
+// makes of it.
+template <class Outside>
+DI Poly clipPolygon(const Poly& in, Outside outside)
 {
+    float beyond[kMaxPolygon];
+    bool cut = false;
+#pragma unroll
+    for (int i = 0; i < kMaxPolygon; i++) {
+        beyond[i] = outside(in.v[i]);
+        if (i < in.n && !(beyond[i] <= 0.f)) cut = true;
+    }
+    if (!cut) return in;
     Poly out;
 #pragma unroll
     for (int j = 0; j < kMaxPolygon; j++) out.v[j] = kZero;
@@ -708,9 +721,12 @@ DI Poly clipPolygon(const Poly& in, V3 normal, float dist)
         if (i >= in.n) break;
         const V3 cur = in.v[i];
         V3 nxt = in.v[0];
-        if (i + 1 < kMaxPolygon && i + 1 < in.n) nxt = in.v[i + 1 < kMaxPolygon ? i + 1 : 0];
-        const float cd = dot(normal, cur) - dist;
-        const float nd = dot(normal, nxt) - dist;
+        float nd = beyond[0];
+        if (i + 1 < kMaxPolygon && i + 1 < in.n) {
+            nxt = in.v[i + 1 < kMaxPolygon ? i + 1 : 0];
+            nd = beyond[i + 1 < kMaxPolygon ? i + 1 : 0];
+        }
+        const float cd = beyond[i];
         const bool ci = cd <= 0.f, ni = nd <= 0.f;
         if (ci && out.n < kMaxPolygon) polyPut(out, cur);
         if (ci != ni && out.n < kMaxPolygon) {
@@ -905,7 +921,8 @@ DI bool triBestContact(const LocalTri& t, const Sat& s, const V3* near, int nNea
         if (a == faceAxis) continue;
 #pragma unroll
         for (int sg = 1; sg >= -1; sg -= 2) {
-            if (poly.n > 0) poly = clipPolygon(poly, unitAxis(a) * (float)sg, comp(kHalf, a));
+            // dot(unitAxis(a) * sg, v) is the component itself
+            if (poly.n > 0) poly = clipPolygon(poly, [&](V3 v) { return comp(v, a) * (float)sg - comp(kHalf, a); });
         }
     }
     const V3 faceNormal = unitAxis(faceAxis) * -copysignf(1.f, comp(s.minAxis, faceAxis));
