@@ -19,6 +19,7 @@
 #pragma once
 
 #include "state.h"
+#include "wave.h"
 
 namespace carl {
 
@@ -1454,110 +1455,132 @@ DI float nonStickyFriction(float z)
     return 0.5f + ((z - 0.7075f) / (1.f - 0.7075f)) * 0.5f;
 }
 
-DI void applySuspension(Body& b, CarRegs& r, const Wheels& w, int tick)
+// What a wheel's force needs of its car.
+struct SuspCar {
+    Q4 rot;
+    V3 cenOffset, vel, ang;                  // box centre - position, velocities before the suspension
+    float steer, handbrake, throttle, drive, brakeTorque;
+    float pushDt;
+};
+
+// What a wheel in contact adds to its car.
+struct WheelForce {
+    V3 dv, directVel, directAng;
+    float lat, lon;                          // the friction factors kept for the next tick
+};
+
+// The suspension spring and the tyre forces of wheel k in contact
+// (CarSuspension.cuh): latUsed and lonUsed are the factors kept by the last tick.
+DI WheelForce wheelForce(const SuspCar& c, int k, float dist, V3 normal, float latUsed, float lonUsed)
 {
-    const float brakeTorque = r.brakePrev * (kCarMass * (14.25f + 1.f / 3.f));
-    const V3 up = rotateZ(b.rot);
-    const V3 cenOffset = b.cen - b.pos;
-    const V3 fwd = rotateX(b.rot);
-    const V3 right = rotateY(b.rot);
-    const V3 vel0 = b.vel, ang0 = b.ang;
-    const V3 angCrossUp = cross(b.ang, up);
-    const float pushDt = tick <= 1 ? kPushbackDtFirst : kDt;
-    V3 normalSum = kZero;
-    int count = 0;
-#pragma unroll
-    for (int k = 0; k < kWheels; k++) {
-        const float dist = w.dist[k];
-        if (dist > wheelRay(k)) continue;
-        const float radius = wheelRadius(k), rest = wheelRest(k);
-        const float suspLen = fmin_(fmax_(dist - radius, rest - kMaxTravel), rest + kMaxTravel);
-        const V3 normal = w.normal[k];
-        const V3 fullRel = (cenOffset + rotate(b.rot, wheelAnchor(k))) - up * dist;
-        const V3 pointVel = vel0 + cross(ang0, fullRel);
-        const float projVel = dot(normal, pointVel);
-        const float den = dot(normal, up);
-        const float clipped = den > 0.1f ? 1.f / den : 10.f;
-        const float damping = projVel * clipped < 0.f ? kDampCompression : kDampRelaxation;
-        float force = ((rest - suspLen) * kSuspStiffness - damping * projVel) * clipped * wheelScale(k);
-        if (force <= 0.f) force = 0.f;
-        float impulse = 0.f;
-        if (force != 0.f) {
-            impulse = force * kDt;
-            const float thr = rest + radius - kSuspSub;
-            if (dist < thr) {
-                const V3 ta = cross(fullRel, normal);
-                const float jac = kCarInvMass + dot(invInertiaWorld(b.rot, ta), ta);
-                const float jacInv = 1.f / fmax_(jac, 1e-8f);
-                const float posErr = kPushbackErp * (thr - dist) / pushDt;
-                float push = (posErr + -projVel) * jacInv;
-                if (push < 0.f) push = 0.f;
-                impulse += push * 0.25f;
-            }
+    const V3 up = rotateZ(c.rot), right = rotateY(c.rot);
+    const float radius = wheelRadius(k), rest = wheelRest(k);
+    const float suspLen = fmin_(fmax_(dist - radius, rest - kMaxTravel), rest + kMaxTravel);
+    const V3 fullRel = (c.cenOffset + rotate(c.rot, wheelAnchor(k))) - up * dist;
+    const V3 pointVel = c.vel + cross(c.ang, fullRel);
+    const float projVel = dot(normal, pointVel);
+    const float den = dot(normal, up);
+    const float clipped = den > 0.1f ? 1.f / den : 10.f;
+    const float damping = projVel * clipped < 0.f ? kDampCompression : kDampRelaxation;
+    float force = ((rest - suspLen) * kSuspStiffness - damping * projVel) * clipped * wheelScale(k);
+    if (force <= 0.f) force = 0.f;
+    const V3 ta = cross(fullRel, normal);
+    const V3 turn = invInertiaWorld(c.rot, ta);
+    float impulse = 0.f;
+    if (force != 0.f) {
+        impulse = force * kDt;
+        const float thr = rest + radius - kSuspSub;
+        if (dist < thr) {
+            const float jac = kCarInvMass + dot(turn, ta);
+            const float jacInv = 1.f / fmax_(jac, 1e-8f);
+            const float posErr = kPushbackErp * (thr - dist) / c.pushDt;
+            float push = (posErr + -projVel) * jacInv;
+            if (push < 0.f) push = 0.f;
+            impulse += push * 0.25f;
         }
-        const V3 dv = normal * (impulse * kCarInvMass);
-        V3 directAng = invInertiaWorld(b.rot, cross(fullRel, normal)) * impulse;
-        V3 directVel = kZero;
-
-        V3 axle = right;
-        if (k < 2 && fabsf(r.steerPrev) > 1e-6f) {
-            float sn, cs;
-            sincos_(r.steerPrev, &sn, &cs);
-            axle = right * cs + cross(up, right) * sn;
-        }
-        V3 axleDir = axle - normal * dot(axle, normal);
-        const float axleSq = lensq(axleDir);
-        if (axleSq > 1e-10f) {
-            axleDir = axleDir * rsqrt_(axleSq);
-            const V3 latRel = fullRel - up * dot(up, fullRel);
-            const V3 hardVel = pointVel + angCrossUp * dist;
-            const V3 curveLong = cross(axle, normal);
-            const V3 fwdDir = cross(normal, axleDir);
-            float curveIn = 0.f;
-            const float baseFric = fabsf(dot(hardVel, axle));
-            if (baseFric > 5.f) curveIn = baseFric / (fabsf(dot(hardVel, curveLong)) + baseFric);
-            const float hb = r.handbrakeVal;
-            float latBase = 1.f - 0.8f * clamp_(curveIn, 0.f, 1.f);
-            float lonBase = 1.f;
-            if (hb > 0.f) {
-                latBase *= (0.1f - 1.f) * hb + 1.f;
-                lonBase *= ((0.5f + 0.4f * clamp_(curveIn, 0.f, 1.f)) - 1.f) * hb + 1.f;
-            }
-            const float fs = r.throttleVal != 0.f ? 1.f : nonStickyFriction(normal.z);
-            const float latUsed = r.latF[k], lonUsed = r.lonF[k];
-            r.latF[k] = latBase * fs;
-            r.lonF[k] = lonBase * fs;
-            const V3 angLat = invInertiaWorld(b.rot, cross(fullRel, axleDir));
-            const float jac = kCarInvMass + dot(axleDir, cross(angLat, fullRel));
-            const float latJacInv = 1.f / fmax_(jac, 1e-8f);
-            const float sideImp = -0.2f * dot(axleDir, pointVel) * latJacInv;
-            const float lonVel = dot(fwdDir, pointVel);
-            const float rolling = r.drivePrev != 0.f ? -0.75f * r.drivePrev
-                                                     : clamp_(-lonVel * 113.73963f, -brakeTorque, brakeTorque);
-            V3 wheelImp = axleDir * (sideImp * latUsed) + fwdDir * (rolling * lonUsed);
-            wheelImp = wheelImp * ((kCarMass / 3.f) * kDt);
-            directVel = wheelImp * kCarInvMass;
-            directAng = directAng + invInertiaWorld(b.rot, cross(latRel, wheelImp));
-        }
-        b.vel = b.vel + directVel;
-        b.ang = b.ang + directAng;
-        b.dVel = b.dVel + dv;
-        normalSum = normalSum + normal;
-        count += 1;
     }
+    WheelForce f{ normal * (impulse * kCarInvMass), kZero, turn * impulse, latUsed, lonUsed };
 
-    // aggregate sticky force and auto-roll, reading the previous tick's manifold
+    V3 axle = right;
+    if (k < 2 && fabsf(c.steer) > 1e-6f) {
+        float sn, cs;
+        sincos_(c.steer, &sn, &cs);
+        axle = right * cs + cross(up, right) * sn;
+    }
+    V3 axleDir = axle - normal * dot(axle, normal);
+    const float axleSq = lensq(axleDir);
+    if (axleSq > 1e-10f) {
+        axleDir = axleDir * rsqrt_(axleSq);
+        const V3 latRel = fullRel - up * dot(up, fullRel);
+        const V3 hardVel = pointVel + cross(c.ang, up) * dist;
+        const V3 curveLong = cross(axle, normal);
+        const V3 fwdDir = cross(normal, axleDir);
+        float curveIn = 0.f;
+        const float baseFric = fabsf(dot(hardVel, axle));
+        if (baseFric > 5.f) curveIn = baseFric / (fabsf(dot(hardVel, curveLong)) + baseFric);
+        const float hb = c.handbrake;
+        float latBase = 1.f - 0.8f * clamp_(curveIn, 0.f, 1.f);
+        float lonBase = 1.f;
+        if (hb > 0.f) {
+            latBase *= (0.1f - 1.f) * hb + 1.f;
+            lonBase *= ((0.5f + 0.4f * clamp_(curveIn, 0.f, 1.f)) - 1.f) * hb + 1.f;
+        }
+        const float fs = c.throttle != 0.f ? 1.f : nonStickyFriction(normal.z);
+        f.lat = latBase * fs;
+        f.lon = lonBase * fs;
+        const V3 angLat = invInertiaWorld(c.rot, cross(fullRel, axleDir));
+        const float jac = kCarInvMass + dot(axleDir, cross(angLat, fullRel));
+        const float latJacInv = 1.f / fmax_(jac, 1e-8f);
+        const float sideImp = -0.2f * dot(axleDir, pointVel) * latJacInv;
+        const float lonVel = dot(fwdDir, pointVel);
+        const float rolling = c.drive != 0.f ? -0.75f * c.drive
+                                             : clamp_(-lonVel * 113.73963f, -c.brakeTorque, c.brakeTorque);
+        V3 wheelImp = axleDir * (sideImp * latUsed) + fwdDir * (rolling * lonUsed);
+        wheelImp = wheelImp * ((kCarMass / 3.f) * kDt);
+        f.directVel = wheelImp * kCarInvMass;
+        f.directAng = f.directAng + invInertiaWorld(c.rot, cross(latRel, wheelImp));
+    }
+    return f;
+}
+
+DI SuspCar suspCar(const Body& b, const CarRegs& r, int tick)
+{
+    return SuspCar{ b.rot, b.cen - b.pos, b.vel, b.ang, r.steerPrev, r.handbrakeVal, r.throttleVal, r.drivePrev,
+                    r.brakePrev * (kCarMass * (14.25f + 1.f / 3.f)), tick <= 1 ? kPushbackDtFirst : kDt };
+}
+
+// The forces of a car's wheels, added in wheel order.
+struct WheelSum {
+    V3 normals = kZero;
+    int count = 0;
+};
+DI void addWheel(Body& b, CarRegs& r, WheelSum& sum, int k, V3 normal, const WheelForce& f)
+{
+    r.latF[k] = f.lat;
+    r.lonF[k] = f.lon;
+    b.vel = b.vel + f.directVel;
+    b.ang = b.ang + f.directAng;
+    b.dVel = b.dVel + f.dv;
+    sum.normals = sum.normals + normal;
+    sum.count += 1;
+}
+
+// aggregate sticky force and auto-roll, reading the previous tick's manifold;
+// c: the car before its wheels' forces
+DI void finishSuspension(Body& b, CarRegs& r, const SuspCar& c, const WheelSum& sum)
+{
     const bool hasRaw = r.rawThrottle != 0.f;
     const bool hasWorld = r.manCount != 0;
+    const V3 fwd = rotateX(b.rot), right = rotateY(b.rot);
     V3 upDir = kZero;
     bool autoroll = false;
-    if (count > 0) {
-        upDir = normalSum * rsqrt_(lensq(normalSum) + 1e-16f);
-        const bool fullStick = r.throttleVal != 0.f || fabsf(dot(vel0, fwd)) > kStoppingVel;
+    if (sum.count > 0) {
+        upDir = sum.normals * rsqrt_(lensq(sum.normals) + 1e-16f);
+        const bool fullStick = r.throttleVal != 0.f || fabsf(dot(c.vel, fwd)) > kStoppingVel;
         float sticky = 0.5f;
         if (fullStick) sticky += 1.f - fabsf(upDir.z);
         b.extVel = b.extVel + upDir * (sticky * kGravity.z * kDt);
-        autoroll = hasRaw && (count < kWheels || hasWorld);
+        autoroll = hasRaw && (sum.count < kWheels || hasWorld);
     } else if (hasWorld) {
         upDir = r.manNormal;
         autoroll = hasRaw;
@@ -1577,6 +1600,101 @@ DI void applySuspension(Body& b, CarRegs& r, const Wheels& w, int tick)
     r.jumpImp = kZero;
     b.extAng = b.extAng + r.angImp;
     r.angImp = kZero;
+}
+
+DI void applySuspension(Body& b, CarRegs& r, const Wheels& w, int tick)
+{
+    const SuspCar c = suspCar(b, r, tick);
+    WheelSum sum;
+#pragma unroll
+    for (int k = 0; k < kWheels; k++) {
+        if (w.dist[k] > wheelRay(k)) continue;
+        addWheel(b, r, sum, k, w.normal[k], wheelForce(c, k, w.dist[k], w.normal[k], r.latF[k], r.lonF[k]));
+    }
+    finishSuspension(b, r, c, sum);
+}
+
+// The same for the cars of a wave (one per lane, where live), the wheels in
+// contact shared out to all lanes.  A rollout's cars spend most of their time
+// in the air or on their roofs: 7 of a wave's 64 cars have wheels on a
+// surface, yet each lane's own pass runs all four wheels' code, 3,000
+// instructions for them.  Here every wheel in contact is an item, 64 of them
+// a round; each lane computes its item's force from its owner's words in LDS,
+// and the owners add theirs in wheel order.  With more than kSuspItems wheels
+// (cars on the ground, 256 of them at kickoffs) a lane's own pass is as full
+// and saves the traffic through LDS.
+constexpr int kSuspItems = 128;
+struct SuspLds {
+    float4 in[5][64];             // rot | cenOffset, steer | vel, handbrake | ang, throttle | drive, brakeTorque, wheels in contact, -
+    float4 lat[64], lon[64];
+    float4 out[3][64];            // of the round's items: dv, lat | directVel, lon | directAng, -
+    int slots[64];
+};
+
+// dist and normal of wheel k of lane o, as the contact phase left them
+template <class WheelAt>
+DI void suspensionGroup(Body& b, CarRegs& r, const Wheels& w, bool live, int tick, SuspLds& L, int lane, WheelAt wheelAt)
+{
+    int mask = 0;
+#pragma unroll
+    for (int k = 0; k < kWheels; k++)
+        if (live && !(w.dist[k] > wheelRay(k))) mask |= 1 << k;
+    const int mine = __popc(mask), incl = waveInclusiveScan(mine), total = __builtin_amdgcn_readlane(incl, 63);
+    const SuspCar c = suspCar(b, r, tick);
+    WheelSum sum;
+    if (total > kSuspItems) {
+#pragma unroll
+        for (int k = 0; k < kWheels; k++) {
+            if (!(mask >> k & 1)) continue;
+            addWheel(b, r, sum, k, w.normal[k], wheelForce(c, k, w.dist[k], w.normal[k], r.latF[k], r.lonF[k]));
+        }
+    } else if (total > 0) {
+        if (mask) {
+            L.in[0][lane] = make_float4(c.rot.x, c.rot.y, c.rot.z, c.rot.w);
+            L.in[1][lane] = make_float4(c.cenOffset.x, c.cenOffset.y, c.cenOffset.z, c.steer);
+            L.in[2][lane] = make_float4(c.vel.x, c.vel.y, c.vel.z, c.handbrake);
+            L.in[3][lane] = make_float4(c.ang.x, c.ang.y, c.ang.z, c.throttle);
+            L.in[4][lane] = make_float4(c.drive, c.brakeTorque, __int_as_float(mask), 0.f);
+            L.lat[lane] = make_float4(r.latF[0], r.latF[1], r.latF[2], r.latF[3]);
+            L.lon[lane] = make_float4(r.lonF[0], r.lonF[1], r.lonF[2], r.lonF[3]);
+        }
+        ItemOwners owners(L.slots, incl - mine, mine);
+        for (int base = 0; base < total; base += 64) {
+            int o, q;
+            owners.next(o, q);
+            waveSync();
+            if (base + lane < total) {
+                const float4 i0 = L.in[0][o], i1 = L.in[1][o], i2 = L.in[2][o], i3 = L.in[3][o], i4 = L.in[4][o];
+                // the owner's q-th wheel in contact
+                int m = __float_as_int(i4.z);
+                for (int i = 0; i < q; i++) m &= m - 1;
+                const int k = __builtin_ctz(m);
+                const SuspCar ic{ Q4{ i0.x, i0.y, i0.z, i0.w }, V3{ i1.x, i1.y, i1.z }, V3{ i2.x, i2.y, i2.z },
+                                  V3{ i3.x, i3.y, i3.z },       i1.w, i2.w, i3.w, i4.x, i4.y, c.pushDt };
+                float dist;
+                V3 normal;
+                wheelAt(k, o, dist, normal);
+                const WheelForce f = wheelForce(ic, k, dist, normal, ((const float*)&L.lat[o])[k], ((const float*)&L.lon[o])[k]);
+                L.out[0][lane] = make_float4(f.dv.x, f.dv.y, f.dv.z, f.lat);
+                L.out[1][lane] = make_float4(f.directVel.x, f.directVel.y, f.directVel.z, f.lon);
+                L.out[2][lane] = make_float4(f.directAng.x, f.directAng.y, f.directAng.z, 0.f);
+            }
+            waveSync();
+            int at = incl - mine - base;   // this lane's next item in the round
+#pragma unroll
+            for (int k = 0; k < kWheels; k++) {
+                if (!(mask >> k & 1)) continue;
+                if (at >= 0 && at < 64) {
+                    const float4 a = L.out[0][at], v = L.out[1][at], g = L.out[2][at];
+                    addWheel(b, r, sum, k, w.normal[k],
+                             WheelForce{ V3{ a.x, a.y, a.z }, V3{ v.x, v.y, v.z }, V3{ g.x, g.y, g.z }, a.w, v.w });
+                }
+                at++;
+            }
+            waveSync();
+        }
+    }
+    if (live) finishSuspension(b, r, c, sum);
 }
 
 // -------------------------------------------------------- contact solver
@@ -1681,11 +1799,9 @@ DI void solveManifold(Body& b, const ManPt* pts, int count)
     }
 }
 
-// suspension, manifold and contact solve of one non-demoed car (Solve.cuh:286-314)
-DI void solveCarArena(CarRegs& r, const Wheels& w, bool hasBest, const ManPt& best, int tick)
+// manifold and contact solve of one non-demoed car after its suspension (Solve.cuh:286-314)
+DI void solveCarArena(CarRegs& r, Body& b, bool hasBest, const ManPt& best)
 {
-    Body b = makeBody(r.pos, r.vel, r.ang, r.cen, r.rot);
-    applySuspension(b, r, w, tick);
     ManPt pts[kMaxManifold];
 #pragma unroll
     for (int i = 0; i < kMaxManifold; i++) pts[i] = ManPt{ kZero, kZero, kZero, 0.f };

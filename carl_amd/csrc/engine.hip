@@ -271,44 +271,57 @@ __global__ __launch_bounds__(kContactBlock) void contactKernel(Dev d, uint32_t* 
 // writes them, and of the stored wheel results only the last tick's are read
 // (by the outputs), so a launch of several ticks stores the controls at its
 // first and the wheels at its last.
-template <class Handoff>
-DI void carArenaCar(const Dev& d, const Handoff& in, int kind, const void* __restrict__ actions, int tick, int car,
-                    int lane, bool first, bool last)
+//
+// susp(b, r, w, live): the suspension of the car (where live), from the body
+// with its controls applied.  With a cooperative one every lane of the wave
+// calls this (car, where ok).
+template <class Handoff, class Suspension>
+DI void carArenaCar(const Dev& d, const Handoff& in, int kind, const void* __restrict__ actions, int car, bool ok, int lane,
+                    bool first, bool last, Suspension susp)
 {
     Wheels w;
-#pragma unroll
-    for (int k = 0; k < kWheels; k++) {
-        w.dist[k] = __uint_as_float(in.get(kWsDist + k, car, lane));
-        w.normal[k] = V3{ __uint_as_float(in.get(kWsNx + k, car, lane)), __uint_as_float(in.get(kWsNy + k, car, lane)),
-                          __uint_as_float(in.get(kWsNz + k, car, lane)) };
-        w.src[k] = (int)in.get(kWsSrc + k, car, lane);
-    }
-    const int best = (int)in.get(kWsBest, car, lane);
-    ManPt bestPt{};
-    if (best >= 0) {
-        float v[10];
-#pragma unroll
-        for (int i = 0; i < 10; i++) v[i] = __uint_as_float(in.get(kWsMan + i, car, lane));
-        bestPt = ManPt{ V3{ v[0], v[1], v[2] }, V3{ v[3], v[4], v[5] }, V3{ v[6], v[7], v[8] }, v[9] };
-    }
-    const Controls ctl = decodeControls(kind, actions, car);
-    const bool demoed = d.ci(CARL_CAR_DEMOED, car) != 0;
     CarRegs r;
-    loadRegs(d, car, r);
-    if (last) storeWheelOutputs(d, car, w);
-    if (first) {
-        d.setf(CARL_CAR_CTRL_THROTTLE, car, ctl.throttle);
-        d.setf(CARL_CAR_CTRL_STEER, car, ctl.steer);
-        d.setf(CARL_CAR_CTRL_YAW, car, ctl.yaw);
-        d.setf(CARL_CAR_CTRL_PITCH, car, ctl.pitch);
-        d.setf(CARL_CAR_CTRL_ROLL, car, ctl.roll);
-        d.seti(CARL_CAR_CTRL_JUMP, car, ctl.jump);
-        d.seti(CARL_CAR_CTRL_BOOST, car, ctl.boost);
-        d.seti(CARL_CAR_CTRL_SLIDE, car, ctl.slide);
+    Body b;
+    ManPt bestPt{};
+    int best = -1;
+    bool live = false;
+    if (ok) {
+#pragma unroll
+        for (int k = 0; k < kWheels; k++) {
+            w.dist[k] = __uint_as_float(in.get(kWsDist + k, car, lane));
+            w.normal[k] = V3{ __uint_as_float(in.get(kWsNx + k, car, lane)), __uint_as_float(in.get(kWsNy + k, car, lane)),
+                              __uint_as_float(in.get(kWsNz + k, car, lane)) };
+            w.src[k] = (int)in.get(kWsSrc + k, car, lane);
+        }
+        best = (int)in.get(kWsBest, car, lane);
+        if (best >= 0) {
+            float v[10];
+#pragma unroll
+            for (int i = 0; i < 10; i++) v[i] = __uint_as_float(in.get(kWsMan + i, car, lane));
+            bestPt = ManPt{ V3{ v[0], v[1], v[2] }, V3{ v[3], v[4], v[5] }, V3{ v[6], v[7], v[8] }, v[9] };
+        }
+        const Controls ctl = decodeControls(kind, actions, car);
+        live = d.ci(CARL_CAR_DEMOED, car) == 0;
+        loadRegs(d, car, r);
+        if (last) storeWheelOutputs(d, car, w);
+        if (first) {
+            d.setf(CARL_CAR_CTRL_THROTTLE, car, ctl.throttle);
+            d.setf(CARL_CAR_CTRL_STEER, car, ctl.steer);
+            d.setf(CARL_CAR_CTRL_YAW, car, ctl.yaw);
+            d.setf(CARL_CAR_CTRL_PITCH, car, ctl.pitch);
+            d.setf(CARL_CAR_CTRL_ROLL, car, ctl.roll);
+            d.seti(CARL_CAR_CTRL_JUMP, car, ctl.jump);
+            d.seti(CARL_CAR_CTRL_BOOST, car, ctl.boost);
+            d.seti(CARL_CAR_CTRL_SLIDE, car, ctl.slide);
+        }
+        if (live) {
+            applyControls(r, ctl, w);
+            b = makeBody(r.pos, r.vel, r.ang, r.cen, r.rot);
+        }
     }
-    if (demoed) return;
-    applyControls(r, ctl, w);
-    solveCarArena(r, w, best >= 0, bestPt, tick);
+    susp(b, r, w, live);
+    if (!live) return;
+    solveCarArena(r, b, best >= 0, bestPt);
     storeRegs(d, car, r);
 }
 
@@ -318,8 +331,10 @@ __global__ __launch_bounds__(kTickBlock, 2) void carArenaKernel(Dev d, const uin
 {
     const int car = range.begin * d.nCars + blockIdx.x * kTickBlock + threadIdx.x;
     if (car < range.end * d.nCars)
-        carArenaCar(d, WsHandoff{ const_cast<uint32_t*>(ws), d.nTotal }, kind, actions, tick, car,
-                    (int)threadIdx.x & 63, true, true);
+        carArenaCar(d, WsHandoff{ const_cast<uint32_t*>(ws), d.nTotal }, kind, actions, car, true, (int)threadIdx.x & 63,
+                    true, true, [&](Body& b, CarRegs& r, const Wheels& w, bool live) {
+                        if (live) applySuspension(b, r, w, tick);
+                    });
 }
 
 // Episode clock and the car-car pairs of one simulation, (b, a) with b the
@@ -527,9 +542,13 @@ constexpr int kWindowContactOwners = CARL_WINDOW_CONTACT_OWNERS;
 // threads of the workgroup wrote in the phase before.
 union WaveLds {
     ContactLdsT<kWindowContactOwners> contact;
-    uint32_t hand[kWsPlanes * 64];   // the contact phase's results, read by the car-arena phase
+    struct {
+        uint32_t hand[kWsPlanes * 64];   // the contact phase's results, read by the car-arena phase
+        SuspLds susp;                    // that phase's wheels in contact
+    };
     BallLds ball;
 };
+static_assert(sizeof(WaveLds) == sizeof(ContactLdsT<kWindowContactOwners>), "the contact search sets the size");
 // Lane l of wave w is contact owner and car-arena thread of the same car: a
 // block holds at most kWindowBlock cars, one contact group per wave, so each
 // car's handoff stays in the lane that produced it.
@@ -538,6 +557,21 @@ struct WindowLds {
     WaveLds wave[kWindowWaves];
 };
 static_assert(4 * sizeof(WindowLds) <= 160 * 1024, "four window workgroups per CU");
+
+// carArenaCar of a wave's cars (one per lane, where ok) from the LDS handoff,
+// their wheels shared out to all lanes.  Every lane of the wave calls it.
+DI void carArenaWave(const Dev& d, WaveLds& L, int kind, const void* __restrict__ actions, int tick, int car, bool ok,
+                     int lane, bool first, bool last)
+{
+    carArenaCar(d, LdsHandoff{ L.hand }, kind, actions, car, ok, lane, first, last,
+                [&](Body& b, CarRegs& r, const Wheels& w, bool live) {
+                    suspensionGroup(b, r, w, live, tick, L.susp, lane, [&](int k, int o, float& dist, V3& normal) {
+                        dist = __uint_as_float(L.hand[(kWsDist + k) * 64 + o]);
+                        normal = V3{ __uint_as_float(L.hand[(kWsNx + k) * 64 + o]), __uint_as_float(L.hand[(kWsNy + k) * 64 + o]),
+                                     __uint_as_float(L.hand[(kWsNz + k) * 64 + o]) };
+                    });
+                });
+}
 
 // Phases of a tick in the window kernel, timed by the stage profile.
 enum WindowStage { kStageContact, kStageCarArena, kStageBall, kStageFinish, kStagePads, kWindowStages };
@@ -752,8 +786,7 @@ DI void tickWindowBody(const Dev& d0, int screen, int kind, const void* __restri
         mark(kStageContact);
         {
             const int car = m.car[lane];
-            if (car >= 0)
-                carArenaCar(d, LdsHandoff{ L.hand }, kind, actions, tick, car, lane, k == 0, k == ticks - 1);
+            carArenaWave(d, L, kind, actions, tick, max(car, 0), car >= 0, lane, k == 0, k == ticks - 1);
         }
         waveSync();
         mark(kStageCarArena);
@@ -885,8 +918,7 @@ __global__ __launch_bounds__(kWindowBlock, 2) void tickWindowBlockKernel(Dev d, 
                                                                car < waveCarEnd, L.wave[wave].contact, lane);
         __syncthreads();
         mark(kStageContact);
-        if (car < waveCarEnd)
-            carArenaCar(d, LdsHandoff{ L.wave[wave].hand }, kind, actions, tick, car, lane, k == 0, k == ticks - 1);
+        carArenaWave(d, L.wave[wave], kind, actions, tick, car, car < waveCarEnd, lane, k == 0, k == ticks - 1);
         __syncthreads();
         mark(kStageCarArena);
         // the block's simulations split evenly between the waves: at most
