@@ -56,11 +56,44 @@ void check(int rc)
     throw std::runtime_error(msg);
 }
 
-py::capsule toCapsule(py::object obj, void* stream)
-{
-    if (py::isinstance<py::capsule>(obj)) return obj.cast<py::capsule>();
-    return obj.attr("__dlpack__")(py::arg("stream") = reinterpret_cast<intptr_t>(stream)).cast<py::capsule>();
-}
+// The DLPack exports of one call's inputs, each ordered before the engine's
+// stream.  A torch tensor's export with a stream records an event on torch's
+// current stream and makes `stream` wait for it, about 20 us of host time,
+// and covers everything that stream was given before: once one plain
+// torch.Tensor on cuda:0 has done so, the further ones of the call are
+// exported as they are (stream -1, no ordering).  Any other producer orders
+// its own data, and since its export may run anything, so does the next
+// tensor after it.  One object per call: nothing outlives it.  A reset and an
+// indexed restore from eleven tensors 360 -> 174 us at 65,536 1v1 simulations.
+class InputOrder {
+    void* stream_;
+    bool ordered_ = false;
+
+    static bool plainTensor(const py::object& obj)
+    {
+        const auto torch = py::reinterpret_steal<py::object>(PyImport_GetModule(py::str("torch").ptr()));
+        if (!torch) {
+            PyErr_Clear();
+            return false;
+        }
+        if (!py::hasattr(torch, "Tensor") || !py::type::of(obj).is(torch.attr("Tensor"))) return false;
+        return obj.attr("is_cuda").cast<bool>() && obj.attr("get_device")().cast<int>() == 0;
+    }
+
+public:
+    explicit InputOrder(void* stream) : stream_(stream) {}
+
+    py::capsule capsule(const py::object& obj)
+    {
+        if (py::isinstance<py::capsule>(obj)) return obj.cast<py::capsule>();
+        const bool plain = plainTensor(obj);
+        const intptr_t on = plain && ordered_ ? -1 : reinterpret_cast<intptr_t>(stream_);
+        ordered_ = false;
+        auto cap = obj.attr("__dlpack__")(py::arg("stream") = on).cast<py::capsule>();
+        ordered_ = plain;
+        return cap;
+    }
+};
 
 struct OwnedShape {
     int64_t shape[3];
@@ -169,10 +202,10 @@ class Env {
         }
     }
 
-    TensorView view(py::object obj, const std::string& name, std::initializer_list<int64_t> shape, uint8_t code,
-                    uint8_t bits) const
+    TensorView view(InputOrder& order, py::object obj, const std::string& name, std::initializer_list<int64_t> shape,
+                    uint8_t code, uint8_t bits) const
     {
-        py::capsule cap = toCapsule(obj, stream());
+        py::capsule cap = order.capsule(obj);
         const auto* m = cap.get_pointer<DLManagedTensor>();
         if (!m) throw py::value_error("invalid DLPack tensor");
         const DLTensor t = m->dl_tensor;
@@ -180,9 +213,9 @@ class Env {
         return TensorView{ std::move(cap), t };
     }
 
-    TensorView selection(py::object obj) const
+    TensorView selection(InputOrder& order, py::object obj) const
     {
-        py::capsule cap = toCapsule(obj, stream());
+        py::capsule cap = order.capsule(obj);
         const auto* m = cap.get_pointer<DLManagedTensor>();
         if (!m) throw py::value_error("invalid DLPack tensor");
         const DLTensor t = m->dl_tensor;
@@ -196,9 +229,9 @@ class Env {
         return TensorView{ std::move(cap), t };
     }
 
-    TensorView demoedView(py::object obj, const std::string& name, int n, bool& byteDemoed) const
+    TensorView demoedView(InputOrder& order, py::object obj, const std::string& name, int n, bool& byteDemoed) const
     {
-        py::capsule cap = toCapsule(obj, stream());
+        py::capsule cap = order.capsule(obj);
         const auto* m = cap.get_pointer<DLManagedTensor>();
         if (!m) throw py::value_error("invalid DLPack tensor");
         const DLTensor t = m->dl_tensor;
@@ -211,7 +244,7 @@ class Env {
 
     TensorView actionData(py::object actions, bool continuous) const
     {
-        py::capsule cap = toCapsule(actions, stream());
+        py::capsule cap = InputOrder(stream()).capsule(actions);
         const auto* m = cap.get_pointer<DLManagedTensor>();
         if (!m) throw py::value_error("invalid DLPack tensor");
         const DLTensor& t = m->dl_tensor;
@@ -284,17 +317,18 @@ public:
 
     void setBall(py::object position, py::object velocity, py::object angular, py::object indices)
     {
+        InputOrder order(stream());
         int n = nSim_;
         std::optional<TensorView> sel;
         const int64_t* idx = nullptr;
         if (!indices.is_none()) {
-            sel.emplace(selection(indices));
+            sel.emplace(selection(order, indices));
             idx = selectionPointer(*sel);
             n = (int)sel->tensor.shape[0];
         }
-        const auto p = view(position, "position", { n, 3 }, kDLFloat, 32);
-        const auto v = view(velocity, "velocity", { n, 3 }, kDLFloat, 32);
-        const auto a = view(angular, "angular_velocity", { n, 3 }, kDLFloat, 32);
+        const auto p = view(order, position, "position", { n, 3 }, kDLFloat, 32);
+        const auto v = view(order, velocity, "velocity", { n, 3 }, kDLFloat, 32);
+        const auto a = view(order, angular, "angular_velocity", { n, 3 }, kDLFloat, 32);
         check(carl_env_set_ball(env_, (const float*)p.data(), (const float*)v.data(), (const float*)a.data(), idx, n));
         check(carl_env_synchronize(env_));
     }
@@ -302,23 +336,24 @@ public:
     void setCar(py::object position, py::object rotation, py::object velocity, py::object angular, py::object demoed,
                 py::object boost, py::object internal, py::object indices)
     {
+        InputOrder order(stream());
         int n = nSim_;
         std::optional<TensorView> sel;
         const int64_t* idx = nullptr;
         if (!indices.is_none()) {
-            sel.emplace(selection(indices));
+            sel.emplace(selection(order, indices));
             idx = selectionPointer(*sel);
             n = (int)sel->tensor.shape[0];
         }
-        const auto p = view(position, "position", { n, nCars_, 3 }, kDLFloat, 32);
-        const auto r = view(rotation, "rotation", { n, nCars_, 4 }, kDLFloat, 32);
-        const auto v = view(velocity, "velocity", { n, nCars_, 3 }, kDLFloat, 32);
-        const auto a = view(angular, "angular_velocity", { n, nCars_, 3 }, kDLFloat, 32);
+        const auto p = view(order, position, "position", { n, nCars_, 3 }, kDLFloat, 32);
+        const auto r = view(order, rotation, "rotation", { n, nCars_, 4 }, kDLFloat, 32);
+        const auto v = view(order, velocity, "velocity", { n, nCars_, 3 }, kDLFloat, 32);
+        const auto a = view(order, angular, "angular_velocity", { n, nCars_, 3 }, kDLFloat, 32);
         bool byteDemoed = false;
-        const auto d = demoedView(demoed, "demoed", n, byteDemoed);
+        const auto d = demoedView(order, demoed, "demoed", n, byteDemoed);
         std::optional<TensorView> b, in;
-        if (!boost.is_none()) b.emplace(view(boost, "boost", { n, nCars_ }, kDLFloat, 32));
-        if (!internal.is_none()) in.emplace(view(internal, "internal_state", { n, nCars_, kInternalSize }, kDLFloat, 32));
+        if (!boost.is_none()) b.emplace(view(order, boost, "boost", { n, nCars_ }, kDLFloat, 32));
+        if (!internal.is_none()) in.emplace(view(order, internal, "internal_state", { n, nCars_, kInternalSize }, kDLFloat, 32));
         check(carl_env_set_car(env_, (const float*)p.data(), (const float*)r.data(), (const float*)v.data(),
                                (const float*)a.data(), d.data(), byteDemoed ? 1 : 0,
                                b ? (const float*)b->data() : nullptr, in ? (const float*)in->data() : nullptr, idx, n));
@@ -332,36 +367,37 @@ public:
         releaseInputs();
         if (!mask.is_none() && !indices.is_none())
             throw py::value_error("specify reset_mask or simulation_indices, not both");
+        InputOrder order(stream());
         int n = nSim_;
         std::optional<TensorView> sel, maskView;
         const int64_t* idx = nullptr;
         if (!indices.is_none()) {
-            sel.emplace(selection(indices));
+            sel.emplace(selection(order, indices));
             idx = selectionPointer(*sel);
             n = (int)sel->tensor.shape[0];
         }
-        if (!mask.is_none()) maskView.emplace(view(mask, "reset_mask", { nSim_ }, kDLBool, 8));
+        if (!mask.is_none()) maskView.emplace(view(order, mask, "reset_mask", { nSim_ }, kDLBool, 8));
         // every input is validated before any state-changing call
-        const auto bp = view(bpos, "ball_position", { n, 3 }, kDLFloat, 32);
-        const auto bv = view(bvel, "ball_velocity", { n, 3 }, kDLFloat, 32);
-        const auto ba = view(bang, "ball_angular_velocity", { n, 3 }, kDLFloat, 32);
-        const auto cp = view(cpos, "car_position", { n, nCars_, 3 }, kDLFloat, 32);
-        const auto cr = view(crot, "car_rotation", { n, nCars_, 4 }, kDLFloat, 32);
-        const auto cv = view(cvel, "car_velocity", { n, nCars_, 3 }, kDLFloat, 32);
-        const auto ca = view(cang, "car_angular_velocity", { n, nCars_, 3 }, kDLFloat, 32);
+        const auto bp = view(order, bpos, "ball_position", { n, 3 }, kDLFloat, 32);
+        const auto bv = view(order, bvel, "ball_velocity", { n, 3 }, kDLFloat, 32);
+        const auto ba = view(order, bang, "ball_angular_velocity", { n, 3 }, kDLFloat, 32);
+        const auto cp = view(order, cpos, "car_position", { n, nCars_, 3 }, kDLFloat, 32);
+        const auto cr = view(order, crot, "car_rotation", { n, nCars_, 4 }, kDLFloat, 32);
+        const auto cv = view(order, cvel, "car_velocity", { n, nCars_, 3 }, kDLFloat, 32);
+        const auto ca = view(order, cang, "car_angular_velocity", { n, nCars_, 3 }, kDLFloat, 32);
         bool byteDemoed = false;
-        const auto dm = demoedView(demoed, "car_demoed", n, byteDemoed);
+        const auto dm = demoedView(order, demoed, "car_demoed", n, byteDemoed);
         std::optional<TensorView> bo, in, bl, orr, tk;
-        if (!boost.is_none()) bo.emplace(view(boost, "car_boost", { n, nCars_ }, kDLFloat, 32));
+        if (!boost.is_none()) bo.emplace(view(order, boost, "car_boost", { n, nCars_ }, kDLFloat, 32));
         if (!internal.is_none())
-            in.emplace(view(internal, "car_internal_state", { n, nCars_, kInternalSize }, kDLFloat, 32));
+            in.emplace(view(order, internal, "car_internal_state", { n, nCars_, kInternalSize }, kDLFloat, 32));
         const bool hasMatch = !blue.is_none();
         if (hasMatch != !orange.is_none() || hasMatch != !ticks.is_none())
             throw py::value_error("blue_score, orange_score and episode_ticks must be supplied together");
         if (hasMatch) {
-            bl.emplace(view(blue, "blue_score", { n }, kDLInt, 32));
-            orr.emplace(view(orange, "orange_score", { n }, kDLInt, 32));
-            tk.emplace(view(ticks, "episode_ticks", { n }, kDLInt, 32));
+            bl.emplace(view(order, blue, "blue_score", { n }, kDLInt, 32));
+            orr.emplace(view(order, orange, "orange_score", { n }, kDLInt, 32));
+            tk.emplace(view(order, ticks, "episode_ticks", { n }, kDLInt, 32));
         }
         if (n == 0) return;
         const uint8_t* m = maskView ? (const uint8_t*)maskView->data() : nullptr;
@@ -393,28 +429,30 @@ public:
 
     void setMatchState(py::object blue, py::object orange, py::object ticks, py::object indices)
     {
+        InputOrder order(stream());
         int n = nSim_;
         std::optional<TensorView> sel;
         const int64_t* idx = nullptr;
         if (!indices.is_none()) {
-            sel.emplace(selection(indices));
+            sel.emplace(selection(order, indices));
             idx = selectionPointer(*sel);
             n = (int)sel->tensor.shape[0];
         }
-        const auto b = view(blue, "blue_score", { n }, kDLInt, 32);
-        const auto o = view(orange, "orange_score", { n }, kDLInt, 32);
-        const auto t = view(ticks, "episode_ticks", { n }, kDLInt, 32);
+        const auto b = view(order, blue, "blue_score", { n }, kDLInt, 32);
+        const auto o = view(order, orange, "orange_score", { n }, kDLInt, 32);
+        const auto t = view(order, ticks, "episode_ticks", { n }, kDLInt, 32);
         check(carl_env_set_match(env_, (const int32_t*)b.data(), (const int32_t*)o.data(), (const int32_t*)t.data(),
                                  idx, n));
     }
 
     void resetBoostPads(py::object indices)
     {
+        InputOrder order(stream());
         int n = nSim_;
         std::optional<TensorView> sel;
         const int64_t* idx = nullptr;
         if (!indices.is_none()) {
-            sel.emplace(selection(indices));
+            sel.emplace(selection(order, indices));
             idx = selectionPointer(*sel);
             n = (int)sel->tensor.shape[0];
         }
@@ -466,7 +504,7 @@ public:
     void tick(py::object actions, int kind, int n)
     {
         releaseInputs();
-        py::capsule cap = toCapsule(actions, stream());
+        py::capsule cap = InputOrder(stream()).capsule(actions);
         const auto* m = cap.get_pointer<DLManagedTensor>();
         if (!m) throw py::value_error("invalid DLPack tensor");
         const DLTensor& t = m->dl_tensor;
