@@ -64,7 +64,7 @@ void check(int rc)
 // exported as they are (stream -1, no ordering).  Any other producer orders
 // its own data, and since its export may run anything, so does the next
 // tensor after it.  One object per call: nothing outlives it.  A reset and an
-// indexed restore from eleven tensors 360 -> 174 us at 65,536 1v1 simulations.
+// indexed restore from ten tensors 360 -> 174 us at 65,536 1v1 simulations.
 class InputOrder {
     void* stream_;
     bool ordered_ = false;
@@ -517,6 +517,32 @@ public:
         holdUntilConsumed({ cap });
     }
 
+    // What CARLTorchVectorEnv.step returns of the last step, into arrays that
+    // its caller has allocated (device addresses, sizes as carl_vector_io
+    // states; 0 for the optional ones).
+    void vectorOutputs(uintptr_t obs, uintptr_t reward, uintptr_t terminated, uintptr_t truncated, uintptr_t done,
+                       uintptr_t returns, uintptr_t lengths, uintptr_t scoreDifference, uintptr_t episodeTicks,
+                       uintptr_t overtime, uintptr_t stepReturns, uintptr_t stepLengths, uintptr_t stepDone,
+                       uintptr_t ended)
+    {
+        carl_vector_io io{};
+        io.obs = reinterpret_cast<float*>(obs);
+        io.reward = reinterpret_cast<float*>(reward);
+        io.terminated = reinterpret_cast<uint8_t*>(terminated);
+        io.truncated = reinterpret_cast<uint8_t*>(truncated);
+        io.done = reinterpret_cast<uint8_t*>(done);
+        io.returns = reinterpret_cast<float*>(returns);
+        io.lengths = reinterpret_cast<int64_t*>(lengths);
+        io.score_difference = reinterpret_cast<int32_t*>(scoreDifference);
+        io.episode_ticks = reinterpret_cast<int32_t*>(episodeTicks);
+        io.overtime = reinterpret_cast<uint8_t*>(overtime);
+        io.step_returns = reinterpret_cast<float*>(stepReturns);
+        io.step_lengths = reinterpret_cast<int64_t*>(stepLengths);
+        io.step_done = reinterpret_cast<uint8_t*>(stepDone);
+        io.ended = reinterpret_cast<int32_t*>(ended);
+        check(carl_env_vector_outputs(env_, &io));
+    }
+
     void resetDones() { check(carl_env_reset_dones(env_)); }
     void synchronize() { check(carl_env_synchronize(env_)); }
     void enableTiming(bool on, bool ticks, bool packing, bool stages)
@@ -709,6 +735,7 @@ PYBIND11_MODULE(_carl, m)
         .def("get_continuous_actions", [](Env& e) { return e.buffer(CARL_BUF_CONTINUOUS_ACTIONS); })
         .def("reset_dones", &Env::resetDones)
         .def("synchronize", &Env::synchronize)
+        .def("_vector_outputs", &Env::vectorOutputs)
         .def("enable_tick_timing", &Env::enableTiming, py::arg("enable") = true, py::arg("ticks") = true,
              py::arg("packing") = false, py::arg("stages") = false)
         .def("tick_timing", &Env::tickTiming)

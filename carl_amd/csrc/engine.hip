@@ -1347,6 +1347,65 @@ __global__ __launch_bounds__(kPackBlock) void stepEnvKernel(Dev d, StepIO io, in
     for (int w = t + kCopyRegs * kPackBlock; w < copyWords; w += kPackBlock) io.actionCopy[w0 + w] = io.actions[w0 + w];
 }
 
+// What a vector environment (one agent per car) returns of a step, in one
+// launch: the observation rows copied to the caller, each agent's reward and
+// flags, its running return and length, and the list of the agents whose
+// episode ended.  Bound by the copy at large sizes and by its launch at small
+// ones; as separate copies and elementwise kernels the same outputs took
+// about 25 launches of about 5 us (a vector step of 50,001 1v1 simulations
+// 849 -> 675 us, of 17 425 -> 333 us).
+constexpr int kVectorBlock = 256;
+constexpr int kVectorBlocks = 4096;
+__global__ __launch_bounds__(kVectorBlock) void vectorOutputsKernel(Dev d, const float* __restrict__ obs, size_t obsWords,
+                                                                   const float* __restrict__ rewards,
+                                                                   const bool* __restrict__ dones,
+                                                                   const int32_t* __restrict__ tscore,
+                                                                   const int32_t* __restrict__ tticks,
+                                                                   const bool* __restrict__ tovertime, carl_vector_io io)
+{
+    const size_t stride = (size_t)gridDim.x * kVectorBlock, i0 = (size_t)blockIdx.x * kVectorBlock + threadIdx.x;
+    for (size_t a = i0; a < (size_t)d.nTotal; a += stride) {
+        const int s = (int)a / d.nCars, local = (int)a % d.nCars;
+        const bool done = dones[s];
+        const float scored = rewards[s];
+        const bool goal = done && scored != 0.f;
+        const float reward = scored * (local < d.nBlue ? 1.f : -1.f);
+        const float total = io.returns[a] + reward;
+        const int64_t length = io.lengths[a] + 1;
+        io.reward[a] = reward;
+        io.terminated[a] = goal;
+        io.truncated[a] = done && !goal;
+        io.done[a] = done;
+        io.returns[a] = done ? 0.f : total;
+        io.lengths[a] = done ? 0 : length;
+        if (io.step_returns) {
+            io.step_returns[a] = total;
+            io.step_lengths[a] = length;
+            io.step_done[a] = done;
+        }
+        if (io.ended && done) {
+            int32_t* at = io.ended + 4 + 4 * (size_t)atomicAdd(io.ended, 1);
+            at[0] = (int32_t)a;
+            at[1] = (int32_t)__float_as_uint(total);
+            at[2] = (int32_t)(length & 0xffffffffll);
+            at[3] = (int32_t)(length >> 32);
+        }
+        if (local == 0) {
+            io.score_difference[s] = done ? 0 : tscore[s];
+            io.episode_ticks[s] = done ? 0 : tticks[s];
+            io.overtime[s] = !done && tovertime[s];
+        }
+    }
+    // 16 bytes per lane and access where the caller's rows allow it
+    size_t from = 0;
+    if (((size_t)io.obs & 15) == 0) {
+        from = obsWords & ~(size_t)3;
+        for (size_t i = i0; i < from / 4; i += stride)
+            __builtin_nontemporal_store(reinterpret_cast<const F4v*>(obs)[i], reinterpret_cast<F4v*>(io.obs) + i);
+    }
+    for (size_t i = from + i0; i < obsWords; i += stride) io.obs[i] = obs[i];
+}
+
 // The rows a mask sets, compacted into list[0..*count): each thread scans
 // kCompactRows consecutive rows, a workgroup scan places the threads' rows,
 // and each workgroup takes its place in the list with one atomic add on the
@@ -2787,6 +2846,26 @@ int carl_env_pack_state(carl_env* e, const uint8_t* mask)
 {
     CARL_TRY(checkEnv(e));
     return packState(e, e->state, 1, (const bool*)mask);
+}
+
+int carl_env_vector_outputs(carl_env* e, const carl_vector_io* io)
+{
+    CARL_TRY(checkEnv(e));
+    if (!io) return fail(CARL_ERR_VALUE, "null vector outputs");
+    if (!io->obs || !io->reward || !io->terminated || !io->truncated || !io->done || !io->returns || !io->lengths ||
+        !io->score_difference || !io->episode_ticks || !io->overtime)
+        return fail(CARL_ERR_VALUE, "null vector output");
+    if ((io->step_returns != nullptr) != (io->step_lengths != nullptr) ||
+        (io->step_returns != nullptr) != (io->step_done != nullptr))
+        return fail(CARL_ERR_VALUE, "step_returns, step_lengths and step_done must be given together");
+    if (io->ended) clearCountKernel<<<1, 1, 0, e->stream>>>(io->ended);
+    const size_t words = (size_t)e->nTotal * e->obsDim;
+    // 8 words per thread; beyond kVectorBlocks the threads stride
+    const size_t blocks = (words + 8 * kVectorBlock - 1) / (8 * kVectorBlock);
+    vectorOutputsKernel<<<(int)std::min<size_t>(blocks, kVectorBlocks), kVectorBlock, 0, e->stream>>>(
+        e->dev(), e->obs, words, e->rewards, e->dones, e->tscore, e->tticks, e->tovertime, *io);
+    HIP_TRY(hipGetLastError());
+    return CARL_OK;
 }
 
 int carl_env_set_actions(carl_env* e, int kind, const void* actions)

@@ -196,6 +196,9 @@ def _request_from_typed(state: CARLResetState, eligible: th.Tensor, n_cars: int,
 
 # ---------------------------------------------------------------- episodes
 
+_REPORT_HEAD = 255   # ended episodes read back together with their count
+
+
 class _EpisodeLedger:
     """Running return and length per agent, and the reports of episodes that
     end: returned by the step that ends them, or (deferred) kept on the
@@ -211,6 +214,17 @@ class _EpisodeLedger:
         self.returns.zero_()
         self.lengths.zero_()
         self.pending.clear()
+
+    def report(self, ended: th.Tensor) -> dict[str, list[Any]] | None:
+        """The report of the episodes in a step's native list (carl_vector_io
+        `ended`), in agent order; None for none."""
+        head = ended[: 4 * (_REPORT_HEAD + 1)].cpu().numpy()
+        count = int(head[0])
+        if count == 0:
+            return None
+        rows = (head if count <= _REPORT_HEAD else ended.cpu().numpy())[4 : 4 * (count + 1)].reshape(count, 4)
+        rows = np.ascontiguousarray(rows[np.argsort(rows[:, 0])])
+        return {"reward": rows.view(np.float32)[:, 1].tolist(), "length": rows.view(np.int64)[:, 1].tolist()}
 
     def record(self, reward: th.Tensor, done: th.Tensor) -> dict[str, list[Any]] | None:
         """Add a step; the report of the episodes it ends (None if none
@@ -469,6 +483,8 @@ class CARLTorchVectorEnv(VectorEnv):
         if actions.shape != (self.n_envs, width):
             raise ValueError(f"Expected actions shaped {(self.n_envs, width)}")
         actions = actions.view(self.n_sim, self.n_cars, width)
+        if self._copy_outputs and not self.reward_funcs and self.reset_state_provider is None:
+            return self._step_native(actions)
 
         self._bridge.join()
         (self._env.step if self.discrete_actions else self._env.step_continuous)(actions)
@@ -502,6 +518,49 @@ class CARLTorchVectorEnv(VectorEnv):
         else:
             info = {**report, "final_obs": self._obs_view(env.get_transition_obs()), "_final_obs": done,
                     **reward_info}
+        return obs, reward, terminated, truncated, info
+
+    def _step_native(self, actions: th.Tensor):
+        """step() with the engine's own reward and resets and copied outputs:
+        everything that it returns is written by one kernel on the engine's
+        stream (by separate torch operations on the engine's buffers a step of
+        17 matches took 425 us, of 50,001 849 us; so 333 and 675 us)."""
+        env, n, device = self._env, self.n_envs, self.device
+        ledger, deferred = self._ledger, self.defer_episode_reporting
+        obs = th.empty((n, self._obs_dim), device=device)
+        reward = th.empty(n, device=device)
+        terminated, truncated, done = (th.empty(n, dtype=th.bool, device=device) for _ in range(3))
+        score = th.empty(self.n_sim, dtype=th.int32, device=device)
+        ticks = th.empty(self.n_sim, dtype=th.int32, device=device)
+        overtime = th.empty(self.n_sim, dtype=th.bool, device=device)
+        if deferred:
+            totals = (th.empty_like(ledger.returns), th.empty_like(ledger.lengths), th.empty_like(done))
+            report_to = (*(x.data_ptr() for x in totals), 0)
+        else:
+            ended = th.empty(4 * (n + 1), dtype=th.int32, device=device)
+            report_to = (0, 0, 0, ended.data_ptr())
+
+        self._bridge.join()
+        try:
+            (env.step if self.discrete_actions else env.step_continuous)(actions)
+            env._vector_outputs(obs.data_ptr(), reward.data_ptr(), terminated.data_ptr(), truncated.data_ptr(),
+                                done.data_ptr(), ledger.returns.data_ptr(), ledger.lengths.data_ptr(),
+                                score.data_ptr(), ticks.data_ptr(), overtime.data_ptr(), *report_to)
+        finally:
+            # no memory above goes back to torch's stream before the engine is done with it
+            self._bridge.join()
+        self._score_difference, self._episode_ticks, self._overtime = score, ticks, overtime
+        self._state = self._observation = None
+        obs = CARLObservation.from_tensor(obs, self.n_cars)
+        if deferred:
+            ledger.pending.append(totals)
+            info = {"final_obs": self._obs_view(env.get_transition_obs()), "_final_obs": done}
+        else:
+            report = ledger.report(ended)
+            if report is None:
+                info = {"reward": [], "length": []}
+            else:
+                info = {**report, "final_obs": self._obs_view(env.get_transition_obs()), "_final_obs": done}
         return obs, reward, terminated, truncated, info
 
     def drain_episode_reports(self) -> dict[str, list[Any]]:

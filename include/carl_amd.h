@@ -290,6 +290,33 @@ int carl_env_reset(carl_env* env);
 /* Reset simulations whose episode ended (goal, timeouts, overtime expiry). */
 int carl_env_reset_dones(carl_env* env);
 
+/* ---- vector environment outputs (no reference counterpart) --------------
+ * What CARLTorchVectorEnv.step returns of the last carl_env_step, for one
+ * agent per car (n_agents = n_sim * n_cars), written by one kernel on the
+ * environment stream into the caller's device arrays.  An agent's reward is
+ * its simulation's score change, negated for orange; an episode that ended on
+ * one is terminated, any other that ended truncated.  returns and lengths run
+ * over an episode: this step is added, and those of episodes that ended are
+ * left at zero. */
+typedef struct carl_vector_io {
+    float* obs;                 /* [n_agents, obs_dim]: a copy of the observations */
+    float* reward;              /* [n_agents] */
+    uint8_t *terminated, *truncated, *done;        /* [n_agents], 0 or 1 */
+    float* returns;             /* [n_agents], read and written */
+    int64_t* lengths;           /* [n_agents], read and written */
+    int32_t *score_difference, *episode_ticks;     /* [n_sim], 0 where the episode ended */
+    uint8_t* overtime;          /* [n_sim], 0 where the episode ended, else 0 or 1 */
+    /* all three or none: this step's totals before the zeroing, and done again */
+    float* step_returns;
+    int64_t* step_lengths;
+    uint8_t* step_done;
+    /* [4 + 4 n_agents] or NULL: the number of agents whose episode ended, then
+     * from word 4 for each, in no order: agent, return (float bits), length
+     * (low word, high word) */
+    int32_t* ended;
+} carl_vector_io;
+int carl_env_vector_outputs(carl_env* env, const carl_vector_io* io);
+
 /* ---- EnvIO packs (for C++ hosts composing the step themselves) ----------
  * The step's post-tick sequence of python/carl.cu:359-367 is
  *   pack_rewards_dones; pack_transition_state(frameskip);
