@@ -974,10 +974,17 @@ __global__ __launch_bounds__(kWindowBlock, 2) void tickWindowBlockKernel(Dev d, 
 // The counts of every deal set and group (one workgroup each).
 __global__ void clearDealKernel(int* counts) { counts[blockIdx.x * blockDim.x + threadIdx.x] = 0; }
 
-__global__ void resetKernel(Dev d, int nOrange)
+// A full reset: the first carBlocks workgroups one car per thread, the others
+// one simulation per thread (one thread for a simulation and all of its cars
+// ran 1,024 waves of 180 stores each at 65,536 1v1 simulations: 23 -> 16 us).
+__global__ __launch_bounds__(kTickBlock) void resetKernel(Dev d, int carBlocks)
 {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < d.nSim) fullResetSim(d, s, nOrange);
+    const int i = ((int)blockIdx.x - ((int)blockIdx.x < carBlocks ? 0 : carBlocks)) * kTickBlock + threadIdx.x;
+    if ((int)blockIdx.x < carBlocks) {
+        if (i < d.nTotal) fullResetCar(d, i / d.nCars, i % d.nCars);
+    } else if (i < d.nSim) {
+        fullResetSimWords(d, i);
+    }
 }
 
 __global__ void resetDonesKernel(Dev d, int nOrange, int tickCount, DoneRule rule)
@@ -998,14 +1005,9 @@ __global__ void rewardsDonesKernel(Dev d, int tickCount, DoneRule rule, float* r
     tOvertime[s] = d.si(CARL_SIM_OVERTIME, s) != 0;
 }
 
-__global__ void matchKernel(Dev d, int* score, int* ticks, bool* overtime, const bool* mask, const int* list,
-                            const int* count)
+__global__ void matchKernel(Dev d, int* score, int* ticks, bool* overtime, const bool* mask)
 {
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (list) {
-        if (s >= *count) return;
-        s = list[s];
-    }
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= d.nSim || (mask && !mask[s])) return;
     score[s] = d.si(CARL_SIM_BLUE_SCORE, s) - d.si(CARL_SIM_ORANGE_SCORE, s);
     ticks[s] = d.si(CARL_SIM_EPISODE_TICKS, s);
@@ -1179,30 +1181,98 @@ DI void packRowsGathered(float* out, int rowLen, int i0, int i1, RowOf&& rowOf, 
     }
 }
 
-// The state rows of the simulations list[0..*count).
-__global__ __launch_bounds__(kPackBlock) void stateListKernel(Dev d, float* out, int stateDimV, int touchWindow,
-                                                             int tickCount, const int* list, const int* count)
+// The outputs that a reset changes, in one launch: the state rows, the
+// observation rows and the match state (and, where asked for, the transition
+// state and the rewards and flags of the last step), each a range of the
+// workgroups.  Every range is a latency chain that leaves the GPU half empty,
+// so side by side they take little longer than the observations alone: at
+// 65,536 1v1 simulations 24 us against 18.3 + 7.4 + 4.1 in three launches (29
+// against 41 with the transition state and rewards), for a quarter of 131,072
+// 2v2 simulations 53 against 38.6 + 21.9 + 5.1.
+struct LivePack {
+    float *obs, *state;
+    float* tstate;                    // null: not packed
+    int32_t *score, *ticks;           // null score: no match state
+    bool* overtime;
+    float* rewards;                   // null: no rewards and flags
+    bool *dones, *tovertime;
+    int32_t *tscore, *tticks;
+    DoneRule rule;
+    int obsDim, stateDim, invert, normalize, prev, tickCount;
+    int obsBlocks, stateBlocks;       // workgroups of each kind of rows
+};
+
+DI void packMatchRow(const Dev& d, const LivePack& p, int s)
 {
-    const int i0 = blockIdx.x * packChunkRows(stateDimV), n = *count;
-    if (i0 >= n) return;
-    packRowsGathered(
-        out, stateDimV, i0, min(i0 + packChunkRows(stateDimV), n), [&](int i) { return list[i]; },
-        [&](int s, int q, float* o) { packStatePart(d, s, touchWindow, tickCount, q, o); });
+    const MatchWords m = matchWords(d, s);
+    if (p.score) {
+        p.score[s] = m.blue - m.orange;
+        p.ticks[s] = m.ep;
+        p.overtime[s] = m.overtime != 0;
+    }
+    if (p.rewards) {
+        p.rewards[s] = (float)m.scorer;
+        p.dones[s] = simDoneFrom(m, p.tickCount, p.rule);
+        p.tscore[s] = m.blue - m.orange;
+        p.tticks[s] = m.ep;
+        p.tovertime[s] = m.overtime != 0;
+    }
 }
 
-// The observation rows of the cars of the simulations list[0..*count).
-__global__ __launch_bounds__(kPackBlock) void obsListKernel(Dev d, float* out, int obsDimV, int invert,
-                                                           int normalizeObs, int prev, const int* list,
-                                                           const int* count)
+// of every simulation
+__global__ __launch_bounds__(kPackBlock) void packLiveKernel(Dev d, LivePack p)
 {
-    const int i0 = blockIdx.x * packChunkRows(obsDimV), n = *count * d.nCars;
-    if (i0 >= n) return;
-    packRowsGathered(
-        out, obsDimV, i0, min(i0 + packChunkRows(obsDimV), n),
-        [&](int i) { return list[i / d.nCars] * d.nCars + i % d.nCars; },
-        [&](int a, int q, float* o) {
-            packObservationPart(d, a / d.nCars, a % d.nCars, invert != 0, normalizeObs != 0, prev != 0, q, o);
-        });
+    int b = blockIdx.x;
+    if (b < p.obsBlocks) {
+        const int r0 = b * packChunkRows(p.obsDim);
+        packRowsParts(
+            p.obs, p.obsDim, r0, min(r0 + packChunkRows(p.obsDim), d.nTotal), [](int) { return true; },
+            [&](int a, int q, float* o) {
+                packObservationPart(d, a / d.nCars, a % d.nCars, p.invert != 0, p.normalize != 0, p.prev != 0, q, o);
+            });
+        return;
+    }
+    b -= p.obsBlocks;
+    const int stateKinds = p.tstate ? 2 : 1;
+    if (b < stateKinds * p.stateBlocks) {
+        const bool live = b < p.stateBlocks;
+        const int r0 = (live ? b : b - p.stateBlocks) * packChunkRows(p.stateDim);
+        packRowsParts(
+            live ? p.state : p.tstate, p.stateDim, r0, min(r0 + packChunkRows(p.stateDim), d.nSim),
+            [](int) { return true; }, [&](int s, int q, float* o) { packStatePart(d, s, 1, p.tickCount, q, o); });
+        return;
+    }
+    const int s = (b - stateKinds * p.stateBlocks) * kPackBlock + threadIdx.x;
+    if (s < d.nSim) packMatchRow(d, p, s);
+}
+
+// of the simulations list[0..*count): the workgroups of a kind stride over its rows
+__global__ __launch_bounds__(kPackBlock) void packListKernel(Dev d, LivePack p, const int* list, const int* count)
+{
+    const int n = *count;
+    int b = blockIdx.x;
+    if (b < p.obsBlocks) {
+        const int chunk = packChunkRows(p.obsDim);
+        for (int i0 = b * chunk; i0 < n * d.nCars; i0 += p.obsBlocks * chunk)
+            packRowsGathered(
+                p.obs, p.obsDim, i0, min(i0 + chunk, n * d.nCars),
+                [&](int i) { return list[i / d.nCars] * d.nCars + i % d.nCars; },
+                [&](int a, int q, float* o) {
+                    packObservationPart(d, a / d.nCars, a % d.nCars, p.invert != 0, p.normalize != 0, p.prev != 0, q, o);
+                });
+        return;
+    }
+    b -= p.obsBlocks;
+    if (b < p.stateBlocks) {
+        const int chunk = packChunkRows(p.stateDim);
+        for (int i0 = b * chunk; i0 < n; i0 += p.stateBlocks * chunk)
+            packRowsGathered(
+                p.state, p.stateDim, i0, min(i0 + chunk, n), [&](int i) { return list[i]; },
+                [&](int s, int q, float* o) { packStatePart(d, s, 1, p.tickCount, q, o); });
+        return;
+    }
+    const int i = (b - p.stateBlocks) * kPackBlock + threadIdx.x;
+    if (i < n) packMatchRow(d, p, list[i]);
 }
 
 // Everything an env step does after its ticks, for `sims` simulations per
@@ -1414,6 +1484,7 @@ __global__ __launch_bounds__(kVectorBlock) void vectorOutputsKernel(Dev d, const
 // and repacking touch that row's simulation only.
 __global__ void clearCountKernel(int* count) { *count = 0; }
 
+constexpr int kSetBlock = 256;
 constexpr int kCompactBlock = 256;
 constexpr int kCompactRows = 16;
 __global__ __launch_bounds__(kCompactBlock) void compactMaskKernel(const uint8_t* __restrict__ mask, int n,
@@ -1446,29 +1517,58 @@ __global__ __launch_bounds__(kCompactBlock) void compactMaskKernel(const uint8_t
         if (bits & (1u << k)) list[at++] = r0 + k;
 }
 
-__global__ void setBallKernel(Dev d, const float* pos, const float* vel, const float* ang, Selection sel)
+// What a restore sets of its simulations (null: not given) and of their cars.
+struct SimInput {
+    const float *pos, *vel, *ang;                    // the ball
+    const int32_t *blue, *orange, *ticks;            // the match
+    bool pads;                                       // every pad available
+};
+struct CarInput {
+    const float *pos, *rot, *vel, *ang;
+    const void* demoed;
+    int byteDemoed;
+    const float *boost, *internal;
+};
+
+DI void setSimRow(const Dev& d, const SimInput& in, int r, int t)
 {
-    const int r = selectedInput(sel, blockIdx.x * blockDim.x + threadIdx.x);
-    if (r < 0) return;
-    const int t = selectRow(sel, r, d.nSim);
-    if (t < 0) return;
-    d.ssetv(CARL_SIM_BALL_POS, t, V3{ pos[3 * r], pos[3 * r + 1], pos[3 * r + 2] });
-    d.ssetv(CARL_SIM_BALL_VEL, t, V3{ vel[3 * r], vel[3 * r + 1], vel[3 * r + 2] });
-    d.ssetv(CARL_SIM_BALL_ANG, t, V3{ ang[3 * r], ang[3 * r + 1], ang[3 * r + 2] });
-    d.ssetv(CARL_SIM_BALL_IMP, t, kZero);
+    if (in.pads)
+        for (int p = 0; p < kPads; p++) d.ssetf(CARL_SIM_PAD_COOLDOWN + p, t, 0.f);
+    if (in.pos) {
+        d.ssetv(CARL_SIM_BALL_POS, t, V3{ in.pos[3 * r], in.pos[3 * r + 1], in.pos[3 * r + 2] });
+        d.ssetv(CARL_SIM_BALL_VEL, t, V3{ in.vel[3 * r], in.vel[3 * r + 1], in.vel[3 * r + 2] });
+        d.ssetv(CARL_SIM_BALL_ANG, t, V3{ in.ang[3 * r], in.ang[3 * r + 1], in.ang[3 * r + 2] });
+        d.ssetv(CARL_SIM_BALL_IMP, t, kZero);
+    }
+    if (in.blue) {
+        d.sseti(CARL_SIM_BLUE_SCORE, t, in.blue[r]);
+        d.sseti(CARL_SIM_ORANGE_SCORE, t, in.orange[r]);
+        d.sseti(CARL_SIM_LAST_SCORER, t, 0);
+        d.sseti(CARL_SIM_OVERTIME, t, 0);
+        d.sseti(CARL_SIM_EPISODE_TICKS, t, in.ticks[r]);
+    }
 }
 
-__global__ void setCarKernel(Dev d, const float* pos, const float* rot, const float* vel, const float* ang,
-                             const void* demoed, int byteDemoed, const float* boost, const float* internal,
-                             Selection sel)
+// The rows of a selection: the first carBlocks workgroups one car per thread
+// (none of them without cars to set), the others one simulation per thread.
+// The two write disjoint words.  Bound by its partly written lines: a quarter
+// of 131,072 2v2 simulations 32-38 us (cars, balls and pads apart 36 in three
+// launches), half of 65,536 1v1 14 (21).
+__global__ __launch_bounds__(kSetBlock) void setRowsKernel(Dev d, SimInput sim, CarInput car, Selection sel, int carBlocks)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int r = selectedInput(sel, i / d.nCars);
+    const bool cars = (int)blockIdx.x < carBlocks;
+    const int i = ((int)blockIdx.x - (cars ? 0 : carBlocks)) * kSetBlock + threadIdx.x;
+    const int r = selectedInput(sel, cars ? i / d.nCars : i);
     if (r < 0) return;
     const int t = selectRow(sel, r, d.nSim);
     if (t < 0) return;
-    const int local = i % d.nCars;
-    setCarRow(d, r * d.nCars + local, t, local, pos, rot, vel, ang, demoed, byteDemoed != 0, boost, internal);
+    if (cars) {
+        const int local = i % d.nCars;
+        setCarRow(d, r * d.nCars + local, t, local, car.pos, car.rot, car.vel, car.ang, car.demoed, car.byteDemoed != 0,
+                  car.boost, car.internal);
+    } else {
+        setSimRow(d, sim, r, t);
+    }
 }
 
 // Wheel contacts of the selected cars against the restored scene (rays only,
@@ -1510,28 +1610,6 @@ __global__ __launch_bounds__(kContactBlock) void refreshKernel(Dev d, Selection 
     Wheels w;
     (void)contactFinish(d, L, lane, car, car / d.nCars, cen, rot, w);
     storeRefreshedWheels(d, car, w);
-}
-
-__global__ void setMatchKernel(Dev d, const int32_t* blue, const int32_t* orange, const int32_t* ticks, Selection sel)
-{
-    const int r = selectedInput(sel, blockIdx.x * blockDim.x + threadIdx.x);
-    if (r < 0) return;
-    const int t = selectRow(sel, r, d.nSim);
-    if (t < 0) return;
-    d.sseti(CARL_SIM_BLUE_SCORE, t, blue[r]);
-    d.sseti(CARL_SIM_ORANGE_SCORE, t, orange[r]);
-    d.sseti(CARL_SIM_LAST_SCORER, t, 0);
-    d.sseti(CARL_SIM_OVERTIME, t, 0);
-    d.sseti(CARL_SIM_EPISODE_TICKS, t, ticks[r]);
-}
-
-__global__ void resetPadsKernel(Dev d, Selection sel)
-{
-    const int r = selectedInput(sel, blockIdx.x * blockDim.x + threadIdx.x);
-    if (r < 0) return;
-    const int t = selectRow(sel, r, d.nSim);
-    if (t < 0) return;
-    for (int p = 0; p < kPads; p++) d.ssetf(CARL_SIM_PAD_COOLDOWN + p, t, 0.f);
 }
 
 // ---- exclusive scan (no library): per-tile wave64 DPP scans, tile totals
@@ -2201,24 +2279,57 @@ int packState(carl_env* e, float* out, int touchWindow, const bool* mask)
 
 int packMatch(carl_env* e, const bool* mask)
 {
-    matchKernel<<<e->grid(e->nSim, 64), 64, 0, e->stream>>>(e->dev(), e->score, e->ticks, e->overtime, mask,
-                                                             nullptr, nullptr);
+    matchKernel<<<e->grid(e->nSim, 64), 64, 0, e->stream>>>(e->dev(), e->score, e->ticks, e->overtime, mask);
+    HIP_TRY(hipGetLastError());
+    return CARL_OK;
+}
+
+// What a call packs after it changed the live state: bits of packLive.
+enum { kPackMatch = 1, kPackTransitionState = 2, kPackRewards = 4 };
+
+LivePack livePack(const carl_env* e, int what)
+{
+    LivePack p{};
+    p.obs = e->obs;
+    p.state = e->state;
+    if (what & kPackTransitionState) p.tstate = e->tstate;
+    if (what & kPackMatch) { p.score = e->score; p.ticks = e->ticks; p.overtime = e->overtime; }
+    if (what & kPackRewards) {
+        p.rewards = e->rewards; p.dones = e->dones; p.tovertime = e->tovertime;
+        p.tscore = e->tscore; p.tticks = e->tticks;
+        p.rule = e->rule();
+    }
+    p.obsDim = e->obsDim; p.stateDim = e->stateDim;
+    p.invert = e->invert; p.normalize = e->normalize; p.prev = e->prevControls;
+    p.tickCount = e->tickCount;
+    p.obsBlocks = e->grid(e->nTotal, packChunkRows(e->obsDim));
+    p.stateBlocks = e->grid(e->nSim, packChunkRows(e->stateDim));
+    return p;
+}
+
+// the observations and the state of every simulation, and `what` beside them
+int packLive(carl_env* e, int what)
+{
+    const LivePack p = livePack(e, what);
+    const int states = p.stateBlocks * (p.tstate ? 2 : 1), match = p.score || p.rewards ? e->grid(e->nSim, kPackBlock) : 0;
+    packLiveKernel<<<p.obsBlocks + states + match, kPackBlock, stepLdsBytes(e->obsDim, e->stateDim), e->stream>>>(e->dev(), p);
     HIP_TRY(hipGetLastError());
     return CARL_OK;
 }
 
 // The outputs a reset changes (observations, state, match state) for the
-// simulations of a compacted selection.
+// simulations of a compacted selection, whose count only the device knows.
+// At most four workgroups of each kind per slot are launched, and stride:
+// those beyond the selection do nothing but start (of 2v2 at 131,072
+// simulations, a quarter selected, 8,200 of 10,900).
 int packSelected(carl_env* e, const Selection& sel)
 {
-    obsListKernel<<<e->grid(e->nTotal, packChunkRows(e->obsDim)), kPackBlock, packLdsBytes(e->obsDim), e->stream>>>(
-        e->dev(), e->obs, e->obsDim, e->invert, e->normalize, e->prevControls, sel.list, sel.count);
-    HIP_TRY(hipGetLastError());
-    stateListKernel<<<e->grid(e->nSim, packChunkRows(e->stateDim)), kPackBlock, packLdsBytes(e->stateDim),
-                      e->stream>>>(e->dev(), e->state, e->stateDim, 1, e->tickCount, sel.list, sel.count);
-    HIP_TRY(hipGetLastError());
-    matchKernel<<<e->grid(e->nSim, 64), 64, 0, e->stream>>>(e->dev(), e->score, e->ticks, e->overtime, nullptr,
-                                                             sel.list, sel.count);
+    LivePack p = livePack(e, kPackMatch);
+    const int most = 4 * std::max(1, e->stepResident);
+    p.obsBlocks = std::min(p.obsBlocks, most);
+    p.stateBlocks = std::min(p.stateBlocks, most);
+    packListKernel<<<p.obsBlocks + p.stateBlocks + e->grid(e->nSim, kPackBlock), kPackBlock,
+                     stepLdsBytes(e->obsDim, e->stateDim), e->stream>>>(e->dev(), p, sel.list, sel.count);
     HIP_TRY(hipGetLastError());
     return CARL_OK;
 }
@@ -2231,59 +2342,31 @@ int packRewardsDones(carl_env* e)
     return CARL_OK;
 }
 
-int initialPacks(carl_env* e)
-{
-    CARL_TRY(packObs(e, e->obs, nullptr));
-    CARL_TRY(packState(e, e->state, 1, nullptr));
-    CARL_TRY(packState(e, e->tstate, 1, nullptr));
-    CARL_TRY(packRewardsDones(e));
-    CARL_TRY(packMatch(e, nullptr));
-    return CARL_OK;
-}
+int initialPacks(carl_env* e) { return packLive(e, kPackMatch | kPackTransitionState | kPackRewards); }
 
 int fullReset(carl_env* e)
 {
     e->tickCount = 0;
-    resetKernel<<<e->grid(e->nSim, 64), 64, 0, e->stream>>>(e->dev(), e->nOrange);
+    const int carBlocks = e->grid(e->nTotal, kTickBlock);
+    resetKernel<<<carBlocks + e->grid(e->nSim, kTickBlock), kTickBlock, 0, e->stream>>>(e->dev(), carBlocks);
     HIP_TRY(hipGetLastError());
     return initialPacks(e);
 }
 
 Selection makeSel(const int64_t* idx, const uint8_t* mask, int n) { return Selection{ idx, mask, n, nullptr, nullptr }; }
 
-int setBallRows(carl_env* e, const float* pos, const float* vel, const float* ang, Selection sel)
+// The selection's simulations and (with car.pos) cars, and those cars' wheel
+// contacts in the scene that leaves.
+int setRows(carl_env* e, const SimInput& sim, const CarInput& car, Selection sel)
 {
     if (sel.n == 0) return CARL_OK;
-    setBallKernel<<<e->grid(sel.n, 64), 64, 0, e->stream>>>(e->dev(), pos, vel, ang, sel);
+    const bool sims = sim.pads || sim.pos || sim.blue;
+    const int cars = car.pos ? sel.n * e->nCars : 0, carBlocks = e->grid(cars, kSetBlock);
+    setRowsKernel<<<carBlocks + (sims ? e->grid(sel.n, kSetBlock) : 0), kSetBlock, 0, e->stream>>>(e->dev(), sim, car, sel,
+                                                                                                 carBlocks);
     HIP_TRY(hipGetLastError());
-    return CARL_OK;
-}
-
-int setCarRows(carl_env* e, const float* pos, const float* rot, const float* vel, const float* ang, const void* demoed,
-               int byteDemoed, const float* boost, const float* internal, Selection sel)
-{
-    if (sel.n == 0) return CARL_OK;
-    const int n = sel.n * e->nCars;
-    setCarKernel<<<e->grid(n, 256), 256, 0, e->stream>>>(e->dev(), pos, rot, vel, ang, demoed, byteDemoed, boost,
-                                                          internal, sel);
-    HIP_TRY(hipGetLastError());
-    refreshKernel<<<e->grid(n, kContactOwners), kContactBlock, 0, e->stream>>>(e->dev(), sel, e->contactScreen);
-    HIP_TRY(hipGetLastError());
-    return CARL_OK;
-}
-
-int setMatchRows(carl_env* e, const int32_t* blue, const int32_t* orange, const int32_t* ticks, Selection sel)
-{
-    if (sel.n == 0) return CARL_OK;
-    setMatchKernel<<<e->grid(sel.n, 64), 64, 0, e->stream>>>(e->dev(), blue, orange, ticks, sel);
-    HIP_TRY(hipGetLastError());
-    return CARL_OK;
-}
-
-int resetPadRows(carl_env* e, Selection sel)
-{
-    if (sel.n == 0) return CARL_OK;
-    resetPadsKernel<<<e->grid(sel.n, 64), 64, 0, e->stream>>>(e->dev(), sel);
+    if (cars == 0) return CARL_OK;
+    refreshKernel<<<e->grid(cars, kContactOwners), kContactBlock, 0, e->stream>>>(e->dev(), sel, e->contactScreen);
     HIP_TRY(hipGetLastError());
     return CARL_OK;
 }
@@ -2497,11 +2580,10 @@ int carl_env_set_ball(carl_env* e, const float* pos, const float* vel, const flo
     if (!idx) n = e->nSim;
     CARL_TRY(checkSelection(e, n));
     if (n > 0 && (!pos || !vel || !ang)) return fail(CARL_ERR_VALUE, "null ball input");
-    CARL_TRY(setBallRows(e, pos, vel, ang, makeSel(idx, nullptr, n)));
-    CARL_TRY(packObs(e, e->obs, nullptr));
-    CARL_TRY(packState(e, e->state, 1, nullptr));
-    CARL_TRY(packState(e, e->tstate, 1, nullptr));
-    return CARL_OK;
+    SimInput in{};
+    in.pos = pos; in.vel = vel; in.ang = ang;
+    CARL_TRY(setRows(e, in, CarInput{}, makeSel(idx, nullptr, n)));
+    return packLive(e, kPackTransitionState);
 }
 
 int carl_env_set_car(carl_env* e, const float* pos, const float* rot, const float* vel, const float* ang,
@@ -2512,11 +2594,9 @@ int carl_env_set_car(carl_env* e, const float* pos, const float* rot, const floa
     if (!idx) n = e->nSim;
     CARL_TRY(checkSelection(e, n));
     if (n > 0 && (!pos || !rot || !vel || !ang || !demoed)) return fail(CARL_ERR_VALUE, "null car input");
-    CARL_TRY(setCarRows(e, pos, rot, vel, ang, demoed, byteDemoed, boost, internal, makeSel(idx, nullptr, n)));
-    CARL_TRY(packObs(e, e->obs, nullptr));
-    CARL_TRY(packState(e, e->state, 1, nullptr));
-    CARL_TRY(packState(e, e->tstate, 1, nullptr));
-    return CARL_OK;
+    CARL_TRY(setRows(e, SimInput{}, CarInput{ pos, rot, vel, ang, demoed, byteDemoed, boost, internal },
+                     makeSel(idx, nullptr, n)));
+    return packLive(e, kPackTransitionState);
 }
 
 int carl_env_apply_reset(carl_env* e, const float* bpos, const float* bvel, const float* bang, const float* cpos,
@@ -2545,15 +2625,9 @@ int carl_env_apply_reset(carl_env* e, const float* bpos, const float* bvel, cons
             mask, n, e->rowList, e->rowList + e->nSim);
         HIP_TRY(hipGetLastError());
     }
-    CARL_TRY(resetPadRows(e, sel));
-    CARL_TRY(setBallRows(e, bpos, bvel, bang, sel));
-    CARL_TRY(setCarRows(e, cpos, crot, cvel, cang, demoed, byteDemoed, boost, internal, sel));
-    if (hasMatch) CARL_TRY(setMatchRows(e, blue, orange, ticks, sel));
-    if (mask) return packSelected(e, sel);
-    CARL_TRY(packObs(e, e->obs, nullptr));
-    CARL_TRY(packState(e, e->state, 1, nullptr));
-    CARL_TRY(packMatch(e, nullptr));
-    return CARL_OK;
+    CARL_TRY(setRows(e, SimInput{ bpos, bvel, bang, blue, orange, ticks, true },
+                     CarInput{ cpos, crot, cvel, cang, demoed, byteDemoed, boost, internal }, sel));
+    return mask ? packSelected(e, sel) : packLive(e, kPackMatch);
 }
 
 int carl_env_set_match(carl_env* e, const int32_t* blue, const int32_t* orange, const int32_t* ticks,
@@ -2563,7 +2637,9 @@ int carl_env_set_match(carl_env* e, const int32_t* blue, const int32_t* orange, 
     if (!idx) n = e->nSim;
     CARL_TRY(checkSelection(e, n));
     if (n > 0 && (!blue || !orange || !ticks)) return fail(CARL_ERR_VALUE, "null match input");
-    return setMatchRows(e, blue, orange, ticks, makeSel(idx, nullptr, n));
+    SimInput in{};
+    in.blue = blue; in.orange = orange; in.ticks = ticks;
+    return setRows(e, in, CarInput{}, makeSel(idx, nullptr, n));
 }
 
 int carl_env_reset_pads(carl_env* e, const int64_t* idx, int n)
@@ -2571,7 +2647,9 @@ int carl_env_reset_pads(carl_env* e, const int64_t* idx, int n)
     CARL_TRY(checkEnv(e));
     if (!idx) n = e->nSim;
     CARL_TRY(checkSelection(e, n));
-    return resetPadRows(e, makeSel(idx, nullptr, n));
+    SimInput in{};
+    in.pads = true;
+    return setRows(e, in, CarInput{}, makeSel(idx, nullptr, n));
 }
 
 int carl_env_buffer(carl_env* e, int id, void** data, int64_t* shape, int* ndim, int* dtype)

@@ -304,13 +304,6 @@ DI void kickoffLocalCar(const Dev& d, int s, int local, int perm)
     kickoffCar(d, s * d.nCars + local, kickoffSpawn(perm, orange ? local - d.nBlue : local), orange);
 }
 
-DI void kickoffSim(const Dev& d, int s, int tickCount, int nOrange)
-{
-    const int perm = kickoffPerm(d, s, tickCount);
-    kickoffBall(d, s);
-    for (int k = 0; k < d.nBlue + nOrange; k++) kickoffLocalCar(d, s, k, perm);
-}
-
 DI void clearCarContacts(const Dev& d, int c)
 {
     d.setf(CARL_CAR_BRAKE_STAGE, c, 0.f);
@@ -323,33 +316,25 @@ DI void clearCarContacts(const Dev& d, int c)
     }
 }
 
-DI void fullResetSim(const Dev& d, int s, int nOrange)
+// A full reset's words of simulation s, and of its car `local`.
+DI void fullResetSimWords(const Dev& d, int s)
 {
     d.sseti(CARL_SIM_EPISODE_TICKS, s, 0);
     d.sseti(CARL_SIM_LAST_TOUCH_TICK, s, 0);
     d.ssetv(CARL_SIM_BALL_IMP, s, kZero);
-    d.sseti(CARL_SIM_BALL_INT_VALID, s, 0);
     for (int p = 0; p < kPads; p++) d.ssetf(CARL_SIM_PAD_COOLDOWN + p, s, 0.f);
     for (int f = CARL_SIM_BLUE_SCORE; f <= CARL_SIM_OVERTIME; f++) d.sseti(f, s, 0);
     d.sseti(CARL_SIM_BALL_ARENA_CONTACT_TICK, s, -1);
-    for (int k = 0; k < d.nCars; k++) {
-        const int c = s * d.nCars + k;
-        d.setv(CARL_CAR_IMP, c, kZero);
-        d.seti(CARL_CAR_DEMOED, c, 0);
-        d.setf(CARL_CAR_DEMO_TIMER, c, 0.f);
-        d.seti(CARL_CAR_CONTACT_IDX, c, -1);
-        d.setf(CARL_CAR_CONTACT_COOLDOWN, c, 0.f);
-        d.seti(CARL_CAR_BALL_HIT_TICK, c, -1);
-        d.seti(CARL_CAR_BALL_CONTACT_TICK, c, -1);
-        for (int w = 0; w < kWheels; w++) {
-            d.seti(CARL_CAR_WHEEL_SOURCE + w, c, kSrcNone);
-            d.seti(CARL_CAR_WHEEL_CONTACT + w, c, 0);
-        }
-        d.seti(CARL_CAR_ARENA_CONTACT_TICK, c, -1);
-        resetInternal(d, c);
-        clearCarContacts(d, c);
-    }
-    kickoffSim(d, s, 0, nOrange);
+    kickoffBall(d, s);
+}
+
+DI void fullResetCar(const Dev& d, int s, int local)
+{
+    const int c = s * d.nCars + local;
+    for (int w = 0; w < kWheels; w++) d.seti(CARL_CAR_WHEEL_SOURCE + w, c, kSrcNone);
+    d.seti(CARL_CAR_ARENA_CONTACT_TICK, c, -1);
+    clearCarContacts(d, c);
+    kickoffLocalCar(d, s, local, kickoffPerm(d, s, 0));
 }
 
 // What the end-of-step reset does to one simulation: nothing, enter
