@@ -502,15 +502,10 @@ __global__ __launch_bounds__(kTickBlock) void finishKernel(Dev d, int simsPerBlo
     if (simOk) boostPads(d, laneSim);
 }
 
-// The whole tick window in one launch: a block owns simulations
-// [begin + blockIdx.x * simsPerBlock, +simsPerBlock) and runs every phase of
-// every tick on them, with block barriers between the phases.  Simulations
-// share nothing but the read-only arena, so no other block is ever waited
-// for: a slow wave holds up its own block, not a grid-wide kernel boundary.
-// Two-wave blocks (four per CU) wait less at the phase barriers than
-// four-wave blocks at the same occupancy (measured +1.7% per step), and
-// measured 1-3% faster than one-wave blocks of 32 simulations, whose
-// barriers cost nothing.
+// The whole tick window in one launch.  Simulations share nothing but the
+// read-only arena, so no wave ever waits for another: a slow one holds up
+// itself, not a workgroup or a grid-wide kernel boundary.  Workgroups of two
+// waves, four per CU.
 #ifndef CARL_WINDOW_BLOCK
 #define CARL_WINDOW_BLOCK 128
 #endif
@@ -537,9 +532,10 @@ constexpr int kWindowContactOwners = CARL_WINDOW_CONTACT_OWNERS;
 // by its ball gather (the phases of one wave never overlap, and no wave
 // touches another wave's area).  With a whole wave of
 // contact owners that is 19.7 KB per wave, 39.4 KB per workgroup: four
-// workgroups per CU, the occupancy the 256-VGPR budget allows.  The phases are
-// still separated by workgroup barriers: a phase reads state words other
-// threads of the workgroup wrote in the phase before.
+// workgroups per CU, the occupancy the 256-VGPR budget allows.  Wave-level
+// fences separate the phases: every state word a phase reads was written by
+// its own wave.  (tickWindowBlockKernel, whose waves share phases, has
+// workgroup barriers there.)
 union WaveLds {
     ContactLdsT<kWindowContactOwners> contact;
     struct {
@@ -1928,7 +1924,7 @@ struct carl_env {
     hipEvent_t fork = nullptr, join[kMaxTickStreams - 1] = {};
     int windowSims = kDefaultWindowSims;  // simulations per block of the tick-window kernel (0: phase kernels)
     // Until the caller sets windowSims, a run too small to fill the device's
-    // resident window workgroups uses smaller ones (effectiveWindowSims): the
+    // resident window workgroups uses smaller ones (windowShape): the
     // kernel's time is one workgroup's latency chain, so spreading the
     // simulations over more compute units shortens it.
     bool windowAuto = true;
