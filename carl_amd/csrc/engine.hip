@@ -821,7 +821,8 @@ DI void tickWindowBody(const Dev& d0, int screen, int kind, const void* __restri
     }
     if (map.outCount && lane < map.rounds && m.unit[lane] >= 0) {
         const int u = m.unit[lane], l = group * kDealLists + dealClass(m.cost[lane]) * kDealSubs + u % kDealSubs;
-        map.outList[(size_t)l * map.listLen + atomicAdd(&map.outCount[l], 1)] = u;
+        const int at = atomicAdd(&map.outCount[l], 1);
+        if (at < map.listLen) map.outList[(size_t)l * map.listLen + at] = u;
     }
     if (prof && lane == 0) {
         for (int st = 0; st < kWindowStages; st++) atomicAdd(&prof[kProfStages + st], m.stage[st]);
@@ -1909,12 +1910,13 @@ struct carl_env {
     uint32_t* ws = nullptr;  // per-tick car workspace (kWsPlanes planes)
     int* rowList = nullptr;  // a masked reset's selected rows (n_sim), then their count
     // the deal of window launches, kDealSets sets of class counts and lists
-    // (dealRoom words each), the dealt launches so far and the units and
-    // groups they dealt in (a launch that deals in others starts over)
+    // (dealRoom words each), the dealt launches so far and the units, groups
+    // and workgroups they dealt to (these set which units a group holds and
+    // where its lists lie: a launch with others starts over)
     int* dealCount = nullptr;
     int* dealList = nullptr;
     size_t dealRoom = 0;      // words of one set of lists
-    int dealUnitSims = 0, dealGroups = 0;
+    int dealUnitSims = 0, dealGroups = 0, dealBlocks = 0;
     long long dealLaunches = 0;
     int balance = 1;                     // deal window launches by cost
     float* ballScratch = nullptr;    // with it: kNativeMaxContacts slots of kNativeSlotWords per simulation
@@ -2195,12 +2197,13 @@ int launchTicks(carl_env* e, int kind, const void* actions, int n)
             map.listLen = w.listLen;
             map.groups = w.groups;
             if (w.dealt) {
-                if (e->dealUnitSims != w.unitSims || e->dealGroups != w.groups) {
+                if (e->dealUnitSims != w.unitSims || e->dealGroups != w.groups || e->dealBlocks != w.blocks) {
                     // lists of other units (or none): the first launch of
                     // these deals the identity and files into cleared counts
                     clearDealKernel<<<kDealSets * kXcds, kDealLists, 0, stream[p]>>>(e->dealCount);
                     e->dealUnitSims = w.unitSims;
                     e->dealGroups = w.groups;
+                    e->dealBlocks = w.blocks;
                     e->dealLaunches = 0;
                 }
                 const long long l = e->dealLaunches++;
