@@ -16,6 +16,7 @@
 #include <initializer_list>
 #include <optional>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/carl_amd.h"
@@ -149,6 +150,76 @@ const int64_t* selectionPointer(const TensorView& sel)
     return p ? p : &kNoIndex;
 }
 
+void validate(const DLTensor& t, const std::string& name, std::initializer_list<int64_t> shape, uint8_t code,
+              uint8_t bits)
+{
+    if (t.dtype.code != code || t.dtype.bits != bits || t.dtype.lanes != 1)
+        throw py::type_error(name + " has an invalid dtype");
+    if (t.device.device_type != kDLROCM || t.device.device_id != 0)
+        throw py::value_error(name + " must be on cuda:0");
+    if (t.ndim != (int32_t)shape.size()) throw py::value_error(name + " has an invalid shape");
+    int dim = 0;
+    for (int64_t want : shape)
+        if (t.shape[dim++] != want) throw py::value_error(name + " has an invalid shape");
+    if (t.strides) {
+        int64_t stride = 1;
+        for (int i = t.ndim - 1; i >= 0; i--) {
+            if (t.shape[i] > 1 && t.strides[i] != stride) throw py::value_error(name + " must be contiguous");
+            stride *= t.shape[i];
+        }
+    }
+}
+
+// The arrays of a vector step's outputs, in carl_vector_io's order: every one
+// is checked like an input before the kernel may write through its address
+// (torch's default dtype decides what an allocation without one holds).  None
+// or a null address where an array is left out.
+struct VectorArrays {
+    static constexpr int kCount = 14;
+    carl_vector_io io{};
+
+    VectorArrays(int nSim, int nCars, int obsDim, const py::args& arrays)
+    {
+        if (arrays.size() != kCount) throw py::type_error("14 vector outputs expected");
+        const int64_t agents = (int64_t)nSim * nCars;
+        auto given = [&](int i) {
+            const py::object o = arrays[i];
+            return !o.is_none() && !(py::isinstance<py::int_>(o) && o.equal(py::int_(0)));
+        };
+        for (int i = 0; i < 10; i++)
+            if (!given(i)) throw py::value_error("null vector output");
+        if (given(10) != given(11) || given(10) != given(12))
+            throw py::value_error("step_returns, step_lengths and step_done must be given together");
+        auto take = [&](auto*& out, int i, const char* name, std::initializer_list<int64_t> shape, uint8_t code, uint8_t bits) {
+            if (!given(i)) return;
+            const py::object o = arrays[i];
+            keep_[i] = py::isinstance<py::capsule>(o) ? o : o.attr("__dlpack__")(py::arg("stream") = -1);
+            const auto* m = keep_[i].cast<py::capsule>().get_pointer<DLManagedTensor>();
+            if (!m) throw py::value_error("invalid DLPack tensor");
+            validate(m->dl_tensor, name, shape, code, bits);
+            out = reinterpret_cast<std::remove_reference_t<decltype(out)>>(static_cast<char*>(m->dl_tensor.data)
+                                                                          + m->dl_tensor.byte_offset);
+        };
+        take(io.obs, 0, "obs", { agents, obsDim }, kDLFloat, 32);
+        take(io.reward, 1, "reward", { agents }, kDLFloat, 32);
+        take(io.terminated, 2, "terminated", { agents }, kDLBool, 8);
+        take(io.truncated, 3, "truncated", { agents }, kDLBool, 8);
+        take(io.done, 4, "done", { agents }, kDLBool, 8);
+        take(io.returns, 5, "returns", { agents }, kDLFloat, 32);
+        take(io.lengths, 6, "lengths", { agents }, kDLInt, 64);
+        take(io.score_difference, 7, "score_difference", { nSim }, kDLInt, 32);
+        take(io.episode_ticks, 8, "episode_ticks", { nSim }, kDLInt, 32);
+        take(io.overtime, 9, "overtime", { nSim }, kDLBool, 8);
+        take(io.step_returns, 10, "step_returns", { agents }, kDLFloat, 32);
+        take(io.step_lengths, 11, "step_lengths", { agents }, kDLInt, 64);
+        take(io.step_done, 12, "step_done", { agents }, kDLBool, 8);
+        take(io.ended, 13, "ended", { 4 * (agents + 1) }, kDLInt, 32);
+    }
+
+private:
+    py::object keep_[kCount];   // what the addresses lie in, for the call
+};
+
 struct PendingInput {
     std::vector<py::object> inputs;
     hipEvent_t done = nullptr;
@@ -179,26 +250,6 @@ class Env {
             if (s == hipErrorNotReady) return;
             if (s != hipSuccess) throw std::runtime_error(hipGetErrorString(s));
             pending_.pop_front();
-        }
-    }
-
-    static void validate(const DLTensor& t, const std::string& name, std::initializer_list<int64_t> shape, uint8_t code,
-                         uint8_t bits)
-    {
-        if (t.dtype.code != code || t.dtype.bits != bits || t.dtype.lanes != 1)
-            throw py::type_error(name + " has an invalid dtype");
-        if (t.device.device_type != kDLROCM || t.device.device_id != 0)
-            throw py::value_error(name + " must be on cuda:0");
-        if (t.ndim != (int32_t)shape.size()) throw py::value_error(name + " has an invalid shape");
-        int dim = 0;
-        for (int64_t want : shape)
-            if (t.shape[dim++] != want) throw py::value_error(name + " has an invalid shape");
-        if (t.strides) {
-            int64_t stride = 1;
-            for (int i = t.ndim - 1; i >= 0; i--) {
-                if (t.shape[i] > 1 && t.strides[i] != stride) throw py::value_error(name + " must be contiguous");
-                stride *= t.shape[i];
-            }
         }
     }
 
@@ -518,29 +569,11 @@ public:
     }
 
     // What CARLTorchVectorEnv.step returns of the last step, into arrays that
-    // its caller has allocated (device addresses, sizes as carl_vector_io
-    // states; 0 for the optional ones).
-    void vectorOutputs(uintptr_t obs, uintptr_t reward, uintptr_t terminated, uintptr_t truncated, uintptr_t done,
-                       uintptr_t returns, uintptr_t lengths, uintptr_t scoreDifference, uintptr_t episodeTicks,
-                       uintptr_t overtime, uintptr_t stepReturns, uintptr_t stepLengths, uintptr_t stepDone,
-                       uintptr_t ended)
+    // its caller has allocated and ordered after its own stream (VectorArrays).
+    void vectorOutputs(const py::args& arrays)
     {
-        carl_vector_io io{};
-        io.obs = reinterpret_cast<float*>(obs);
-        io.reward = reinterpret_cast<float*>(reward);
-        io.terminated = reinterpret_cast<uint8_t*>(terminated);
-        io.truncated = reinterpret_cast<uint8_t*>(truncated);
-        io.done = reinterpret_cast<uint8_t*>(done);
-        io.returns = reinterpret_cast<float*>(returns);
-        io.lengths = reinterpret_cast<int64_t*>(lengths);
-        io.score_difference = reinterpret_cast<int32_t*>(scoreDifference);
-        io.episode_ticks = reinterpret_cast<int32_t*>(episodeTicks);
-        io.overtime = reinterpret_cast<uint8_t*>(overtime);
-        io.step_returns = reinterpret_cast<float*>(stepReturns);
-        io.step_lengths = reinterpret_cast<int64_t*>(stepLengths);
-        io.step_done = reinterpret_cast<uint8_t*>(stepDone);
-        io.ended = reinterpret_cast<int32_t*>(ended);
-        check(carl_env_vector_outputs(env_, &io));
+        const VectorArrays v(nSim_, nCars_, param(CARL_PARAM_OBS_DIM), arrays);
+        check(carl_env_vector_outputs(env_, &v.io));
     }
 
     void resetDones() { check(carl_env_reset_dones(env_)); }
@@ -736,6 +769,10 @@ PYBIND11_MODULE(_carl, m)
         .def("reset_dones", &Env::resetDones)
         .def("synchronize", &Env::synchronize)
         .def("_vector_outputs", &Env::vectorOutputs)
+        .def_static(
+            "_check_vector_outputs",
+            [](int nSim, int nCars, int obsDim, const py::args& arrays) { VectorArrays(nSim, nCars, obsDim, arrays); },
+            "The checks of _vector_outputs for an environment of these sizes, without one.")
         .def("enable_tick_timing", &Env::enableTiming, py::arg("enable") = true, py::arg("ticks") = true,
              py::arg("packing") = false, py::arg("stages") = false)
         .def("tick_timing", &Env::tickTiming)

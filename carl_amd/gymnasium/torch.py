@@ -26,6 +26,7 @@ from typing import Any, NamedTuple
 import numpy as np
 import torch as th
 import torch.nn.functional as F
+from torch.utils.dlpack import to_dlpack
 
 import carl_amd as carl
 
@@ -206,7 +207,8 @@ class _EpisodeLedger:
 
     def __init__(self, n_envs: int, device: th.device, deferred: bool):
         self.deferred = deferred
-        self.returns = th.zeros(n_envs, device=device)
+        # float32, or wider where the program's default is
+        self.returns = th.zeros(n_envs, dtype=th.promote_types(th.float32, th.get_default_dtype()), device=device)
         self.lengths = th.zeros(n_envs, dtype=th.int64, device=device)
         self.pending: list[tuple[th.Tensor, th.Tensor, th.Tensor]] = []
 
@@ -483,7 +485,9 @@ class CARLTorchVectorEnv(VectorEnv):
         if actions.shape != (self.n_envs, width):
             raise ValueError(f"Expected actions shaped {(self.n_envs, width)}")
         actions = actions.view(self.n_sim, self.n_cars, width)
-        if self._copy_outputs and not self.reward_funcs and self.reset_state_provider is None:
+        # (an environment made under a float64 default keeps float64 rewards and returns)
+        if (self._copy_outputs and not self.reward_funcs and self.reset_state_provider is None
+                and self._ledger.returns.dtype == th.float32):
             return self._step_native(actions)
 
         self._bridge.join()
@@ -527,25 +531,25 @@ class CARLTorchVectorEnv(VectorEnv):
         17 matches took 425 us, of 50,001 849 us; so 333 and 675 us)."""
         env, n, device = self._env, self.n_envs, self.device
         ledger, deferred = self._ledger, self.defer_episode_reporting
-        obs = th.empty((n, self._obs_dim), device=device)
-        reward = th.empty(n, device=device)
+        obs = th.empty((n, self._obs_dim), dtype=th.float32, device=device)
+        reward = th.empty(n, dtype=th.float32, device=device)
         terminated, truncated, done = (th.empty(n, dtype=th.bool, device=device) for _ in range(3))
         score = th.empty(self.n_sim, dtype=th.int32, device=device)
         ticks = th.empty(self.n_sim, dtype=th.int32, device=device)
         overtime = th.empty(self.n_sim, dtype=th.bool, device=device)
         if deferred:
             totals = (th.empty_like(ledger.returns), th.empty_like(ledger.lengths), th.empty_like(done))
-            report_to = (*(x.data_ptr() for x in totals), 0)
+            report_to = (*totals, None)
         else:
             ended = th.empty(4 * (n + 1), dtype=th.int32, device=device)
-            report_to = (0, 0, 0, ended.data_ptr())
+            report_to = (None, None, None, ended)
 
         self._bridge.join()
         try:
             (env.step if self.discrete_actions else env.step_continuous)(actions)
-            env._vector_outputs(obs.data_ptr(), reward.data_ptr(), terminated.data_ptr(), truncated.data_ptr(),
-                                done.data_ptr(), ledger.returns.data_ptr(), ledger.lengths.data_ptr(),
-                                score.data_ptr(), ticks.data_ptr(), overtime.data_ptr(), *report_to)
+            env._vector_outputs(*(x if x is None else to_dlpack(x) for x in (
+                obs, reward, terminated, truncated, done, ledger.returns, ledger.lengths, score, ticks, overtime,
+                *report_to)))
         finally:
             # no memory above goes back to torch's stream before the engine is done with it
             self._bridge.join()

@@ -5,6 +5,8 @@ immediate reports, side streams, and the sizes at which the report is read in
 two parts."""
 from __future__ import annotations
 
+from contextlib import contextmanager
+
 import numpy as np
 import pytest
 import torch
@@ -28,6 +30,66 @@ def team_reward(env):
 def actions(gen, env, discrete):
     u = torch.rand((env.n_envs, 7), generator=gen, device="cuda")
     return (u * torch.tensor([3, 3, 3, 2, 2, 3, 2], device="cuda")).int() if discrete else u * 2 - 1
+
+
+def place_balls(envs, gen):
+    """Balls beyond either goal line and in the field, the same in every
+    environment: a third of the matches ends with a goal for each team."""
+    n = envs[0].n_sim
+    third = torch.randperm(n, generator=gen, device="cuda") % 3
+    position = torch.zeros((n, 3), dtype=torch.float32, device="cuda")
+    position[:, 1] = (third == 1) * 5300.0 - (third == 2) * 5300.0
+    position[:, 2] = 100.0
+    still = torch.zeros_like(position)
+    for env in envs:
+        env.set_ball(position, still, still)
+
+
+@contextmanager
+def default_dtype(dtype):
+    before = torch.get_default_dtype()
+    torch.set_default_dtype(dtype)
+    try:
+        yield
+    finally:
+        torch.set_default_dtype(before)
+
+
+@pytest.mark.parametrize("deferred", [False, True])
+@pytest.mark.parametrize("made,stepped", [
+    (torch.float64, torch.float64), (torch.bfloat16, torch.bfloat16), (torch.float16, torch.float16),
+    (torch.float32, torch.float64), (torch.float32, torch.bfloat16), (torch.float64, torch.bfloat16),
+    (torch.bfloat16, torch.float64),
+])
+def test_steps_do_not_depend_on_the_default_dtype(made, stepped, deferred):
+    """A program's default dtype, set before the environment is made or
+    between its steps, changes no value.  The observations stay the engine's
+    float32; rewards are float32, or float64 where the environment was made
+    under that."""
+    want = make(33, 2, 1, False, deferred, 16)
+    with default_dtype(made):
+        ours = make(33, 2, 1, False, deferred, 16)
+        first = ours.reset()
+    torch.testing.assert_close(first, want.reset(), rtol=0, atol=0)
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    signs = set()
+    for step in range(12):
+        if step % 5 == 2:
+            place_balls((ours, want), gen)
+        a = actions(gen, want, False)
+        ref = want.step(a)
+        with default_dtype(stepped):
+            got = ours.step(a)
+        assert got[0].dtype == torch.float32 and got[1].dtype == torch.promote_types(torch.float32, made)
+        for g, w in zip(got[:4], ref[:4]):
+            torch.testing.assert_close(g.to(w.dtype), w, rtol=0, atol=0)
+        assert got[4].keys() == ref[4].keys()
+        if not deferred:
+            assert got[4]["reward"] == ref[4]["reward"] and got[4]["length"] == ref[4]["length"]
+        signs |= set(ref[1].tolist())
+    assert signs == {-1.0, 0.0, 1.0}
+    assert ours.drain_episode_reports() == want.drain_episode_reports()
+    torch.testing.assert_close(ours._ledger.returns.float(), want._ledger.returns, rtol=0, atol=0)
 
 
 # 1 agent; a row length and agent count of every remainder; more ended agents
