@@ -125,8 +125,9 @@ enum {
     CARL_PARAM_TICK_WINDOW = 13,   /* > 0: all ticks of a step in one launch per partition, this many
                                       simulations per workgroup of two waves (at most 128 cars; until it
                                       is set, the fewest with which the workgroups still fit the
-                                      GPU together); 0: four phase kernels per tick.  Results are identical; no reference
-                                      counterpart */
+                                      GPU together, and with native arena meshes the default halved,
+                                      down to 8, while they do); 0: four phase kernels per tick.
+                                      Results are identical; no reference counterpart */
     CARL_PARAM_NATIVE_ARENA = 14,  /* read-only: 1 when the environment was created with native mesh
                                       metadata (the reference's ArenaMesh::hasNativeMetadata) */
     CARL_PARAM_TICK_WINDOW_LAUNCH = 15, /* read-only: simulations per workgroup the next window launch

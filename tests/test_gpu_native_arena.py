@@ -15,6 +15,7 @@ after every step, on the window kernel and on the phase kernels.
 import numpy as np
 import pytest
 
+import carl_amd
 import native_meta
 from carl_amd import workloads
 from gpu_harness import Pair, dense_geometry_reset_state
@@ -92,5 +93,46 @@ def test_stage_profile_refuses_the_native_branch(gpu, tmp_path, monkeypatch, are
             pair.gpu.enable_tick_timing(True, stages=True)
         pair.gpu.enable_tick_timing(True)      # whole-launch timing still works
         pair.gpu.enable_tick_timing(False)
+    finally:
+        pair.close()
+
+
+@pytest.mark.parametrize("n_sim,n_blue,n_orange,streams,launch", [
+    (1, 1, 1, 1, 8),           # the smallest: one workgroup
+    (1000, 1, 1, 1, 8),        # 125 workgroups where 64 simulations each would make 16
+    (100, 1, 0, 1, 8),
+    (11_001, 1, 1, 1, 16),     # 8 simulations each would be 1,376 workgroups: more than fit a GPU that holds 1,024
+    (70_001, 1, 1, 1, 64),     # the GPU is full: as set
+    (9000, 1, 1, 2, 16),       # two partitions share the GPU
+    (200, 4, 4, 1, 8),         # from 16, what 128 cars allow
+    (50, 3, 2, 1, 12),         # from 25
+])
+def test_native_runs_are_spread_over_the_gpu(gpu, tmp_path, monkeypatch, arena, n_sim, n_blue, n_orange, streams,
+                                             launch):
+    """Until tick_window is set, workgroups of the tick-window kernel are
+    halved, down to 8 simulations, while they still fit the GPU together.
+    Setting the size fixes it."""
+    monkeypatch.setenv("CARL_ARENA_METADATA", native_meta.write(tmp_path / "arena.meta",
+                                                                native_meta.restating(*arena)))
+    env = carl_amd.Env(n_sim, n_blue, n_orange, 1, 4, True, False, False)
+    env.tick_streams = streams
+    assert env.native_arena and env.tick_window_launch == launch
+    env.tick_window = 64
+    assert env.tick_window_launch == min(64, 128 // (n_blue + n_orange))
+
+
+@pytest.mark.parametrize("n_sim,team", [(1, 1), (203, 1), (67, 4)])
+def test_native_runs_of_automatic_size_match_the_oracle(gpu, tmp_path, monkeypatch, arena, n_sim, team):
+    rng = np.random.default_rng(n_sim)
+    monkeypatch.setenv("CARL_ARENA_METADATA", native_meta.write(tmp_path / "arena.meta",
+                                                                native_meta.synthetic(*arena, rng, n_meshes=5)))
+    pair = Pair(n_sim, team, team, seed=61, frameskip=4)
+    try:
+        assert pair.gpu.tick_window_launch == 8
+        pair.apply_reset_state(dense_geometry_reset_state(rng, n_sim, 2 * team))
+        for step in range(10):
+            pair.step_continuous(workloads.random_continuous_actions(rng, n_sim, 2 * team))
+            report = pair.state_mismatches() + pair.output_mismatches()
+            assert not report, f"after step {step}:\n  " + "\n  ".join(report)
     finally:
         pair.close()
