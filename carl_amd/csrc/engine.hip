@@ -514,6 +514,7 @@ __global__ __launch_bounds__(kTickBlock) void finishKernel(Dev d, int simsPerBlo
 #endif
 constexpr int kWindowBlock = CARL_WINDOW_BLOCK;
 constexpr int kWindowWaves = kWindowBlock / 64;
+static_assert(kWindowWaves == 2, "an odd windowSims leaves the second wave one simulation fewer");
 constexpr int kDefaultWindowSims = CARL_WINDOW_SIMS;
 constexpr int kNativeWindowMin = 8;   // smallest automatic workgroup of a native arena's run (simulations)
 // rounds of candidate-index loads the window kernel's contact search keeps in
@@ -661,6 +662,7 @@ struct WindowMap {
     int* outList;
     int* clearCount;      // the counts the next launch files into
     int unitSims, nUnits, rounds, listLen, groups;
+    int odd;              // 1: a workgroup's second wave holds one simulation fewer (unitSims - 1)
 };
 
 // What a wave of the window kernel keeps in LDS about its share.
@@ -741,15 +743,17 @@ DI void tickWindowBody(const Dev& d0, int screen, int kind, const void* __restri
     {
         const int unitCars = map.unitSims * d.nCars, slot = lane / unitCars, at = lane - slot * unitCars;
         int car = -1, sim = -1;
+        // simulation i of unit u, or -1
+        auto simOf = [&](int u, int i) {
+            const int s = range.begin + u * map.unitSims - (map.odd ? u >> 1 : 0) + i;
+            return s < range.end && i < map.unitSims - (map.odd & u) ? s : -1;
+        };
         if (slot < map.rounds && m.unit[slot] >= 0) {
-            const int s = range.begin + m.unit[slot] * map.unitSims + at / d.nCars;
-            if (s < range.end) car = s * d.nCars + at % d.nCars;
+            const int s = simOf(m.unit[slot], at / d.nCars);
+            if (s >= 0) car = s * d.nCars + at % d.nCars;
         }
         const int bslot = lane / map.unitSims;
-        if (bslot < map.rounds && m.unit[bslot] >= 0) {
-            const int s = range.begin + m.unit[bslot] * map.unitSims + (lane - bslot * map.unitSims);
-            if (s < range.end) sim = s;
-        }
+        if (bslot < map.rounds && m.unit[bslot] >= 0) sim = simOf(m.unit[bslot], lane - bslot * map.unitSims);
         m.car[lane] = car;
         m.sim[lane] = sim;
     }
@@ -2073,7 +2077,7 @@ struct WindowShape {
     bool block = false;    // the workgroup-wide kernel (simsPerBlock simulations each)
     bool dealt = false;
     int blocks = 0, simsPerBlock = 0;          // simsPerBlock: at most, of a workgroup's two waves
-    int unitSims = 0, nUnits = 0, rounds = 0, listLen = 0, groups = 1;  // WindowMap
+    int unitSims = 0, nUnits = 0, rounds = 0, listLen = 0, groups = 1, odd = 0;  // WindowMap
 };
 
 // The deal's unit for waves of up to waveSims simulations: in a large run one
@@ -2100,7 +2104,7 @@ constexpr int kDealMinTicks = 4;
 // the device: a launch lasts as long as its slowest wave's chain of phases,
 // and that chain grows with the cars per wave (the candidate lists it walks,
 // the branches its lanes take between them).  A set windowSims gives each of
-// a workgroup's waves half of it.  With native arena meshes a workgroup's size
+// a workgroup's waves half of it, the first one more where it is odd.  With native arena meshes a workgroup's size
 // is halved from windowSims, down to kNativeWindowMin, while the workgroups
 // still fit the device together: each lane gathers its own ball's contacts, and
 // 8 lanes a wave wait for fewer of them than 64 (1v1 steps of 8 ticks at 1,000
@@ -2119,6 +2123,7 @@ WindowShape windowShape(const carl_env* e, int n, int parts, int ticks)
     bool dealable = e->balance && !e->native() && parts == 1 && ticks >= kDealMinTicks && e->dealList;
     if (e->windowAuto && !e->native()) {
         waveSims = std::min(most, std::max(1, e->grid(n, resident)));
+        w.simsPerBlock = kWindowWaves * waveSims;
         if (waveSims * (long long)resident < n) dealable = dealable && (nC == 2 || nC == 4) && n % (4 * line) == 0;
     } else {
         w.simsPerBlock = std::min(e->windowSims, kWindowBlock / nC);
@@ -2133,12 +2138,12 @@ WindowShape windowShape(const carl_env* e, int n, int parts, int ticks)
             return w;
         }
     }
-    w.simsPerBlock = kWindowWaves * waveSims;
+    w.odd = w.simsPerBlock % kWindowWaves;
     w.blocks = e->grid(n, w.simsPerBlock);
     w.groups = kWindowWaves * w.blocks <= resident && w.blocks >= kXcds ? kXcds : 1;
     auto take = [&](int unitSims) {
         w.unitSims = unitSims;
-        w.nUnits = e->grid(n, unitSims);
+        w.nUnits = w.odd ? kWindowWaves * w.blocks : e->grid(n, unitSims);
         w.rounds = w.listLen = 0;
         for (int g = 0; g < w.groups; g++) {
             const int waves = (groupBlocksBefore(w.blocks, w.groups, g + 1) - groupBlocksBefore(w.blocks, w.groups, g)) * kWindowWaves;
@@ -2204,6 +2209,7 @@ int launchTicks(carl_env* e, int kind, const void* actions, int n)
             map.rounds = w.rounds;
             map.listLen = w.listLen;
             map.groups = w.groups;
+            map.odd = w.odd;
             if (w.dealt) {
                 if (e->dealUnitSims != w.unitSims || e->dealGroups != w.groups || e->dealBlocks != w.blocks) {
                     // lists of other units (or none): the first launch of

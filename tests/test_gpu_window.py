@@ -64,6 +64,23 @@ def test_window_block_sizes_and_partitions(gpu, window, streams):
     _run_both(3001, 1, 1, 8, 12, workloads.random_reset_state, seed=42, window=window, streams=streams)
 
 
+@pytest.mark.parametrize("n,n_blue,n_orange,window", [
+    (1, 1, 1, 1), (2, 1, 1, 1),     # one simulation per workgroup: its second wave holds none
+    (17, 1, 1, 3), (3001, 1, 1, 63), (3001, 1, 0, 127),
+    (62_000, 1, 1, 21),             # more workgroups than are resident
+    (401, 2, 2, 31), (200, 3, 2, 7), (200, 4, 4, 15),
+    (21 * 7, 1, 1, 21),             # the last workgroup full
+])
+def test_window_sizes_that_do_not_halve(gpu, n, n_blue, n_orange, window):
+    """An odd size is kept: the first of a workgroup's waves takes one more."""
+    env = carl_amd.Env(n, n_blue, n_orange, 5, 4, True, False, True)
+    env.tick_window = window
+    assert env.tick_window_launch == window and not env.tick_balanced_launch
+    del env
+    _run_both(n, n_blue, n_orange, 4, 6, workloads.clustered_reset_state, seed=n + window, window=window, streams=1,
+              reset_every=3)
+
+
 def test_window_dense_geometry_3v3_and_2v2(gpu):
     _run_both(1024, 3, 3, 4, 20, dense_geometry_reset_state, seed=43)
     _run_both(2048, 2, 2, 4, 20, dense_geometry_reset_state, seed=44, window=32)
