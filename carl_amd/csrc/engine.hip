@@ -698,7 +698,8 @@ DI void tickWindowBody(const Dev& d0, int screen, int kind, const void* __restri
         m.cost[lane] = 0;
     }
     waveSync();
-    if (map.inCount) {
+    bool dealt = map.inCount != nullptr;
+    if (dealt) {
         // the lists' first ranks, costliest class first, in the LDS the
         // contact phase takes over afterwards; each lane scans kListsPerLane
         // of them: list k in rank order holds class kDealClasses - 1 - k / kDealSubs
@@ -706,20 +707,26 @@ DI void tickWindowBody(const Dev& d0, int screen, int kind, const void* __restri
                       "the deal's scan: whole lists per lane, in one wave's LDS");
         int* first = reinterpret_cast<int*>(&L);
         int n[kListsPerLane], sum = 0;
+        bool whole = true;
 #pragma unroll
         for (int i = 0; i < kListsPerLane; i++) {
             const int k = kListsPerLane * lane + i;
             n[i] = map.inCount[group * kDealLists + (kDealClasses - 1 - k / kDealSubs) * kDealSubs + k % kDealSubs];
             sum += n[i];
+            whole = whole && n[i] <= map.listLen;
         }
-        int r = waveInclusiveScan(sum) - sum;
+        const int incl = waveInclusiveScan(sum);
+        int r = incl - sum;
+        // lists that do not hold each of the group's units once (a captured
+        // launch that is replayed files its units again) are not dealt from
+        dealt = __builtin_amdgcn_readlane(incl, 63) == nUnits && __ballot(!whole) == 0;
 #pragma unroll
         for (int i = 0; i < kListsPerLane; i++) {
             first[kListsPerLane * lane + i] = r;
             r += n[i];
         }
         waveSync();
-        if (lane < map.rounds) {
+        if (dealt && lane < map.rounds) {
             const int rank = lane == 0 ? wv : lane * waves + (waves - 1 - wv);
             if (rank < nUnits) {
                 // the last list whose first rank is at most rank
@@ -727,10 +734,11 @@ DI void tickWindowBody(const Dev& d0, int screen, int kind, const void* __restri
                 for (int step = kDealLists / 2; step > 0; step >>= 1)
                     if (lo + step < kDealLists && first[lo + step] <= rank) lo += step;
                 const int k = (kDealClasses - 1 - lo / kDealSubs) * kDealSubs + lo % kDealSubs;
-                m.unit[lane] = map.inList[(size_t)(group * kDealLists + k) * map.listLen + min(rank - first[lo], map.listLen - 1)];
+                m.unit[lane] = map.inList[(size_t)(group * kDealLists + k) * map.listLen + (rank - first[lo])];
             }
         }
-    } else if (lane < map.rounds) {
+    }
+    if (!dealt && lane < map.rounds) {
         const int u = wv * map.rounds + lane;
         m.unit[lane] = u < nUnits ? unit0 + u : -1;
     }
@@ -1917,7 +1925,8 @@ struct carl_env {
     // the deal of window launches, kDealSets sets of class counts and lists
     // (dealRoom words each), the dealt launches so far and the units, groups
     // and workgroups they dealt to (these set which units a group holds and
-    // where its lists lie: a launch with others starts over)
+    // where its lists lie: a launch with others, or after one that failed,
+    // starts over)
     int* dealCount = nullptr;
     int* dealList = nullptr;
     size_t dealRoom = 0;      // words of one set of lists
@@ -2215,12 +2224,14 @@ int launchTicks(carl_env* e, int kind, const void* actions, int n)
                     // lists of other units (or none): the first launch of
                     // these deals the identity and files into cleared counts
                     clearDealKernel<<<kDealSets * kXcds, kDealLists, 0, stream[p]>>>(e->dealCount);
-                    e->dealUnitSims = w.unitSims;
                     e->dealGroups = w.groups;
                     e->dealBlocks = w.blocks;
                     e->dealLaunches = 0;
                 }
-                const long long l = e->dealLaunches++;
+                // no lists until this launch is queued: where that fails, the
+                // next one starts over
+                e->dealUnitSims = 0;
+                const long long l = e->dealLaunches;
                 const size_t per = (size_t)map.groups * kDealLists * map.listLen;
                 auto set = [&](long long k, int* base, size_t len) { return base + (size_t)(k % kDealSets) * len; };
                 map.inCount = l > 0 ? set(l, e->dealCount, kXcds * kDealLists) : nullptr;
@@ -2232,6 +2243,11 @@ int launchTicks(carl_env* e, int kind, const void* actions, int n)
             CARL_MARK(launchTick(e, timed, CARL_KERNEL_WINDOW, windowKernelFor(e->nCars), dim3(w.blocks),
                                  dim3(kWindowBlock), 0, stream[p], d, e->contactScreen, kind, actions, e->tickCount + 1, n,
                                  r, map, prof));
+            if (w.dealt) {
+                HIP_TRY(hipGetLastError());
+                e->dealUnitSims = w.unitSims;
+                e->dealLaunches++;
+            }
         }
     }
     for (int k = 0; e->windowSims == 0 && k < n; k++) {
