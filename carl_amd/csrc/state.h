@@ -75,10 +75,12 @@ DI Tri unpackTri(const float4* rec)
 DI Tri loadTri(const ArenaView& a, int ref) { return unpackTri(a.rec + 4 * (size_t)ref); }
 DI Tri loadTriIdx(const ArenaView& a, int idx) { return unpackTri(a.tri + 4 * (size_t)idx); }
 
-// max(x, 0) / c as the correctly rounded quotient, by a reciprocal and one
-// residual step (4 operations where the division's own scaling takes 10; the
-// three cell sizes checked against / for every float in [0, 1e5]).  Beyond
-// 1e5 the caller's clamp to the grid decides, and there x is held at 1e5.
+// max(x, 0) / c by a reciprocal and one residual step (4 operations where the
+// division's own scaling takes 10).  Not always the division's quotient: of
+// the floats in [0, 1e5] 51,806 give the next one for the x cells, 33,554 for
+// the y cells and none for the z cells.  None of them comes to another whole
+// number, so the cell is the division's for every one (tests/test_cell_lookup.py).
+// Beyond 1e5 the caller's clamp to the grid decides, and there x is held at 1e5.
 HDI float overCell(float x, float c)
 {
     const float r = 1.f / c;   // folded: c is a constant
