@@ -1,8 +1,8 @@
 """The vector environment's step written by one kernel equals the same step
 through separate torch operations (which a reward function selects) over
-steps in which episodes end: odd sizes, both action kinds, deferred and
-immediate reports, side streams, and the sizes at which the report is read in
-two parts."""
+steps in which episodes end, by goals for either team and by timeouts: odd
+sizes, both action kinds, deferred and immediate reports, side streams,
+returns and lengths carried in, and the sizes at which the report is read in two parts."""
 from __future__ import annotations
 
 from contextlib import contextmanager
@@ -32,11 +32,11 @@ def actions(gen, env, discrete):
     return (u * torch.tensor([3, 3, 3, 2, 2, 3, 2], device="cuda")).int() if discrete else u * 2 - 1
 
 
-def place_balls(envs, gen):
+def place_balls(envs, gen, shift=0):
     """Balls beyond either goal line and in the field, the same in every
     environment: a third of the matches ends with a goal for each team."""
     n = envs[0].n_sim
-    third = torch.randperm(n, generator=gen, device="cuda") % 3
+    third = (torch.randperm(n, generator=gen, device="cuda") + shift) % 3
     position = torch.zeros((n, 3), dtype=torch.float32, device="cuda")
     position[:, 1] = (third == 1) * 5300.0 - (third == 2) * 5300.0
     position[:, 2] = 100.0
@@ -112,8 +112,16 @@ def test_one_kernel_equals_separate_operations(n_sim, blue, orange, discrete, de
     stream.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(stream):
         torch.testing.assert_close(ours.reset(), want.reset(), rtol=0, atol=0)
+        # totals from before, as after many steps: both words of a length
+        agent = torch.arange(ours.n_envs, device="cuda")
+        for env in (ours, want):
+            env._ledger.returns.copy_(agent % 7 - 2.75)
+            env._ledger.lengths.copy_((agent % 3) * (1 << 33) + agent % 11)
         ended = 0
-        for _ in range(14):
+        signs, flags = set(), set()
+        for step in range(14):
+            if step in (1, 6, 11):
+                place_balls((ours, want), gen, shift=step // 5)
             a = actions(gen, ours, discrete)
             got, ref = ours.step(a), want.step(a)
             for g, w in zip(got[:4], ref[:4]):
@@ -131,7 +139,10 @@ def test_one_kernel_equals_separate_operations(n_sim, blue, orange, discrete, de
             for name in ("_score_difference", "_episode_ticks", "_overtime"):
                 torch.testing.assert_close(getattr(ours, name), getattr(want, name), rtol=0, atol=0)
             ended += int((got[2] | got[3]).sum())
+            signs |= set(got[1].tolist())
+            flags |= set(zip(got[2].tolist(), got[3].tolist()))
         assert ended >= ours.n_envs
+        assert signs == {-1.0, 0.0, 1.0} and flags == {(False, False), (True, False), (False, True)}
         if deferred:
             assert ours.drain_episode_reports() == want.drain_episode_reports()
         torch.testing.assert_close(ours._ledger.returns, want._ledger.returns, rtol=0, atol=0)
