@@ -5,12 +5,14 @@ sizes, both action kinds, deferred and immediate reports, side streams,
 returns and lengths carried in, and the sizes at which the report is read in two parts."""
 from __future__ import annotations
 
+import ctypes as C
 from contextlib import contextmanager
 
 import numpy as np
 import pytest
 import torch
 
+from carl_amd import build
 from carl_amd.gymnasium import torch as vec
 
 pytestmark = pytest.mark.gpu
@@ -176,3 +178,50 @@ def test_null_outputs_are_refused():
     t = env._ledger.returns.data_ptr()
     with pytest.raises(ValueError, match="given together"):
         env._env._vector_outputs(*[t] * 10, t, 0, 0, 0)
+
+
+class VectorIo(C.Structure):
+    """carl_vector_io"""
+    _fields_ = [(name, C.c_void_p) for name in (
+        "obs", "reward", "terminated", "truncated", "done", "returns", "lengths", "score_difference",
+        "episode_ticks", "overtime", "step_returns", "step_lengths", "step_done", "ended")]
+
+
+# addresses of every alignment a float may have; numbers of words that leave a
+# remainder of the copy's four, and more of them than one pass of the threads takes
+@pytest.mark.parametrize("n_sim,blue,orange", [(1, 1, 0), (7, 1, 0), (3, 2, 1), (20_001, 2, 2)])
+@pytest.mark.parametrize("offset", [0, 1, 2, 3])
+def test_observations_are_copied_to_any_address(n_sim, blue, orange, offset):
+    """A C caller's observation array may lie at any float's address; the
+    words around it stay as they were."""
+    engine = C.CDLL(str(build.engine_path()))
+    engine.carl_last_error.restype = C.c_char_p
+    agents = n_sim * (blue + orange)
+    env = C.c_void_p()
+    assert engine.carl_env_create(n_sim, blue, orange, 3, 1, 1, C.byref(env)) == 0, engine.carl_last_error()
+    dim = engine.carl_observation_dim(blue + orange, 0)
+    words = agents * dim
+    buffer = torch.full((words + 8,), 7.25, dtype=torch.float32, device="cuda")
+    assert buffer.data_ptr() % 16 == 0
+    sizes = {"lengths": torch.int64, "returns": torch.float32, "reward": torch.float32, "score_difference": torch.int32,
+             "episode_ticks": torch.int32}
+    rest = {name: torch.zeros(agents, dtype=sizes.get(name, torch.bool), device="cuda") for name, _ in VectorIo._fields_[1:10]}
+    torch.cuda.synchronize()
+    io = VectorIo(buffer.data_ptr() + 4 * offset, *(x.data_ptr() for x in rest.values()), None, None, None, None)
+    assert engine.carl_env_vector_outputs(env, C.byref(io)) == 0, engine.carl_last_error()
+    assert engine.carl_env_synchronize(env) == 0
+    data, shape, ndim, dtype = C.c_void_p(), (C.c_int64 * 3)(), C.c_int(), C.c_int()
+    assert engine.carl_env_buffer(env, 0, C.byref(data), shape, C.byref(ndim), C.byref(dtype)) == 0
+    assert list(shape)[:2] == [n_sim, blue + orange] and shape[2] == dim
+    want = np.empty(words, dtype=np.float32)
+    assert hip_to_host(want, data) == 0
+    got = buffer.cpu().numpy()
+    assert np.array_equal(got[offset:offset + words].view(np.uint32), want.view(np.uint32))
+    assert (got[:offset] == 7.25).all() and (got[offset + words:] == 7.25).all()
+    assert (rest["lengths"] == 1).all()
+    engine.carl_env_destroy(env)
+
+
+def hip_to_host(out, data):
+    hip = C.CDLL("libamdhip64.so")
+    return hip.hipMemcpy(C.c_void_p(out.ctypes.data), data, C.c_size_t(out.nbytes), 2)
