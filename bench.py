@@ -263,8 +263,8 @@ def main() -> None:
                     help="simulations per workgroup of the tick-window kernel, 0 for phase kernels "
                          "(-1: engine default)")
     ap.add_argument("--tick-balance", type=int, default=-1, choices=(-1, 0, 1),
-                    help="1v1 window launches dealt to the workgroups by the last launch's contact work "
-                         "(1), or workgroups of consecutive simulations (0); -1: engine default")
+                    help="window launches dealt to the waves by the dealt launch before's contact work (1), "
+                         "or waves of consecutive simulations (0); -1: engine default")
     ap.add_argument("--calibrate-copy", type=int, default=0, metavar="MIB",
                     help="only run a plain device copy of MIB MiB (HBM counter calibration) and exit")
     ap.add_argument("--summarize-rocprof", nargs=5, metavar=("TRACE", "FETCH", "WRITE", "COPY_FETCH", "COPY_WRITE"),

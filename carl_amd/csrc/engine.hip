@@ -1428,7 +1428,7 @@ __global__ __launch_bounds__(kPackBlock) void stepEnvKernel(Dev d, StepIO io, in
 }
 
 // What a vector environment (one agent per car) returns of a step, in one
-// launch: the observation rows copied to the caller, each agent's reward and
+// launch (after clearCountKernel where it lists the ended episodes): the observation rows copied to the caller, each agent's reward and
 // flags, its running return and length, and the list of the agents whose
 // episode ended.  Bound by the copy at large sizes and by its launch at small
 // ones; as separate copies and elementwise kernels the same outputs took

@@ -1447,16 +1447,13 @@ DI void finishBall(const Dev& d, int s)
     d.ssetv(CARL_SIM_BALL_IMP, s, kZero);
 }
 
-// pads of one simulation, in pad order; the last overlapping car takes the pad.
-// The cars' positions, demo flags and boost live in registers for the whole
-// pass (at most MaxCars per simulation, the loops over them unrolled);
-// boosts are written back once.  The pass is instantiated for two, four and
-// eight cars, so that 1v1 runs a quarter of the 8-car code (measured 3% per
-// step on the 1v1 window kernel).
-
-// Boost pads of simulation s in one thread: cooldowns, pickups and the boost
-// they give.  No car position lies in two pads' cylinders (the closest pair
-// of cylinders is 773 uu apart), so a car takes boost from at most one pad per
+// The phase kernels' boost pads of simulation s, in one thread and in pad
+// order: cooldowns, pickups and the boost they give; the last overlapping car
+// takes a pad.  The cars' positions, demo flags and boost live in registers
+// for the whole pass (at most MaxCars per simulation, the loops over them
+// unrolled; two, four or eight, by the team sizes); boosts are written back
+// once.  No car position lies in two pads' cylinders (the closest pair of
+// cylinders is 773 uu apart), so a car takes boost from at most one pad per
 // tick.
 template <int MaxCars>
 DI void boostPadsT(const Dev& d, int s)

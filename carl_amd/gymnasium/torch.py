@@ -527,7 +527,7 @@ class CARLTorchVectorEnv(VectorEnv):
     def _step_native(self, actions: th.Tensor):
         """step() with the engine's own reward and resets and copied outputs:
         everything that it returns is written by one kernel on the engine's
-        stream (by separate torch operations on the engine's buffers a step of
+        stream, after one that clears the count of ended episodes (by separate torch operations on the engine's buffers a step of
         17 matches took 425 us, of 50,001 849 us; so 333 and 675 us)."""
         env, n, device = self._env, self.n_envs, self.device
         ledger, deferred = self._ledger, self.defer_episode_reporting

@@ -293,8 +293,9 @@ int carl_env_reset_dones(carl_env* env);
 
 /* ---- vector environment outputs (no reference counterpart) --------------
  * What CARLTorchVectorEnv.step returns of the last carl_env_step, for one
- * agent per car (n_agents = n_sim * n_cars), written by one kernel on the
- * environment stream into the caller's device arrays.  An agent's reward is
+ * agent per car (n_agents = n_sim * n_cars), written by one kernel (with
+ * `ended`, after one that clears its count) on the environment stream into
+ * the caller's device arrays.  An agent's reward is
  * its simulation's score change, negated for orange; an episode that ended on
  * one is terminated, any other that ended truncated.  returns and lengths run
  * over an episode: this step is added, and those of episodes that ended are

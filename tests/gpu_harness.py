@@ -201,7 +201,7 @@ def pad_reset_state(rng: np.random.Generator, n_rows: int, n_cars: int) -> dict[
     """Reset inputs with every car parked on a boost pad (about a third of the
     cars share the first car's pad, so the last car in order takes it), with
     empty, partial or full boost and a few cars demoed: pickups, pad
-    cooldowns and the pad split across threads on every tick."""
+    cooldowns and the cars that share a pad on every tick."""
     pads = rng.integers(0, len(PAD_XYZ), (n_rows, n_cars))
     share = rng.uniform(size=(n_rows, n_cars)) < 0.35
     pads[:, 1:] = np.where(share[:, 1:], pads[:, :1], pads[:, 1:])

@@ -97,9 +97,9 @@ def test_null_handles_are_value_errors(lib):
 
 
 def test_boost_pad_cylinders_are_disjoint():
-    """The window kernel splits a simulation's boost pads over several threads,
-    which gives the serial result only if no car position can lie in two pads'
-    cylinders: every pair of pad circles in the engine's table is apart."""
+    """The window kernel takes pickups car by car, each at the one pad it stands
+    in, which gives the serial result only if no car position can lie in two
+    pads' cylinders: every pair of pad circles in the engine's table is apart."""
     import itertools
     import re
     from pathlib import Path

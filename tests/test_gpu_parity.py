@@ -149,17 +149,18 @@ def test_boost_pad_pickups(gpu, n_blue, n_orange):
 
 
 @pytest.mark.parametrize("n_blue,n_orange,window,frameskip", [
-    (1, 0, 128, 2),   # one car per simulation: one range of all 34 pads
-    (1, 1, 64, 2),    # two ranges of 17 (launches too short to be dealt)
-    (1, 1, 32, 2),    # four ranges of 8 or 9
+    (1, 0, 128, 2),   # one car per simulation, 64 per wave: one range of all 34 pads
+    (1, 1, 64, 2),    # 32 per wave: two ranges of 17 (launches too short to be dealt)
+    (1, 1, 32, 2),    # 16 per wave: four ranges of 8 or 9
     (2, 2, 32, 8),    # dealt 2v2 launches: four ranges of 8 or 9
-    (3, 3, 21, 2),    # six ranges of 5 or 6
+    (3, 3, 21, 2),    # the workgroup-wide kernel: six ranges of 5 or 6
 ])
 def test_boost_pad_ranges_by_workgroup_size(gpu, n_blue, n_orange, window, frameskip):
-    """The window kernel splits each simulation's pads into as many ranges as
-    its workgroup has threads per simulation; cars parked on pads, for every
-    split the workgroup sizes give: pickups and cooldowns against the
-    oracle."""
+    """The window kernel counts each simulation's cooldowns down in as many
+    ranges of its pads as a wave has lanes per simulation (the workgroup-wide
+    kernel, 21 simulations of 3v3: as its workgroup has threads); cars parked
+    on pads, for every split the workgroup sizes give: pickups and cooldowns
+    against the oracle."""
     rng = np.random.default_rng(window + 7 * n_blue + n_orange)
     n, nc = 128, n_blue + n_orange
     p = Pair(n, n_blue, n_orange, seed=6, frameskip=frameskip)

@@ -1,12 +1,12 @@
 """The stage profile (CARL_TIME_STAGES) of the tick.
 
-The window kernel's profiled twin reads the wall clock at every phase
-barrier.  Its clock must agree with the HIP events around the same launches:
-the span from the first workgroup start to the last workgroup end is 95% to
-101% of the launch time (the launch also holds the dispatch before the first
-clock read and the end after the last).  The critical path, the phases of
-the workgroup that finished each launch last plus its start delay, sums to
-the span within 1% (the clock reads between its phases).  The per-stage
+With it on, the window kernel's waves read the wall clock after every phase.
+The clock must agree with the HIP events around the same launches: the span
+from the first wave's start to the last wave's end is 90% to 101% of the
+launch time (the launch also holds the dispatch before the first clock read
+and the end after the last).  The critical path, the phases of the wave that
+finished each launch last plus its start delay, sums to the span within 1%
+(the clock reads between its phases).  The per-stage
 device shares sum to no more than the span.  The figures hold whether the
 grid fits the device at once, fills it exactly, or runs in several rounds.
 The profiled kernel computes the same state as the plain one, and the

@@ -1,9 +1,10 @@
 """Wheel rays at bodies near the end of their reach, engine against oracle.
 
 The engine does not cast a car's wheel rays at another car or at the ball
-whose centre lies beyond the rays' reach plus that body's bounding radius
-(car_phase.h: kCarRayReach, 189.7 uu, and kBallRayReach, 200.9 uu), since
-every such ray would miss; the oracle casts every ray.  Here each simulation
+whose centre lies farther from the point half way down the rays than their
+bounding sphere plus that body's radius (car_phase.h: kCarRayReach, 145.5 uu,
+and kBallRayReach, 156.8 uu), since every such ray would miss; the oracle
+casts every ray.  Here each simulation
 puts the other car, or the ball, where one wheel ray just reaches it, a
 little before the ray's end: a corner of the other car's box, turned so that
 the box lies beyond it as seen from the car's centre (the farthest a hit

@@ -164,9 +164,9 @@ def test_window_single_car(gpu):
 
 @pytest.mark.parametrize("n_blue,n_orange,window", [(1, 1, 64), (2, 2, 37), (4, 3, 18), (4, 4, 64)])
 def test_window_boost_pad_split_and_large_teams(gpu, n_blue, n_orange, window):
-    """Cars parked on pads (some sharing one): the window kernel splits each
-    simulation's pads over several threads, the phase kernels take them in one
-    thread; both must give the same boosts and cooldowns."""
+    """Cars parked on pads (some sharing one): the window kernel takes pickups
+    car by car and the cooldowns over several lanes, the phase kernels both in
+    one thread per simulation; the boosts and cooldowns must be the same."""
     _run_both(900, n_blue, n_orange, 2, 12, pad_reset_state, seed=47 + n_blue + n_orange, window=window)
 
 
